@@ -144,6 +144,8 @@ int spc5_hip_mat_load(const char* path, spc5_hip_mat_t* out);
  * every block of a block-row covers the same rows (stencils: all blocks of
  * a block-row add to the same r rows at the same step), costs extra work
  * for irregular masks.  Results agree with the default order to rounding.
+ * Matrices whose neighbouring blocks read neighbouring parts of x run a
+ * kernel with one block per lane, which the option does not change.
  * No counterpart in the reference (a property of the GPU kernel). */
 #define SPC5_HIP_OPT_ROW_SORT 1
 /* SPMM_COLUMNS (0 or 1, default 0; used for r = 2, 4 and 8): spc5_hip_spmm
@@ -153,8 +155,9 @@ int spc5_hip_mat_load(const char* path, spc5_hip_mat_t* out);
  * to rounding.  No counterpart in the reference. */
 #define SPC5_HIP_OPT_SPMM_COLUMNS 2
 /* TILE_VALUES (0, or 64 .. 2^24): values one wave's tile aims at; a tile
- * also ends every 128 rows.  0 restores the default (nnz / 8192, clamped
- * to [512, 8192]).  Rebuilds the tile plan (synchronises the device); a
+ * also ends every 128 rows (64 for r = 1), and the rows between are cut into
+ * equal parts of at most that many values.  0 restores the default: nnz / 2048
+ * clamped to [128, 512] or, if larger, nnz / 8192 up to 2048.  Rebuilds the tile plan (synchronises the device); a
  * batch created afterwards uses the new tiles.  No counterpart in the
  * reference (the work split of the GPU kernel). */
 #define SPC5_HIP_OPT_TILE_VALUES 3

@@ -13,6 +13,7 @@
 // the row-sorted tile (as the single-matrix product does).
 // The launch is captured once into a hipGraph; every product replays it.
 #include "spc5_mat.hpp"
+#include "spmv_lane.hpp"
 #include "spmv_tile.hpp"
 
 #include <algorithm>
@@ -26,12 +27,11 @@ struct BatchEntry {
     const void* val;
     const void* x;
     void* y;
-    const int* tile_br;
-    const int* tile_val;
+    const int4* tiles;
     int64_t nrows;
     int64_t ncols;
     int r;
-    int pad;
+    int lanes;  // 1: lane-block tile
 };
 
 struct spc5_hip_batch {
@@ -41,7 +41,8 @@ struct spc5_hip_batch {
     int64_t ntiles = 0;
     int waves = 0;
     int only_r = 0;         // the r shared by every matrix, 0 if they differ
-    int sorted = 0;         // only_r is 2 or 4 and every matrix has row sorting on
+    int lanes = 0;          // only_r, and every matrix runs the lane-block tile
+    int sorted = 0;         // only_r is 2 or 4, not all lane-block, and every matrix has row sorting on
     DeviceBuffer entries;   // BatchEntry[nmats]
     DeviceBuffer tile_mat;  // int32[ntiles]: matrix of each tile
     DeviceBuffer tile_loc;  // int32[ntiles]: tile index inside its matrix
@@ -69,8 +70,17 @@ union BatchSmem {
     TileSmem<ACC, 4, expand_cap<V>()> r4;
     TileSmem<ACC, 8, expand_cap<V>()> r8;
 };
+// Any r and either tile.
+template <class V, class ACC, int MB>
+union MixedSmem {
+    BatchSmem<V, ACC> order;
+    LaneSmem<V, ACC, 1, MB> l1;
+    LaneSmem<V, ACC, 2, MB> l2;
+    LaneSmem<V, ACC, 4, MB> l4;
+    LaneSmem<V, ACC, 8, MB> l8;
+};
 #define SPC5_BATCH_TILE(RR, SMEM) \
-    spmv_tile<V, X, ACC, RR, VS, MB>(SMEM, m.bptr, m.hdr, val, x, y, br0, br1, v0, v1, m.nrows, m.ncols, ep)
+    spmv_tile<V, X, ACC, RR, VS, MB>(SMEM, m.bptr, m.hdr, val, x, y, first, last, m.nrows, m.ncols, ep)
 
 // Waves per SIMD of the batch kernel: with every r body (ONLY_R = 0) the
 // most that compile without spills; with one r, the tile kernel's rule.
@@ -78,6 +88,9 @@ constexpr int batch_waves_per_eu(int only_r, bool wide_x, int value_bytes, bool 
     // the persistent loop's own state costs one wave (two with 8-byte values)
     return only_r == 0 ? 5 : tile_waves_per_eu(only_r, sorted, wide_x) - (value_bytes == 8 ? 2 : 1);
 }
+
+#define SPC5_BATCH_LANES(RR, SMEM) \
+    spmv_lane_tile<V, X, ACC, RR, VS, MB>(SMEM, m.bptr, m.hdr, val, x, y, first, last, m.nrows, m.ncols, ep)
 
 // The batch loop over tiles: tile t of the list runs body(matrix entry,
 // tile bounds) on its wave.
@@ -93,103 +106,123 @@ __device__ __forceinline__ void batch_tiles(const BatchEntry* __restrict__ mats,
     for (int64_t t = t0; t < ntiles; t += stride) {
         const BatchEntry& m = mats[tile_mat[t]];
         const int lt = tile_loc[t];
-        body(m, m.tile_br[lt], m.tile_br[lt + 1], m.tile_val[lt], m.tile_val[lt + 1]);
+        body(m, m.tiles[lt], m.tiles[lt + 1]);
         wave_sync();
     }
 }
 
-// Every matrix has r = R and row sorting on.
+// Every matrix has r = R and row sorting on; those that run the lane-block
+// tile keep it.
 template <class V, class X, class ACC, int VS, int MB, int R>
 __global__ __launch_bounds__(kWavesPerGroup * 64, batch_waves_per_eu(R, sizeof(X) > sizeof(ACC), sizeof(V), true)) void
 k_spmv_batch_sorted(const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat,
                     const int* __restrict__ tile_loc, int64_t ntiles) {
     static_assert(R == 2 || R == 4, "row-sorted tiles exist for r = 2 and 4");
-    __shared__ TileSmem<ACC, R, expand_cap<V>(), true> sm[kWavesPerGroup];
+    __shared__ union {
+        TileSmem<ACC, R, expand_cap<V>(), true> order;
+        LaneSmem<V, ACC, R, MB> lanes;
+    } sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const Epilogue ep;
-    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int br0, int br1, int v0, int v1) {
-        spmv_tile<V, X, ACC, R, VS, MB, true>(sm[w], m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
-                                              reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), br0, br1,
-                                              v0, v1, m.nrows, m.ncols, ep);
+    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
+        if (m.lanes)
+            spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w].lanes, m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
+                                                 reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first,
+                                                 last, m.nrows, m.ncols, ep);
+        else
+            spmv_tile<V, X, ACC, R, VS, MB, true>(sm[w].order, m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
+                                              reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first, last,
+                                              m.nrows, m.ncols, ep);
     });
 }
 
-template <class V, class X, class ACC, int VS, int MB, int ONLY_R>
-__global__ __launch_bounds__(kWavesPerGroup * 64, batch_waves_per_eu(ONLY_R, sizeof(X) > sizeof(ACC), sizeof(V))) void
-k_spmv_batch(const BatchEntry* __restrict__ mats,
-                                                                     const int* __restrict__ tile_mat,
-                                                                     const int* __restrict__ tile_loc,
-                                                                     int64_t ntiles) {
-    __shared__ BatchSmem<V, ACC> sm[kWavesPerGroup];
+// Every matrix has r = R and runs the lane-block tile.
+template <class V, class X, class ACC, int VS, int MB, int R>
+__global__ __launch_bounds__(kWavesPerGroup * 64, lane_waves_per_eu(R, VS, sizeof(X)) - 1) void k_spmv_batch_lanes(
+    const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat, const int* __restrict__ tile_loc,
+    int64_t ntiles) {
+    __shared__ LaneSmem<V, ACC, R, MB> sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
-    const int64_t stride = (int64_t)gridDim.x * kWavesPerGroup;
     const Epilogue ep;
-    // The tile index is the same on every lane (it comes from the wave index,
-    // which the compiler cannot tell is uniform): read it as a scalar, so the
-    // matrix descriptor is loaded into scalar registers.
-    const int64_t t0 = (int64_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerGroup + w));
-    for (int64_t t = t0; t < ntiles; t += stride) {
-        const BatchEntry& m = mats[tile_mat[t]];
-        const int lt = tile_loc[t];
-        const int br0 = m.tile_br[lt], br1 = m.tile_br[lt + 1], v0 = m.tile_val[lt], v1 = m.tile_val[lt + 1];
+    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
+        spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w], m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
+                                             reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first, last,
+                                             m.nrows, m.ncols, ep);
+    });
+}
+
+// Every matrix has r = R and runs the value-order tile.
+template <class V, class X, class ACC, int VS, int MB, int R>
+__global__ __launch_bounds__(kWavesPerGroup * 64, batch_waves_per_eu(R, sizeof(X) > sizeof(ACC), sizeof(V))) void
+k_spmv_batch(const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat, const int* __restrict__ tile_loc,
+             int64_t ntiles) {
+    __shared__ TileSmem<ACC, R, expand_cap<V>()> sm[kWavesPerGroup];
+    const int w = threadIdx.x >> 6;
+    const Epilogue ep;
+    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
+        spmv_tile<V, X, ACC, R, VS, MB>(sm[w], m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
+                                        reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first, last,
+                                        m.nrows, m.ncols, ep);
+    });
+}
+
+// Any r and either tile per matrix.
+template <class V, class X, class ACC, int VS, int MB>
+__global__ __launch_bounds__(kWavesPerGroup * 64, batch_waves_per_eu(0, sizeof(X) > sizeof(ACC), sizeof(V))) void
+k_spmv_batch_mixed(const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat,
+                   const int* __restrict__ tile_loc, int64_t ntiles) {
+    __shared__ MixedSmem<V, ACC, MB> sm[kWavesPerGroup];
+    const int w = threadIdx.x >> 6;
+    const Epilogue ep;
+    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
         const V* val = reinterpret_cast<const V*>(m.val);
         const X* x = reinterpret_cast<const X*>(m.x);
         X* y = reinterpret_cast<X*>(m.y);
-        switch (ONLY_R ? ONLY_R : m.r) {
-        case 1:
-            SPC5_BATCH_TILE(1, sm[w].r1);
-            break;
-        case 2:
-            SPC5_BATCH_TILE(2, sm[w].r2);
-            break;
-        case 4:
-            SPC5_BATCH_TILE(4, sm[w].r4);
-            break;
-        default:
-            SPC5_BATCH_TILE(8, sm[w].r8);
-            break;
+        switch (m.lanes ? -m.r : m.r) {
+        case 1: SPC5_BATCH_TILE(1, sm[w].order.r1); break;
+        case 2: SPC5_BATCH_TILE(2, sm[w].order.r2); break;
+        case 4: SPC5_BATCH_TILE(4, sm[w].order.r4); break;
+        case 8: SPC5_BATCH_TILE(8, sm[w].order.r8); break;
+        case -1: SPC5_BATCH_LANES(1, sm[w].l1); break;
+        case -2: SPC5_BATCH_LANES(2, sm[w].l2); break;
+        case -4: SPC5_BATCH_LANES(4, sm[w].l4); break;
+        default: SPC5_BATCH_LANES(8, sm[w].l8); break;
         }
-        wave_sync();
-    }
+    });
 }
 
-template <class V, class X, class ACC, int VS, int MB, int ONLY_R>
-void launch_batch_r(const spc5_hip_batch& b, hipStream_t s) {
+template <class Kernel>
+void launch_batch_kernel(const spc5_hip_batch& b, Kernel k, hipStream_t s) {
     const unsigned groups = (unsigned)((b.waves + kWavesPerGroup - 1) / kWavesPerGroup);
-    hipLaunchKernelGGL((k_spmv_batch<V, X, ACC, VS, MB, ONLY_R>), dim3(groups), dim3(kWavesPerGroup * 64), 0, s,
-                       b.entries.as<const BatchEntry>(), b.tile_mat.as<const int>(), b.tile_loc.as<const int>(),
-                       b.ntiles);
-}
-
-template <class V, class X, class ACC, int VS, int MB, int R>
-void launch_batch_sorted(const spc5_hip_batch& b, hipStream_t s) {
-    const unsigned groups = (unsigned)((b.waves + kWavesPerGroup - 1) / kWavesPerGroup);
-    hipLaunchKernelGGL((k_spmv_batch_sorted<V, X, ACC, VS, MB, R>), dim3(groups), dim3(kWavesPerGroup * 64), 0, s,
-                       b.entries.as<const BatchEntry>(), b.tile_mat.as<const int>(), b.tile_loc.as<const int>(),
-                       b.ntiles);
+    hipLaunchKernelGGL(k, dim3(groups), dim3(kWavesPerGroup * 64), 0, s, b.entries.as<const BatchEntry>(),
+                       b.tile_mat.as<const int>(), b.tile_loc.as<const int>(), b.ntiles);
 }
 
 template <class V, class X, class ACC, int VS, int MB>
 void launch_batch(const spc5_hip_batch& b, hipStream_t s) {
     if (b.sorted) {
-        if (b.only_r == 2) launch_batch_sorted<V, X, ACC, VS, MB, 2>(b, s);
-        else launch_batch_sorted<V, X, ACC, VS, MB, 4>(b, s);
+        if (b.only_r == 2) launch_batch_kernel(b, k_spmv_batch_sorted<V, X, ACC, VS, MB, 2>, s);
+        else launch_batch_kernel(b, k_spmv_batch_sorted<V, X, ACC, VS, MB, 4>, s);
         return;
     }
-    switch (b.only_r) {
-    case 1: launch_batch_r<V, X, ACC, VS, MB, 1>(b, s); break;
-    case 2: launch_batch_r<V, X, ACC, VS, MB, 2>(b, s); break;
-    case 4: launch_batch_r<V, X, ACC, VS, MB, 4>(b, s); break;
-    case 8: launch_batch_r<V, X, ACC, VS, MB, 8>(b, s); break;
-    default: launch_batch_r<V, X, ACC, VS, MB, 0>(b, s); break;
+    switch (b.lanes ? -b.only_r : b.only_r) {
+    case 1: launch_batch_kernel(b, k_spmv_batch<V, X, ACC, VS, MB, 1>, s); break;
+    case 2: launch_batch_kernel(b, k_spmv_batch<V, X, ACC, VS, MB, 2>, s); break;
+    case 4: launch_batch_kernel(b, k_spmv_batch<V, X, ACC, VS, MB, 4>, s); break;
+    case 8: launch_batch_kernel(b, k_spmv_batch<V, X, ACC, VS, MB, 8>, s); break;
+    case -1: launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, 1>, s); break;
+    case -2: launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, 2>, s); break;
+    case -4: launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, 4>, s); break;
+    case -8: launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, 8>, s); break;
+    default: launch_batch_kernel(b, k_spmv_batch_mixed<V, X, ACC, VS, MB>, s); break;
     }
 }
 
 // Waves per SIMD the batch's kernel runs at (sizes the persistent grid).
-int batch_kernel_waves(int value_type, int only_r, bool sorted) {
-    const bool wide_x = false;  // batches use the matrices' own vector type
-    return batch_waves_per_eu(only_r, wide_x, value_type == SPC5_HIP_F64 ? 8 : value_type == SPC5_HIP_F32 ? 4 : 2,
-                              sorted);
+int batch_kernel_waves(const spc5_hip_batch& b) {
+    const int vb = (int)value_bytes(b.value_type);
+    if (b.lanes) return lane_waves_per_eu(b.only_r, b.vs, vb == 8 ? 8 : 4) - 1;
+    return batch_waves_per_eu(b.only_r, false, vb, b.sorted != 0);
 }
 
 int launch_batch_any(const spc5_hip_batch& b, hipStream_t s) {
@@ -232,16 +265,12 @@ int spc5_hip_batch_create(int nmats, const spc5_hip_mat_t* mats, const void* con
         e.val = m->values;
         e.x = d_x[i];
         e.y = d_y[i];
-        e.tile_br = m->plan.ntiles ? m->plan.tile_br->as<const int>() : nullptr;
-        e.tile_val = m->plan.ntiles ? m->plan.tile_val->as<const int>() : nullptr;
-        if (m->plan.ntiles) {
-            b->tiles_kept.push_back(m->plan.tile_br);
-            b->tiles_kept.push_back(m->plan.tile_val);
-        }
+        e.tiles = m->plan.ntiles ? m->plan.tiles->as<const int4>() : nullptr;
+        if (m->plan.ntiles) b->tiles_kept.push_back(m->plan.tiles);
         e.nrows = m->nrows;
         e.ncols = m->ncols;
         e.r = m->r;
-        e.pad = 0;
+        e.lanes = m->lane_body;
         for (int64_t t = 0; t < m->plan.ntiles; ++t) {
             tmat.push_back(i);
             tloc.push_back((int)t);
@@ -254,13 +283,17 @@ int spc5_hip_batch_create(int nmats, const spc5_hip_mat_t* mats, const void* con
     SPC5_HIP_TRY(hipGetDevice(&dev));
     SPC5_HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     b->only_r = mats[0]->r;
-    bool all_sorted = true;
+    bool all_sorted = true, all_lanes = true, any_lanes = false;
     for (int i = 0; i < nmats; ++i) {
-        if (mats[i]->r != b->only_r) b->only_r = 0;
+        if (mats[i]->r != mats[0]->r) b->only_r = 0;
+        all_lanes = all_lanes && mats[i]->lane_body;
+        any_lanes = any_lanes || mats[i]->lane_body;
         all_sorted = all_sorted && mats[i]->row_sort != 0;
     }
-    b->sorted = (b->only_r == 2 || b->only_r == 4) && all_sorted ? 1 : 0;
-    int64_t wv = waves > 0 ? waves : (int64_t)ncu * 4 * batch_kernel_waves(b->value_type, b->only_r, b->sorted != 0);
+    b->lanes = b->only_r && all_lanes ? 1 : 0;
+    b->sorted = (b->only_r == 2 || b->only_r == 4) && !b->lanes && all_sorted ? 1 : 0;
+    if (b->only_r && !b->lanes && !b->sorted && any_lanes) b->only_r = 0;  // both tiles: the mixed kernel
+    int64_t wv = waves > 0 ? waves : (int64_t)ncu * 4 * batch_kernel_waves(*b);
     if (wv > b->ntiles) wv = std::max<int64_t>(b->ntiles, 1);
     b->waves = (int)wv;
     SPC5_HIP_TRY(b->entries.alloc(sizeof(BatchEntry) * (size_t)nmats));

@@ -66,18 +66,20 @@ __device__ __forceinline__ void wave_sync() {
 // together ahead of their first use.
 __device__ __forceinline__ void compiler_fence() { asm volatile("" ::: "memory"); }
 
+// DPP broadcasts of a 16-lane row's last lane into the next row (0x142) and
+// of lane 31 into the upper half (0x143), limited to the rows of the mask.
+constexpr int kDppRowBcast15 = 0x142;
+constexpr int kDppRowBcast31 = 0x143;
+
 // Inclusive prefix sum of an int over the 64 lanes: DPP shifts inside each
-// 16-lane row, then the three row totals are added with scalar readlanes.
+// 16-lane row, then the row totals by two broadcasts (six additions in all).
 __device__ __forceinline__ int wave_incl_scan(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr1, 0xf, 0xf, true);
     v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr2, 0xf, 0xf, true);
     v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr4, 0xf, 0xf, true);
     v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr8, 0xf, 0xf, true);
-    const int r0 = __builtin_amdgcn_readlane(v, 15);
-    const int r1 = __builtin_amdgcn_readlane(v, 31);
-    const int r2 = __builtin_amdgcn_readlane(v, 47);
-    const int row = lane_id() >> 4;
-    v += (row >= 1 ? r0 : 0) + (row >= 2 ? r1 : 0) + (row >= 3 ? r2 : 0);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast31, 0xc, 0xf, false);
     return v;
 }
 
@@ -88,11 +90,9 @@ __device__ __forceinline__ int wave_incl_max(int v) {
     v = max(v, __builtin_amdgcn_update_dpp(0, v, kDppRowShr2, 0xf, 0xf, true));
     v = max(v, __builtin_amdgcn_update_dpp(0, v, kDppRowShr4, 0xf, 0xf, true));
     v = max(v, __builtin_amdgcn_update_dpp(0, v, kDppRowShr8, 0xf, 0xf, true));
-    const int c1 = __builtin_amdgcn_readlane(v, 15);
-    const int c2 = max(c1, __builtin_amdgcn_readlane(v, 31));
-    const int c3 = max(c2, __builtin_amdgcn_readlane(v, 47));
-    const int row = lane_id() >> 4;
-    return max(v, row == 0 ? 0 : (row == 1 ? c1 : (row == 2 ? c2 : c3)));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xa, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, kDppRowBcast31, 0xc, 0xf, false));
+    return v;
 }
 
 // v of lane-1 across the whole wave (GFX9 wave_shr:1); `first` on lane 0.
@@ -161,7 +161,7 @@ __device__ __forceinline__ int wave_reduce_add(int v) {
     return __builtin_amdgcn_readlane(wave_incl_scan(v), 63);
 }
 
-__device__ __forceinline__ unsigned long long ballot64(bool p) { return __ballot(p); }
+__device__ __forceinline__ unsigned long long ballot64(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
 // Unaligned little-endian loads from the packed header stream.  gfx950
 // supports unaligned global accesses; the compiler emits a single dword (or

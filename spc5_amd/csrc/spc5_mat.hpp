@@ -9,10 +9,11 @@
 namespace spc5 {
 
 // Work plan of one matrix: a tile is a run of whole block-rows processed by
-// one wave.  Tiles are cut where the running value count crosses a multiple
-// of the value target, and at least every kMaxRows/r block-rows, so every
-// tile's rows fit the wave's LDS accumulators and every tile carries about
-// the same number of values.
+// one wave.  Tiles are cut every tile_rows(r) rows, so that a tile's rows fit
+// the wave's LDS accumulators, and the rows between into equal parts of at
+// most the target number of values (cutting at multiples of the target too
+// left every second tile a fragment: clustered 4 M rows 49 K tiles instead of
+// 33 K).
 #ifndef SPC5_MAX_ROWS
 #define SPC5_MAX_ROWS 128
 #endif
@@ -42,6 +43,9 @@ using FloatAcc = double;
 using FloatAcc = float;
 #endif
 constexpr int kMaxRows = SPC5_MAX_ROWS;              // scalar rows per tile (LDS accumulators), <= 256
+// Rows of a product's tile: at most 64 block-rows (the lane-block tile keeps
+// one block-row pointer per lane), at most kMaxRows rows.
+constexpr int tile_rows(int r) { return 64 * r < kMaxRows ? 64 * r : kMaxRows; }
 constexpr int kWavesPerGroup = SPC5_WAVES_PER_GROUP; // independent waves per workgroup
 static_assert(kMaxRows <= 255, "tile-local rows are stored as bytes, kMaxRows marks none");
 // Values expanded into LDS per batch for value type V.
@@ -68,8 +72,9 @@ struct Plan {
     int64_t ntiles = 0;
     int target = 0;                   // values per tile aimed at
     std::shared_ptr<DeviceBuffer> valptr;    // int32[nbr+1]: first value of each block-row
-    std::shared_ptr<DeviceBuffer> tile_br;   // int32[ntiles+1]: first block-row of each tile
-    std::shared_ptr<DeviceBuffer> tile_val;  // int32[ntiles+1]: first value of each tile
+    // int4[ntiles+1] (block-row, block, value, 0): where each tile starts, one
+    // 16-byte record so that a wave knows its whole range after one request.
+    std::shared_ptr<DeviceBuffer> tiles;
 };
 
 }  // namespace spc5
@@ -86,6 +91,8 @@ struct spc5_hip_mat {
     int row_sort = 0;                     // SPC5_HIP_OPT_ROW_SORT
     int spmm_cols = 0;                    // SPC5_HIP_OPT_SPMM_COLUMNS
     int spmm_x16 = -1;                    // SPC5_HIP_OPT_SPMM_X16; -1: 1 for double vectors, else 0
+    double scatter = 0.0;                 // distinct 128-byte lines of x per block, among 64 neighbours (sampled)
+    int lane_body = 0;                    // products run the lane-block tile (spmv_lane.hpp; see lane_block_wins)
     spc5::Plan plan;
     std::vector<std::shared_ptr<spc5::DeviceBuffer>> owned;  // buffers the handle allocated itself
 };
@@ -102,6 +109,8 @@ int launch_spmv_f64vec(const spc5_hip_mat& m, const double* x, double* y, hipStr
 int build_plan(spc5_hip_mat& m, hipStream_t s);
 // Values per tile of the default plan (defined in spmv.hip).
 int default_tile_values(int64_t nnz);
+// Whether a handle's products run the lane-block tile (defined in spmv.hip).
+bool lane_block_wins(const spc5_hip_mat& m);
 // Another tile list of the same matrix with at most `maxrows` rows per tile
 // (needs the value offsets of m.plan; defined in spmv.hip).
 int build_tiles(const spc5_hip_mat& m, Plan& p, int maxrows, int target, hipStream_t s);

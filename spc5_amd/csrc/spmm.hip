@@ -183,7 +183,7 @@ template <class V, class X, class ACC, int R, int VS, int MB, int KC, bool WIDE,
 __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr, const unsigned char* __restrict__ hdr,
                                                     const V* __restrict__ val, const X* __restrict__ x, int64_t ldx,
                                                     X* __restrict__ y, int64_t ldy, int k, int kt,
-                                                    const int* __restrict__ tile_br, const int* __restrict__ tile_val,
+                                                    const int4* __restrict__ tiles,
                                                     int64_t ntiles, int64_t nrows, int maxrows, ACC alpha, ACC beta) {
     constexpr int CAP = spmm_cap<KC, X, CPL>();
     constexpr int K = CAP / 64;
@@ -210,10 +210,11 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
     const X* __restrict__ xcol = x + c0 + (colok ? jl : 0);
     const unsigned lane_off = (unsigned)(c0 + (colok ? jl : 0)) * (unsigned)sizeof(X);  // byte offset in an X row
     const unsigned row_bytes = (unsigned)ldx * (unsigned)sizeof(X);
-    const int br0 = tile_br[t], br1 = tile_br[t + 1];
+    const int4 first = tiles[t], last = tiles[t + 1];
+    const int br0 = first.x, br1 = last.x;
     const int nbr = br1 - br0;
-    const int b0 = bptr[br0], b1 = bptr[br1];
-    int v = tile_val[t];
+    const int b0 = first.y, b1 = last.y;
+    int v = first.z;
     const int64_t row0 = (int64_t)br0 * R;
     const int64_t rows_left = nrows - row0;
     const int nrow_t = (int)((int64_t)nbr * R < rows_left ? (int64_t)nbr * R : rows_left);
@@ -421,7 +422,7 @@ template <class V, class X, class ACC, int R, int VS, int MB, int KC, bool WIDE,
 __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, const unsigned char* __restrict__ hdr,
                                                    const V* __restrict__ val, const X* __restrict__ x, int64_t ldx,
                                                    X* __restrict__ y, int64_t ldy, int k, int kt,
-                                                   const int* __restrict__ tile_br, const int* __restrict__ tile_val,
+                                                   const int4* __restrict__ tiles,
                                                    int64_t ntiles, int64_t nrows, int maxrows, ACC alpha, ACC beta) {
     constexpr int CAPR = spmm_col_cap_rec<R>();
     constexpr int CAP = spmm_col_cap_val<R>();
@@ -455,10 +456,11 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
     const X* __restrict__ xcol = x + c0 + (colok ? jl : 0);
     const unsigned lane_off = (unsigned)(c0 + (colok ? jl : 0)) * (unsigned)sizeof(X);
     const unsigned row_bytes = (unsigned)ldx * (unsigned)sizeof(X);
-    const int br0 = tile_br[t], br1 = tile_br[t + 1];
+    const int4 first = tiles[t], last = tiles[t + 1];
+    const int br0 = first.x, br1 = last.x;
     const int nbr = br1 - br0;
-    const int b0 = bptr[br0], b1 = bptr[br1];
-    int v = tile_val[t];
+    const int b0 = first.y, b1 = last.y;
+    int v = first.z;
     const int64_t row0 = (int64_t)br0 * R;
     const int64_t rows_left = nrows - row0;
     const int nrow_t = (int)((int64_t)nbr * R < rows_left ? (int64_t)nbr * R : rows_left);
@@ -681,8 +683,7 @@ template <class V, class X, class ACC, int VS, int MB, int KC, bool WIDE, int CP
 int launch_spmm_cols(const spc5_hip_mat& m, const Plan& p, int maxrows, const void* x, int64_t ldx, void* y,
                      int64_t ldy, int k, int kt, double alpha, double beta, hipStream_t s) {
     const dim3 grid(spmm_grid(p.ntiles, k, kt));
-    const int* tb = p.tile_br->as<int>();
-    const int* tv = p.tile_val->as<int>();
+    const int4* tl = p.tiles->as<int4>();
     const V* val = reinterpret_cast<const V*>(m.values);
     const X* xx = reinterpret_cast<const X*>(x);
     X* yy = reinterpret_cast<X*>(y);
@@ -691,7 +692,7 @@ int launch_spmm_cols(const spc5_hip_mat& m, const Plan& p, int maxrows, const vo
         const size_t shm = spmm_col_smem_bytes<ACC, R>(maxrows, kt, spmm_col_direct<KC, CPL>());                  \
         hipLaunchKernelGGL((k_spmm_cols<V, X, ACC, R, VS, MB, KC, WIDE, CPL>), grid, dim3(64), shm, s, m.bptr, m.hdr, \
                            val,                                                                                    \
-                           xx, ldx, yy, ldy, k, kt, tb, tv, p.ntiles, m.nrows, maxrows, (ACC)alpha, (ACC)beta);       \
+                           xx, ldx, yy, ldy, k, kt, tl, p.ntiles, m.nrows, maxrows, (ACC)alpha, (ACC)beta);       \
     }
     switch (m.r) {
     case 2: SPC5_SPMM_COLS(2); break;
@@ -709,14 +710,13 @@ int launch_spmm_vals(const spc5_hip_mat& m, const Plan& p, int maxrows, const vo
                      int64_t ldy, int k, int kt, double alpha, double beta, hipStream_t s) {
     const dim3 grid(spmm_grid(p.ntiles, k, kt));
     const size_t shm = spmm_smem_bytes<ACC, KC, X, CPL>(maxrows, kt, m.r);
-    const int* tb = p.tile_br->as<int>();
-    const int* tv = p.tile_val->as<int>();
+    const int4* tl = p.tiles->as<int4>();
     const V* val = reinterpret_cast<const V*>(m.values);
     const X* xx = reinterpret_cast<const X*>(x);
     X* yy = reinterpret_cast<X*>(y);
 #define SPC5_SPMM_LAUNCH(R)                                                                                   \
     hipLaunchKernelGGL((k_spmm_tiles<V, X, ACC, R, VS, MB, KC, WIDE, CPL>), grid, dim3(64), shm, s, m.bptr, m.hdr, \
-                       val, xx, ldx, yy, ldy, k, kt, tb, tv, p.ntiles, m.nrows, maxrows, (ACC)alpha, (ACC)beta)
+                       val, xx, ldx, yy, ldy, k, kt, tl, p.ntiles, m.nrows, maxrows, (ACC)alpha, (ACC)beta)
     switch (m.r) {
     case 1: SPC5_SPMM_LAUNCH(1); break;
     case 2: SPC5_SPMM_LAUNCH(2); break;

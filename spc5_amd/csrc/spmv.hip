@@ -16,7 +16,12 @@
 //     lane, multiplied by x[column] and added into per-row LDS accumulators;
 //   * at the end of the tile every row does one y[row] += sum (rows of a
 //     tile belong to it alone, so no global atomics and no second pass).
+//
+// That is the value-order tile (spmv_tile.hpp).  Matrices whose neighbouring
+// blocks read neighbouring parts of x run the lane-block tile instead
+// (spmv_lane.hpp); lane_block_wins() decides per handle.
 #include "spc5_mat.hpp"
+#include "spmv_lane.hpp"
 #include "spmv_tile.hpp"
 
 #include <mutex>
@@ -48,16 +53,29 @@ template <class V, class X, class ACC, int R, int VS, int MB, bool SORT>
 __global__ __launch_bounds__(kWavesPerGroup * 64, tile_waves_per_eu(R, SORT, sizeof(X) > sizeof(ACC))) void
 k_spmv_tiles(
     const int* __restrict__ bptr, const unsigned char* __restrict__ hdr, const V* __restrict__ val,
-    const X* __restrict__ x, X* __restrict__ y, const int* __restrict__ tile_br,
-    const int* __restrict__ tile_val, int64_t ntiles, int64_t nrows, int64_t ncols, Epilogue ep) {
+    const X* __restrict__ x, X* __restrict__ y, const int4* __restrict__ tiles, int64_t ntiles, int64_t nrows,
+    int64_t ncols, Epilogue ep) {
     __shared__ TileSmem<ACC, R, expand_cap<V>(), SORT> sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const int64_t t = xcd_tile(w);
     if (t >= ntiles) return;  // whole wave leaves; no workgroup barrier is used
     Epilogue e = ep;
     if (e.dot) e.dot += t;  // one partial per tile
-    spmv_tile<V, X, ACC, R, VS, MB, SORT>(sm[w], bptr, hdr, val, x, y, tile_br[t], tile_br[t + 1], tile_val[t],
-                                          tile_val[t + 1], nrows, ncols, e);
+    spmv_tile<V, X, ACC, R, VS, MB, SORT>(sm[w], bptr, hdr, val, x, y, tiles[t], tiles[t + 1], nrows, ncols, e);
+}
+
+template <class V, class X, class ACC, int R, int VS, int MB>
+__global__ __launch_bounds__(kWavesPerGroup * 64, lane_waves_per_eu(R, VS, sizeof(X))) void k_spmv_lanes(
+    const int* __restrict__ bptr, const unsigned char* __restrict__ hdr, const V* __restrict__ val,
+    const X* __restrict__ x, X* __restrict__ y, const int4* __restrict__ tiles, int64_t ntiles, int64_t nrows,
+    int64_t ncols, Epilogue ep) {
+    __shared__ LaneSmem<V, ACC, R, MB> sm[kWavesPerGroup];
+    const int w = threadIdx.x >> 6;
+    const int64_t t = xcd_tile(w);
+    if (t >= ntiles) return;  // whole wave leaves; no workgroup barrier is used
+    Epilogue e = ep;
+    if (e.dot) e.dot += t;  // one partial per tile
+    spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w], bptr, hdr, val, x, y, tiles[t], tiles[t + 1], nrows, ncols, e);
 }
 
 // ---- access probe ----------------------------------------------------------
@@ -76,9 +94,9 @@ k_spmv_tiles(
 // on an impossible value, which keeps every load live.
 template <int MODE>
 __global__ __launch_bounds__(kWavesPerGroup * 64) void k_access_probe(
-    const int* __restrict__ bptr, const unsigned char* __restrict__ hdr, const double* __restrict__ val,
-    const double* __restrict__ x, const int* __restrict__ tile_br, const int* __restrict__ tile_val, int64_t ntiles,
-    int64_t ncols, double* __restrict__ out) {
+    const unsigned char* __restrict__ hdr, const double* __restrict__ val, const double* __restrict__ x,
+    const int4* __restrict__ tiles, int64_t ntiles, int64_t ncols,
+    double* __restrict__ out) {
     constexpr int H = 5;  // int32 first column + one mask byte
     __shared__ int scol[kWavesPerGroup][512];
     const int w = threadIdx.x >> 6;
@@ -86,8 +104,8 @@ __global__ __launch_bounds__(kWavesPerGroup * 64) void k_access_probe(
     if (t >= ntiles) return;
     const int lane = threadIdx.x & 63;
     int* sc = scol[w];
-    const int b0 = bptr[tile_br[t]], b1 = bptr[tile_br[t + 1]];
-    int64_t v = tile_val[t];
+    const int b0 = tiles[t].y, b1 = tiles[t + 1].y;
+    int64_t v = tiles[t].z;
     double acc = 0.0;
     int cs = 0;
     unsigned m = 0;
@@ -163,9 +181,11 @@ __global__ void k_check_bptr(const int* __restrict__ bptr, int64_t nbr, int64_t 
 template <int R, int MB, int VS>
 __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__ bptr,
                                                          const unsigned char* __restrict__ hdr, int64_t nbr,
-                                                         int64_t ncols, int* __restrict__ cnt_out, int* err) {
+                                                         int64_t ncols, int* __restrict__ cnt_out, int* err,
+                                                         int xbytes, unsigned every) {
     constexpr int H = 4 + R * MB;
     using MW = MaskWords<R * MB>;
+    __shared__ unsigned sline[4][64];
     __shared__ int sptr[4][65];
     __shared__ int scnt[4][64];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -178,15 +198,25 @@ __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__
         sp[lane] = bptr[i < nbr ? i : nbr];
         if (lane == 0) sp[64] = bptr[br0 + 64 < nbr ? br0 + 64 : nbr];
         sc[lane] = 0;
+        sline[w][lane] = 0u;
     }
     wave_sync();
     const int b0 = sp[0], bE = sp[64];
+    // One group in `every` also counts the distinct 128-byte lines of x that
+    // its first 64 blocks start in (a hash into 2,048 bits): err[1] sums the
+    // lines, err[2] the blocks.
+    const bool sample = (blockIdx.x * 4u + (unsigned)w) % every == 0;
     bool bad = false;
     for (int b = b0 + lane; b < bE; b += 64) {
         const unsigned char* h = hdr + (int64_t)b * H;
         const int cs = load_i32_unaligned(h);
         unsigned long long mw[MW::kWords];
         MW::load(h + 4, mw);
+        if (sample && b < b0 + 64) {
+            const unsigned line = (unsigned)(((uint64_t)(unsigned)cs * (unsigned)xbytes) >> 7);
+            const unsigned h = (line * 0x9e3779b1u) >> 21;
+            atomicOr(&sline[w][h >> 5], 1u << (h & 31u));
+        }
         int c = 0;
         unsigned rowor = 0;
         for (int k = 0; k < MW::kWords; ++k) {
@@ -209,41 +239,52 @@ __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__
     wave_sync();
     if (br0 + lane < nbr) cnt_out[br0 + lane] = sc[lane];
     if (bad) atomicOr(err, 2);
+    if (sample && bE > b0) {
+        const int lines = wave_reduce_add(__popc(sline[w][lane]));
+        if (lane == 0) {
+            atomicAdd(err + 1, lines);
+            atomicAdd(err + 2, bE - b0 < 64 ? bE - b0 : 64);
+        }
+    }
 }
 
-__device__ __forceinline__ bool tile_starts(const int* valptr, int64_t br, int target, int maxbr) {
-    if (br % maxbr == 0) return true;
-    return valptr[br] / target != valptr[br - 1] / target;
+// Tiles never cross a multiple of maxbr block-rows; each such run of
+// block-rows is cut into ceil(values / target) pieces of about equal values.
+__device__ __forceinline__ bool tile_starts(const int* valptr, int64_t br, int64_t nbr, int target, int maxbr) {
+    const int64_t first = br / maxbr * maxbr;
+    if (br == first) return true;
+    const int64_t v0 = valptr[first], all = valptr[first + maxbr < nbr ? first + maxbr : nbr] - v0;
+    if (all <= target) return false;
+    const int64_t pieces = (all + target - 1) / target;
+    return (valptr[br] - v0) * pieces / all != (valptr[br - 1] - v0) * pieces / all;
 }
 
 __global__ void k_tile_flags(const int* __restrict__ valptr, int64_t nbr, int target, int maxbr,
                              int* __restrict__ flags) {
     const int64_t br = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (br >= nbr) return;
-    flags[br] = tile_starts(valptr, br, target, maxbr) ? 1 : 0;
+    flags[br] = tile_starts(valptr, br, nbr, target, maxbr) ? 1 : 0;
 }
 
-__global__ void k_tile_scatter(const int* __restrict__ valptr, int64_t nbr, int target, int maxbr,
-                               const int* __restrict__ idx, int64_t ntiles, int* __restrict__ tile_br,
-                               int* __restrict__ tile_val) {
+__global__ void k_tile_scatter(const int* __restrict__ valptr, const int* __restrict__ bptr, int64_t nbr, int target,
+                               int maxbr, const int* __restrict__ idx, int64_t ntiles, int4* __restrict__ tiles) {
     const int64_t br = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (br > nbr) return;
     if (br == nbr) {
-        tile_br[ntiles] = (int)nbr;
-        tile_val[ntiles] = valptr[nbr];
+        tiles[ntiles] = make_int4((int)nbr, bptr[nbr], valptr[nbr], 0);
         return;
     }
-    if (tile_starts(valptr, br, target, maxbr)) {
-        tile_br[idx[br]] = (int)br;
-        tile_val[idx[br]] = valptr[br];
+    if (tile_starts(valptr, br, nbr, target, maxbr)) {
+        tiles[idx[br]] = make_int4((int)br, bptr[br], valptr[br], 0);
     }
 }
 
 template <int R, int MB, int VS>
 void launch_blockrow_values(const spc5_hip_mat& m, int* cnt, int* err, hipStream_t s) {
     const unsigned g = (unsigned)((m.nbr + 255) / 256);  // 4 waves of 64 block-rows per workgroup
+    const unsigned every = g * 4 > 1024 ? g * 4 / 1024 : 1;  // about 1,000 sampled groups
     hipLaunchKernelGGL((k_blockrow_values<R, MB, VS>), dim3(g), dim3(256), 0, s, m.bptr, m.hdr, m.nbr, m.ncols, cnt,
-                       err);
+                       err, m.value_type == SPC5_HIP_F64 ? 8 : 4, every);
 }
 
 template <class V, class X, class ACC, int R, int VS, int MB, bool SORT>
@@ -252,13 +293,34 @@ void launch_tiles(const spc5_hip_mat& m, const void* x, void* y, hipStream_t s, 
     const unsigned grid = (unsigned)((groups + 7) / 8 * 8);
     hipLaunchKernelGGL((k_spmv_tiles<V, X, ACC, R, VS, MB, SORT>), dim3(grid), dim3(kWavesPerGroup * 64), 0, s,
                        m.bptr, m.hdr, reinterpret_cast<const V*>(m.values), reinterpret_cast<const X*>(x),
-                       reinterpret_cast<X*>(y), m.plan.tile_br->as<int>(), m.plan.tile_val->as<int>(),
-                       m.plan.ntiles, m.nrows, m.ncols, ep);
+                       reinterpret_cast<X*>(y), m.plan.tiles->as<int4>(), m.plan.ntiles, m.nrows,
+                       m.ncols, ep);
+}
+
+template <class V, class X, class ACC, int R, int VS, int MB>
+void launch_lanes(const spc5_hip_mat& m, const void* x, void* y, hipStream_t s, const Epilogue& ep) {
+    const int64_t groups = (m.plan.ntiles + kWavesPerGroup - 1) / kWavesPerGroup;
+    const unsigned grid = (unsigned)((groups + 7) / 8 * 8);
+    hipLaunchKernelGGL((k_spmv_lanes<V, X, ACC, R, VS, MB>), dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.bptr,
+                       m.hdr, reinterpret_cast<const V*>(m.values), reinterpret_cast<const X*>(x),
+                       reinterpret_cast<X*>(y), m.plan.tiles->as<int4>(), m.plan.ntiles, m.nrows, m.ncols, ep);
 }
 
 template <class V, class X, class ACC, int VS, int MB>
 int launch_spmv_vs(const spc5_hip_mat& m, const void* x, void* y, hipStream_t s, const Epilogue& ep) {
     const bool sort = m.row_sort != 0;
+    if constexpr (lane_block_fits(VS, sizeof(X))) {
+        if (m.lane_body) {
+            switch (m.r) {
+            case 1: launch_lanes<V, X, ACC, 1, VS, MB>(m, x, y, s, ep); break;
+            case 2: launch_lanes<V, X, ACC, 2, VS, MB>(m, x, y, s, ep); break;
+            case 4: launch_lanes<V, X, ACC, 4, VS, MB>(m, x, y, s, ep); break;
+            default: launch_lanes<V, X, ACC, 8, VS, MB>(m, x, y, s, ep); break;
+            }
+            SPC5_HIP_TRY(hipGetLastError());
+            return SPC5_HIP_OK;
+        }
+    }
     switch (m.r) {
     case 1: launch_tiles<V, X, ACC, 1, VS, MB, false>(m, x, y, s, ep); break;
     case 2:
@@ -321,8 +383,8 @@ int build_plan(spc5_hip_mat& m, hipStream_t s) {
     p.ntiles = 0;
     if (m.nbr == 0) return SPC5_HIP_OK;
     DeviceBuffer err;
-    SPC5_HIP_TRY(err.alloc(sizeof(int)));
-    SPC5_HIP_TRY(hipMemsetAsync(err.p, 0, sizeof(int), s));
+    SPC5_HIP_TRY(err.alloc(3 * sizeof(int)));  // flags, sampled lines, sampled blocks
+    SPC5_HIP_TRY(hipMemsetAsync(err.p, 0, 3 * sizeof(int), s));
     {
         const unsigned g = (unsigned)((m.nbr + 1 + 255) / 256);
         hipLaunchKernelGGL(k_check_bptr, dim3(g), dim3(256), 0, s, m.bptr, m.nbr, m.nblocks, err.as<int>());
@@ -357,8 +419,9 @@ int build_plan(spc5_hip_mat& m, hipStream_t s) {
     // Counts are < 2^31 each; the scan is checked against nnz below.
     int rc = scan_exclusive_i32(valptr, m.nbr + 1, dtotal.as<int>(), s);
     if (rc) return rc;
-    int herr = 0, hnnz = 0;
-    SPC5_HIP_TRY(hipMemcpyAsync(&herr, err.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    int hstat[3] = {0, 0, 0}, hnnz = 0;
+    const int& herr = hstat[0];
+    SPC5_HIP_TRY(hipMemcpyAsync(hstat, err.p, 3 * sizeof(int), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipMemcpyAsync(&hnnz, valptr + m.nbr, sizeof(int), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipStreamSynchronize(s));
     if (herr) {
@@ -369,16 +432,52 @@ int build_plan(spc5_hip_mat& m, hipStream_t s) {
         set_error("nnz (" + std::to_string(m.nnz) + ") differs from the mask popcount (" + std::to_string(hnnz) + ")");
         return SPC5_HIP_ERR_INVALID;
     }
-    return build_tiles(m, p, kMaxRows, default_tile_values(m.nnz), s);
+    m.scatter = hstat[2] > 0 ? (double)hstat[1] / hstat[2] : 0.0;
+    m.lane_body = lane_block_wins(m);
+    return build_tiles(m, p, tile_rows(m.r), default_tile_values(m.nnz), s);
 }
 
-// Values per tile aimed at when no tile size is set: about 8192 tiles, at
-// least 512 and at most 8192 values each (a tile also ends every
-// kMaxRows rows).
+// Which tile a product runs: lane-block (one block per lane, spmv_lane.hpp)
+// or value-order (spmv_tile.hpp).  The lane-block tile costs a fixed number of
+// instructions per block position and one or more 16-byte x loads per block;
+// the value-order tile costs about three times as many instructions per value
+// but gathers x with fewer distinct lines per request.  So the line is drawn
+// on `scatter`, the distinct 128-byte lines of x per block among 64 blocks in a
+// row: stencils, banded matrices and Laplacians have 0.04 .. 0.41, the
+// clustered matrix 0.52 .. 0.97 (value-order / lane-block, us):
+//   27-point stencil 128^3, scatter 0.2: float beta(2,16) 101 / 66, bfloat16
+//     beta(2,8) 95 / 53, double beta(2,8) 121 / 108
+//   banded 100,000 rows, half-width 130, scatter 0.14 .. 0.27: float beta(4,16)
+//     29 / 19, double beta(4,8) 28 / 21
+//   clustered 1 M rows, scatter 0.8 .. 0.97: double beta(1,8) 88 / 102, float
+//     beta(2,16) 61 / 66, but bfloat16 beta(2,8) 66 / 55
+//   clustered 60,000 rows (x and matrix in the L2s): double beta(2,8) 10.5 /
+//     8.6, float beta(4,16) 11.5 / 10.2, double beta(4,8) 10.4 / 11.4
+// Double blocks of 8 rows (64 positions of 8 bytes, mostly empty) stay in value
+// order: Laplacian 1400^2 37 / 47, stencil 128^3 149 / 176.
+bool lane_block_wins(const spc5_hip_mat& m) {
+    if ((uint64_t)m.ncols * 8 > 0xffffffffull || m.ncols < 16) return false;  // 32-bit x offsets, a whole window
+    const bool f64 = m.value_type == SPC5_HIP_F64;
+    if (f64 && m.r == 8) return false;
+    if (m.scatter < 0.48) return true;
+    const bool small = m.nnz < (4 << 20);
+    if (f64) return m.r <= 2 && small;
+    if (m.value_type == SPC5_HIP_F32 && m.vs == 16) return m.r <= 4 && small;
+    return m.r <= 2 || (m.r == 4 && small);
+}
+
+// Values per tile aimed at when no tile size is set (a tile also ends every
+// tile_rows(r) rows).  Small matrices need many waves more than long ones (at
+// 128 values the 64^2 Laplacian takes 3.2 us, at 512 4.2 us, double beta(2,8));
+// large ones have 8,192 tiles or more whatever the size, and 2,048 values are
+// short enough to even out uneven rows (clustered 1 M rows, double beta(1,8):
+// 2,048 values 84 us, 4,096 values 94 us).
 int default_tile_values(int64_t nnz) {
-    int64_t target = nnz / 8192;
-    if (target < 512) target = 512;
-    if (target > 8192) target = 8192;
+    int64_t target = nnz / 2048;
+    if (target < 128) target = 128;
+    if (target > 512) target = 512;
+    if (target < nnz / 8192) target = nnz / 8192;
+    if (target > 2048) target = 2048;
     return (int)target;
 }
 
@@ -406,12 +505,10 @@ int build_tiles(const spc5_hip_mat& m, Plan& p, int maxrows, int target, hipStre
     SPC5_HIP_TRY(hipMemcpyAsync(&hn, dtotal.p, sizeof(int), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipStreamSynchronize(s));
     p.ntiles = hn;
-    p.tile_br = std::make_shared<DeviceBuffer>();
-    p.tile_val = std::make_shared<DeviceBuffer>();
-    SPC5_HIP_TRY(p.tile_br->alloc(sizeof(int) * (size_t)(hn + 1)));
-    SPC5_HIP_TRY(p.tile_val->alloc(sizeof(int) * (size_t)(hn + 1)));
-    hipLaunchKernelGGL(k_tile_scatter, dim3(g), dim3(256), 0, s, valptr, m.nbr, p.target, maxbr, flags.as<int>(),
-                       (int64_t)hn, p.tile_br->as<int>(), p.tile_val->as<int>());
+    p.tiles = std::make_shared<DeviceBuffer>();
+    SPC5_HIP_TRY(p.tiles->alloc(sizeof(int4) * (size_t)(hn + 1)));
+    hipLaunchKernelGGL(k_tile_scatter, dim3(g), dim3(256), 0, s, valptr, m.bptr, m.nbr, p.target, maxbr,
+                       flags.as<int>(), (int64_t)hn, p.tiles->as<int4>());
     SPC5_HIP_TRY(hipGetLastError());
     SPC5_HIP_TRY(hipStreamSynchronize(s));
     return SPC5_HIP_OK;
@@ -467,6 +564,7 @@ int spc5_hip_mat_create_values_view(spc5_hip_mat_t base, int value_type, const v
     std::unique_ptr<spc5_hip_mat> m(new spc5_hip_mat(*base));
     m->value_type = value_type;
     m->values = d_values;
+    m->lane_body = lane_block_wins(*m);
     *out = m.release();
     return SPC5_HIP_OK;
 }
@@ -507,7 +605,7 @@ int spc5_hip_mat_set_option(spc5_hip_mat_t h, int option, int64_t value) {
         if (h->nbr == 0 || target == h->plan.target) return SPC5_HIP_OK;
         Plan np;
         np.valptr = h->plan.valptr;
-        const int rc = build_tiles(*h, np, kMaxRows, target, nullptr);
+        const int rc = build_tiles(*h, np, tile_rows(h->r), target, nullptr);
         if (rc) return rc;
         h->plan = np;  // shared buffers of the old plan stay alive while views or batches use them
         return SPC5_HIP_OK;
@@ -531,20 +629,19 @@ int spc5_hip_access_probe(spc5_hip_mat_t h, int mode, const void* d_x, void* d_o
     const double* xv = reinterpret_cast<const double*>(d_x);
     const double* vv = reinterpret_cast<const double*>(m.values);
     double* o = reinterpret_cast<double*>(d_out);
-    const int* tb = m.plan.tile_br->as<int>();
-    const int* tv = m.plan.tile_val->as<int>();
+    const int4* tl = m.plan.tiles->as<int4>();
     hipStream_t s = as_stream(stream);
     switch (mode) {
     case 0:
-        hipLaunchKernelGGL(k_access_probe<0>, dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.bptr, m.hdr, vv, xv, tb, tv,
+        hipLaunchKernelGGL(k_access_probe<0>, dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.hdr, vv, xv, tl,
                            m.plan.ntiles, m.ncols, o);
         break;
     case 1:
-        hipLaunchKernelGGL(k_access_probe<1>, dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.bptr, m.hdr, vv, xv, tb, tv,
+        hipLaunchKernelGGL(k_access_probe<1>, dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.hdr, vv, xv, tl,
                            m.plan.ntiles, m.ncols, o);
         break;
     default:
-        hipLaunchKernelGGL(k_access_probe<2>, dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.bptr, m.hdr, vv, xv, tb, tv,
+        hipLaunchKernelGGL(k_access_probe<2>, dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.hdr, vv, xv, tl,
                            m.plan.ntiles, m.ncols, o);
         break;
     }

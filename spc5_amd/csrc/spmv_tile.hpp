@@ -572,8 +572,8 @@ template <class V, class X, class ACC, int R, int VS, int MB, bool kSort, bool k
 __device__ __forceinline__ void spmv_tile_body(TileSmem<ACC, R, expand_cap<V>(), kSort>& sm,
                                                const int* __restrict__ bptr,
                                                const unsigned char* __restrict__ hdr, const V* __restrict__ val,
-                                               const X* __restrict__ x, X* __restrict__ y, int br0, int br1,
-                                               int vstart, int vend, int64_t nrows, const Epilogue& ep) {
+                                               const X* __restrict__ x, X* __restrict__ y, int4 first, int4 last,
+                                               int64_t nrows, const Epilogue& ep) {
     constexpr int CAP = expand_cap<V>();
     constexpr int K = CAP / 64;  // batch positions owned by one lane in the row sums
     constexpr int NW = MaskWords<R * MB>::kWords;
@@ -582,14 +582,11 @@ __device__ __forceinline__ void spmv_tile_body(TileSmem<ACC, R, expand_cap<V>(),
     const int lane = lane_id();
     // The tile bounds are the same on every lane (the tile index comes from
     // the wave index, which the compiler cannot tell is uniform).
-    br0 = __builtin_amdgcn_readfirstlane(br0);
-    br1 = __builtin_amdgcn_readfirstlane(br1);
-    vstart = __builtin_amdgcn_readfirstlane(vstart);
-    vend = __builtin_amdgcn_readfirstlane(vend);
+    const int br0 = __builtin_amdgcn_readfirstlane(first.x), br1 = __builtin_amdgcn_readfirstlane(last.x);
+    const int b0 = __builtin_amdgcn_readfirstlane(first.y), b1 = __builtin_amdgcn_readfirstlane(last.y);
+    const int vstart = __builtin_amdgcn_readfirstlane(first.z), vend = __builtin_amdgcn_readfirstlane(last.z);
 
     const int nbr = br1 - br0;
-    const int b0 = bptr[br0];
-    const int b1 = bptr[br1];
     int v = vstart;
     const int64_t row0 = (int64_t)br0 * R;
     const int64_t rows_left = nrows - row0;
@@ -662,14 +659,12 @@ template <class V, class X, class ACC, int R, int VS, int MB, bool kSort = false
 __device__ __forceinline__ void spmv_tile(TileSmem<ACC, R, expand_cap<V>(), kSort>& sm,
                                           const int* __restrict__ bptr,
                                           const unsigned char* __restrict__ hdr, const V* __restrict__ val,
-                                          const X* __restrict__ x, X* __restrict__ y, int br0, int br1, int vstart,
-                                          int vend, int64_t nrows, int64_t ncols, const Epilogue& ep) {
+                                          const X* __restrict__ x, X* __restrict__ y, int4 first, int4 last,
+                                          int64_t nrows, int64_t ncols, const Epilogue& ep) {
     if (SPC5_X32 && (uint64_t)ncols * sizeof(X) <= 0xffffffffull)
-        spmv_tile_body<V, X, ACC, R, VS, MB, kSort, false>(sm, bptr, hdr, val, x, y, br0, br1, vstart, vend, nrows,
-                                                           ep);
+        spmv_tile_body<V, X, ACC, R, VS, MB, kSort, false>(sm, bptr, hdr, val, x, y, first, last, nrows, ep);
     else
-        spmv_tile_body<V, X, ACC, R, VS, MB, kSort, true>(sm, bptr, hdr, val, x, y, br0, br1, vstart, vend, nrows,
-                                                          ep);
+        spmv_tile_body<V, X, ACC, R, VS, MB, kSort, true>(sm, bptr, hdr, val, x, y, first, last, nrows, ep);
 }
 
 }  // namespace spc5

@@ -222,8 +222,10 @@ class DeviceMatrix:
 
     def tile_target(self) -> int:
         """Values per tile the current plan aims at (the set tile size, or
-        the default rule nnz / 8192 clamped to [512, 8192])."""
-        return self.tile_values or min(8192, max(512, self.nnz // 8192))
+        the default rule of spc5_hip_mat_set_option)."""
+        if self.tile_values:
+            return self.tile_values
+        return min(2048, max(128, min(512, self.nnz // 2048), self.nnz // 8192))
 
     @property
     def format_name(self):
