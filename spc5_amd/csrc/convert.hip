@@ -33,24 +33,39 @@ __global__ void k_check_rowptr(const int* __restrict__ rowptr, int64_t nrows, in
 }
 
 // Groups: one wave converts kGroupRows = 64 consecutive rows, one lane per
-// row; the r lanes of a block-row form a lane group.  For every block the
-// group agrees on its start (the minimum of the r row heads, a shuffle
-// reduction), each lane consumes its own row's columns inside the block's
-// window, and a group prefix sum of the counts places the values (row-major
-// inside the block).  The group's column indices are staged in LDS with
-// coalesced loads when they fit the stage; the fill pass builds the group's
-// packed headers and a destination map of its values in LDS and writes both
-// out with coalesced stores.  A group too large for the stage reads its
-// columns from global memory and writes directly (the same arithmetic).
+// row; the r lanes of a block-row form a lane group.  The group's column
+// indices are staged in LDS with coalesced loads, the first entry of every row
+// replaced by a value larger than any column (its lane keeps the column), so
+// that a window of a row always ends at the row's end.  Per block
+// (walk_staged):
+//   * every lane reads the next VS entries of its row; the first is its head,
+//     and the block starts at the minimum of the r heads (DPP);
+//   * one median per entry clamps the window to [.., start + VS) and carries
+//     the clamp past the first entry outside, and one shift-or per entry
+//     collects the bits modulo 32; a rotation by the start gives the row mask,
+//     its popcount the lane's values in the block.
+// The fill pass stores each header as it is made and leaves, at the stage
+// position of the lane's first value in the block, the distance from source to
+// destination; a last pass reads the values in CSR order and every lane takes
+// the distance of the last such position at or before it.  (With r = 1 the
+// values keep their order.)
 //
-// The stage is dynamic LDS sized at launch from the matrix's mean values and
-// header bytes per group (half as much again as the mean, at least 256 more):
-// a small stage keeps many waves resident per CU, which hides the latency of
-// each wave's few dependent memory round trips.
+// What bounds it: the chain of one LDS round trip and about 30 instructions per
+// block, as long as the longest block-row of the wave, with the waves per CU
+// that the staged columns leave room for; then HBM in the fill.  Clustered
+// matrix of 1 M rows, double beta(4,8): count 200 -> 104 us, fill 476 -> 200 us
+// (before: a chain of compares and selects per window entry, VS LDS writes of
+// destinations per lane and block, and 96 registers of prefetched values).
+//
+// A group too large for the stage reads its columns from global memory and
+// writes directly (walk_group).
+//
+// The stage is dynamic LDS sized at launch from the matrix's mean values per
+// group (half as much again as the mean, at least 256 more): a small stage
+// keeps many waves resident per CU.
 constexpr int kGroupRows = 64;
 constexpr int kPrefetch = 32;             // words per lane loaded at once: 2048 per group
 constexpr int kMaxStageValues = 8192;     // 32 KiB of staged columns
-constexpr int kMaxStageHdrBytes = 16384;  // staged header bytes
 constexpr int kStagePad = 32;             // words after the staged columns read by the walk's windows
 
 template <int R>
@@ -64,14 +79,6 @@ int stage_values(int64_t nnz, int64_t ngroups) {
     int64_t s = round_up64(avg + (avg / 2 > 256 ? avg / 2 : 256));
     if (s < 512) s = 512;
     return (int)(s < kMaxStageValues ? s : kMaxStageValues);
-}
-
-// Staged header bytes per group, by the same rule.
-int stage_header_bytes(int64_t nblocks, int h, int64_t ngroups) {
-    const int64_t avg = ngroups > 0 ? (nblocks * h + ngroups - 1) / ngroups : 0;
-    int64_t s = round_up64(avg + (avg / 2 > 256 ? avg / 2 : 256));
-    if (s < 512) s = 512;
-    return (int)(s < kMaxStageHdrBytes ? s : kMaxStageHdrBytes);
 }
 
 // Lane-group collectives over R = 1, 2, 4 or 8 consecutive lanes, as DPP
@@ -94,6 +101,13 @@ __device__ __forceinline__ int group_min(int v) {
     if constexpr (R >= 2) v = min(v, dpp_i32<kDppQuadXor1>(v));
     if constexpr (R >= 4) v = min(v, dpp_i32<kDppQuadXor2>(v));
     if constexpr (R >= 8) v = min(v, dpp_i32<kDppRowHalfMirror>(v));
+    return v;
+}
+template <int R>
+__device__ __forceinline__ unsigned group_min(unsigned v) {
+    if constexpr (R >= 2) v = min(v, (unsigned)dpp_i32<kDppQuadXor1>((int)v));
+    if constexpr (R >= 4) v = min(v, (unsigned)dpp_i32<kDppQuadXor2>((int)v));
+    if constexpr (R >= 8) v = min(v, (unsigned)dpp_i32<kDppRowHalfMirror>((int)v));
     return v;
 }
 template <int R>
@@ -122,31 +136,27 @@ __device__ __forceinline__ int group_excl_scan(int v, int t) {
     return incl - v;
 }
 
-// Walks the block-rows of a group; for each block of a lane's block-row
-// calls on_block(k, start, t, first, n, mask, src0) on every lane of the
-// group: k is the block's index in its block-row, t the lane's row in the
-// block, first the value position (block order) of the lane's first value in
-// the block, n its count and mask its VS-bit row mask; the lane's values were
-// at source positions [src0, src0 + n), whose columns the walk never reads
-// again.  With CHECK, returns whether a lane saw columns that break the
-// format's precondition (non-negative, strictly increasing); without, the
-// caller has checked them and it returns false.
+// Walks the block-rows of a group over global columns; for each block of a
+// lane's block-row calls on_block(k, start, t, first, n, mask, src0) on every
+// lane of the group: k is the block's index in its block-row, t the lane's row
+// in the block, first the value position (block order) of the lane's first
+// value in the block, n its count and mask its VS-bit row mask; the lane's
+// values are at source positions [src0, src0 + n).  With CHECK, returns whether
+// a lane saw columns that break the format's precondition (non-negative,
+// strictly increasing); without, the caller has checked them and it returns
+// false.
 //
-// `col` is indexed by global value position minus `base` (0 for the global
-// array, the group's first value for the stage).  Per block a lane reads the
-// window of its next VS + 1 columns at once: its values in the block are the
-// window's leading run below start + VS (at most VS, the columns being
-// strictly increasing), the entry after them is the next head, and adjacent
-// window entries check the precondition (CHECK).  PADDED: `col` may be read up to
-// VS + 1 entries past the group's last value (the stage's pad), so the window
-// is read without clamping; otherwise each index is clamped to the row.
-template <int R, int VS, bool PADDED, bool CHECK, class C, class F>
-__device__ __forceinline__ bool walk_group(int rb, int re, C col, int base, F on_block) {
+// Per block a lane reads the window of its next VS + 1 columns at once (clamped
+// to the row): its values in the block are the window's leading run below
+// start + VS (at most VS, the columns being strictly increasing), the entry
+// after them is the next head, and adjacent entries check the precondition.
+template <int R, int VS, bool CHECK, class F>
+__device__ __forceinline__ bool walk_group(int rb, int re, const int* __restrict__ col, F on_block) {
     const int lane = threadIdx.x;
     const int t = lane % R;
     const int end = re;
     int cur = rb;
-    int head = cur < end ? col[cur - base] : INT_MAX;  // INT_MAX once the row is consumed
+    int head = cur < end ? col[cur] : INT_MAX;  // INT_MAX once the row is consumed
     bool bad = CHECK && head < 0;
     // the block-row's first value: the row pointer of its row 0
     int vbase = __shfl(rb, lane - t, 64);
@@ -156,15 +166,9 @@ __device__ __forceinline__ bool walk_group(int rb, int re, C col, int base, F on
         if (!ballot64(start != INT_MAX)) break;  // every block-row of the wave is done
         if (start != INT_MAX) {
             int w[VS + 1];
-            if constexpr (PADDED) {
-                const auto p = col + (cur - base);
+            const int last = end - 1 > cur ? end - 1 : cur;
 #pragma unroll
-                for (int j = 0; j <= VS; ++j) w[j] = p[j];
-            } else {
-                const int last = end - 1 > cur ? end - 1 : cur;
-#pragma unroll
-                for (int j = 0; j <= VS; ++j) w[j] = cur < end ? col[(cur + j < last ? cur + j : last) - base] : 0;
-            }
+            for (int j = 0; j <= VS; ++j) w[j] = cur < end ? col[cur + j < last ? cur + j : last] : 0;
             unsigned mask = 0;
             int n = 0;
             bool alive = true;
@@ -191,26 +195,6 @@ __device__ __forceinline__ bool walk_group(int rb, int re, C col, int base, F on
         }
     }
     return bad;
-}
-
-// Coalesced copy of n words to LDS, 8 loads in flight per lane per step (a
-// load-then-store loop would wait for every load in turn).
-template <class T>
-__device__ __forceinline__ void stage_words(const T* __restrict__ src, T* dst, int n, int lane) {
-    constexpr int U = 8;
-    for (int i0 = 0; i0 < n; i0 += 64 * U) {
-        T v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = i0 + lane + 64 * u;
-            v[u] = i < n ? src[i] : T(0);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = i0 + lane + 64 * u;
-            if (i < n) dst[i] = v[u];
-        }
-    }
 }
 
 // Raw buffer loads of one word type (a read past the resource's range
@@ -253,17 +237,92 @@ __device__ __forceinline__ void prefetch_words(const T* __restrict__ src, int n,
     for (int u = 0; u < kPrefetch; ++u) v[u] = RawWord<T>::get(r, (lane + 64 * u) * (int)sizeof(T));
 }
 
-// Stages n column indices in LDS: the first 64 kPrefetch from registers
-// already loaded, the rest with stage_words.
-__device__ __forceinline__ void stage_columns(const int* __restrict__ src, int* dst, int n, int lane,
-                                              const int (&v)[kPrefetch]) {
+// Stage entries that are no column: the first of every row, and (from
+// kMovedBase) the first value of a row's part of a block, once the walk has
+// left the distance to its destination there.  Both exceed every block's end.
+constexpr unsigned kRowStart = 0xffffffffu;
+constexpr unsigned kMovedBase = 0xc0000000u;
+constexpr int kMovedZero = 1 << 16;  // encodes distance 0
+
+// Stages n column indices in LDS, 64 kPrefetch at a time; true where a lane
+// saw a negative one.
+__device__ __forceinline__ bool stage_columns(const int* __restrict__ src, unsigned* dst, int n, int lane) {
+    bool bad = false;
+    for (int i0 = 0; i0 < n; i0 += 64 * kPrefetch) {
+        int v[kPrefetch];
+        prefetch_words(src + i0, n - i0, lane, v);
 #pragma unroll
-    for (int u = 0; u < kPrefetch; ++u) {
-        const int i = lane + 64 * u;
-        if (i < n) dst[i] = v[u];
+        for (int u = 0; u < kPrefetch; ++u) {
+            const int i = i0 + lane + 64 * u;
+            if (64 * u < n - i0) {
+                if (i < n) dst[i] = (unsigned)v[u];
+                bad |= v[u] < 0;
+            }
+        }
     }
-    if (n > 64 * kPrefetch) stage_words(src + 64 * kPrefetch, dst + 64 * kPrefetch, n - 64 * kPrefetch, lane);
+    if (lane == 0) dst[n] = kRowStart;
     wave_sync();
+    return bad;
+}
+
+// The row starts marked in the stage; returns the column of the lane's first
+// entry (kRowStart for an empty row).  CHECK: *bad is set where the columns of
+// a row do not strictly increase.
+template <bool CHECK>
+__device__ __forceinline__ unsigned mark_rows(unsigned* scol, int cur, int end, int n, int lane, bool* bad) {
+    const unsigned first = cur < end ? scol[cur] : kRowStart;
+    if (CHECK && cur + 1 < end) *bad |= scol[cur + 1] <= first;
+    wave_sync();
+    if (cur < end) scol[cur] = kRowStart;
+    wave_sync();
+    if constexpr (CHECK) {
+#pragma unroll 4
+        for (int i = lane; i < n; i += 64) {
+            const unsigned c0 = scol[i], c1 = scol[i + 1];
+            *bad |= c0 != kRowStart && c1 <= c0;
+        }
+    }
+    return first;
+}
+
+// Walks the block-rows of a staged group: [cur, end) are the lane's stage
+// positions and `first` its first column.  Calls on_block(k, more, start, n,
+// mask, src) on every lane; `more` where the block-row has a k-th block: n
+// values from stage position src on, with the row mask `mask`.  MOVED: on_block leaves moved marks
+// in the stage.  At most nv steps, whatever the columns.
+template <int R, int VS, bool MOVED, class F>
+__device__ __forceinline__ void walk_staged(const unsigned* scol, int cur, unsigned first, int nv, F on_block) {
+    const int begin = cur;
+    const int steps = __builtin_amdgcn_readfirstlane(nv);
+    for (int k = 0; k < steps; ++k) {
+        unsigned w[VS];
+#pragma unroll
+        for (int j = 0; j < VS; ++j) w[j] = scol[cur + j];
+        // the whole window in one LDS round trip (the reads would otherwise
+        // sink below the start they do not need)
+#pragma unroll
+        for (int j = 0; j < VS; ++j) asm volatile("" : "+v"(w[j]));
+        // past the row's end: the mark at the start of the next row
+        const unsigned next = MOVED && w[0] >= kMovedBase ? kRowStart : w[0];
+        const unsigned head = cur == begin ? first : next;
+        const unsigned start = group_min<R>(head);
+        const bool more = start != kRowStart;
+        if (!ballot64(more)) break;
+        // entries clamped to the block's end; the first one outside and all
+        // that follow it count as the end
+        const unsigned lim = start + VS;
+        unsigned q = head < lim ? head : lim;
+        unsigned bits = 1u << (q & 31u);
+#pragma unroll
+        for (int j = 1; j < VS; ++j) {
+            asm("v_med3_u32 %0, %1, %2, %3" : "=v"(q) : "v"(q), "v"(w[j]), "v"(lim));
+            bits |= 1u << (q & 31u);
+        }
+        const unsigned mask = __builtin_amdgcn_alignbit(bits, bits, start & 31u) & ((1u << VS) - 1u);
+        const int n = more ? __popc(mask) : 0;
+        on_block(k, more, start, n, mask, cur);
+        cur += n;
+    }
 }
 
 // A group's rows, one per lane: [rb, re) are the lane's values (rows past the
@@ -282,172 +341,175 @@ __device__ __forceinline__ GroupRows group_rows(const int* __restrict__ rowptr, 
     return g;
 }
 
-// Row-start bitmap words after a stage of sv values (bit i: value i starts
-// a row; one spare word).
-__host__ __device__ constexpr int row_start_words(int sv) { return sv / 32 + 2; }
-
-// The column precondition over a group's staged columns (non-negative,
-// strictly increasing inside each row), one coalesced pass: value i and its
-// successor are compared unless the successor starts a row, as the lanes mark
-// their rows' first values in the bitmap `rs`.  True when broken.
-__device__ __forceinline__ bool staged_columns_bad(const int* scol, unsigned* rs, int nv, int rb, int re, int v0,
-                                                   int lane) {
-    const int nw = nv / 32 + 2;
-    for (int i = lane; i < nw; i += 64) rs[i] = 0u;
-    wave_sync();
-    if (rb < re) atomicOr(&rs[(rb - v0) >> 5], 1u << ((rb - v0) & 31));
-    wave_sync();
-    bool bad = false;
-#pragma unroll 4
-    for (int i = lane; i < nv; i += 64) {
-        const int c0 = scol[i];
-        const int c1 = scol[i + 1];  // the stage's pad when i + 1 == nv
-        const bool next_starts_row = i + 1 >= nv || ((rs[(i + 1) >> 5] >> ((i + 1) & 31)) & 1u);
-        bad |= c0 < 0 || (!next_starts_row && c1 <= c0);
+// The next run of a group's rows, from row `lo` on, that is converted at once:
+// all of them, or the largest aligned half, quarter, ... whose values fit the
+// stage of sv (down to one block-row, which may not fit).  Lanes of other rows
+// hold empty ones.  A group read from global memory instead takes two memory
+// round trips per block, and a few such groups outlast all others: on the
+// clustered matrix one group in a thousand exceeds 1.5 times the mean.
+struct RowRun {
+    int rows;        // rows of the run
+    int rb, re;      // the lane's values
+    int v0, nv;      // the run's
+};
+template <int R>
+__device__ __forceinline__ RowRun row_run(const GroupRows& g, int lo, int sv, int lane) {
+    RowRun p;
+    p.rows = lo == 0 ? kGroupRows : lo & -lo;
+    p.v0 = __builtin_amdgcn_readlane(g.rb, lo);
+    for (;;) {
+        p.nv = __builtin_amdgcn_readlane(g.re, lo + p.rows - 1) - p.v0;
+        if (p.nv <= sv || p.rows == R) break;
+        p.rows >>= 1;
     }
-    return bad;
+    const bool mine = lane >= lo && lane < lo + p.rows;
+    p.rb = mine ? g.rb : p.v0;
+    p.re = mine ? g.re : p.v0;
+    return p;
 }
 
 // Blocks per block-row (the count pass).  A violation of the column
 // precondition sets bit 0 of *err; the fill pass is then never run.  Dynamic
-// LDS: sv staged column indices, kStagePad words of pad, then
-// row_start_words(sv) words of row-start bitmap.
+// LDS: sv staged column indices and kStagePad words of pad.
 template <int R, int VS>
 __global__ __launch_bounds__(64) void k_convert_count(int64_t nrows, int64_t nbr, const int* __restrict__ rowptr,
                                                       const int* __restrict__ col, int* __restrict__ cnt_out,
                                                       int* __restrict__ err, int sv) {
     constexpr int BR = group_blockrows<R>();
     extern __shared__ __align__(16) unsigned char smem[];
-    int* scol = reinterpret_cast<int*>(smem);
-    unsigned* rstart = reinterpret_cast<unsigned*>(smem + 4 * (size_t)(sv + kStagePad));
+    unsigned* scol = reinterpret_cast<unsigned*>(smem);
     const int lane = threadIdx.x;
     const int64_t br0 = (int64_t)blockIdx.x * BR;
     const GroupRows g = group_rows(rowptr, br0 * R, nrows, lane);
     int nb = 0;
-    auto on_block = [&](int, int, int, int, int, unsigned, int) { ++nb; };
     bool bad = false;
-    if (g.nv <= sv) {
-        if (g.nv > 0) {
-            int c[kPrefetch];
-            prefetch_words(col + g.v0, g.nv, lane, c);
-            stage_columns(col + g.v0, scol, g.nv, lane, c);
-            bad = staged_columns_bad(scol, rstart, g.nv, g.rb, g.re, g.v0, lane);
+    for (int lo = 0; lo < kGroupRows;) {
+        const RowRun p = row_run<R>(g, lo, sv, lane);
+        lo += p.rows;
+        if (p.nv == 0) continue;
+        if (p.nv <= sv) {
+            bad |= stage_columns(col + p.v0, scol, p.nv, lane);
+            const unsigned first = mark_rows<true>(scol, p.rb - p.v0, p.re - p.v0, p.nv, lane, &bad);
+            if (!ballot64(bad))
+                walk_staged<R, VS, false>(scol, p.rb - p.v0, first, p.nv,
+                                          [&](int, bool more, unsigned, int, unsigned, int) { nb += more ? 1 : 0; });
+            wave_sync();
+        } else {
+            bad |= walk_group<R, VS, true>(p.rb, p.re, col, [&](int, int, int, int, int, unsigned, int) { ++nb; });
         }
-        walk_group<R, VS, true, false>(g.rb, g.re, scol, g.v0, on_block);
-    } else {
-        bad = walk_group<R, VS, false, true>(g.rb, g.re, col, 0, on_block);
     }
     const int64_t br = br0 + lane / R;
     if (lane % R == 0 && br < nbr) cnt_out[br] = nb;
     if (bad) atomicOr(err, 1);
 }
 
-// Headers and values of the groups' blocks.  Dynamic LDS: sv staged column
-// indices (and kStagePad words of pad), overwritten in place by the
-// destination of each value once the walk has consumed its column, then
-// shb + 4 header bytes (the group's headers, offset by the byte alignment of
-// their destination).
+// Header of one block, the lanes of its block-row together: lane t = 0 writes
+// the first column, and the r masks are gathered into whole dwords by DPP.
+template <int R, int VS, int MB>
+__device__ __forceinline__ void store_header(unsigned char* h, unsigned start, unsigned mask, int t) {
+    constexpr int LPD = 4 / MB;  // lanes per dword of masks
+    unsigned m = mask << (8 * MB * (t % LPD));
+    if constexpr (R >= 2) m |= (unsigned)dpp_i32<kDppQuadXor1>((int)m);
+    if constexpr (R >= 4 && LPD == 4) m |= (unsigned)dpp_i32<kDppQuadXor2>((int)m);
+    if constexpr (R * MB <= 4) {
+        if (t == 0) {
+            if constexpr (R * MB == 4) {
+                const uint2 both = make_uint2(start, m);
+                __builtin_memcpy(h, &both, 8);
+            } else {
+                __builtin_memcpy(h, &start, 4);
+                __builtin_memcpy(h + 4, &m, R * MB);
+            }
+        }
+    } else {
+        if (t == 0) __builtin_memcpy(h, &start, 4);
+        if (t % LPD == 0) __builtin_memcpy(h + 4 + t * MB, &m, 4);
+    }
+}
+
+// Headers and values of the groups' blocks.  Dynamic LDS as the count pass.
 template <class W, int R, int VS, int MB>
 __global__ __launch_bounds__(64) void k_convert_fill(int64_t nrows, int64_t nbr, const int* __restrict__ rowptr,
                                                      const int* __restrict__ col, const W* __restrict__ vin,
                                                      const int* __restrict__ bptr, int64_t nblocks,
-                                                     unsigned char* __restrict__ hdr, W* __restrict__ vout, int sv,
-                                                     int shb) {
+                                                     unsigned char* __restrict__ hdr, W* __restrict__ vout, int sv) {
     constexpr int BR = group_blockrows<R>();
     constexpr int H = 4 + R * MB;
+    constexpr int U = 8;  // values per lane in flight
     extern __shared__ __align__(16) unsigned char smem[];
-    int* scol = reinterpret_cast<int*>(smem);  // columns, then value destinations
-    unsigned char* shdr = smem + 4 * (size_t)(sv + kStagePad);
+    unsigned* scol = reinterpret_cast<unsigned*>(smem);
     const int lane = threadIdx.x;
+    const int t = lane % R;
     const int64_t br0 = (int64_t)blockIdx.x * BR;
     const int64_t br = br0 + lane / R;
     // row pointers and block-row pointers, loaded together
     const GroupRows g = group_rows(rowptr, br0 * R, nrows, lane);
     const int b_lo = bptr[br < nbr ? br : nbr];
     const int b_hi = bptr[br + 1 < nbr ? br + 1 : nbr];
-    const int64_t blk0 = __shfl(b_lo, 0, 64);
-    const int64_t b_last = __shfl(b_hi, 63, 64);  // pointer past the group's last block-row
-    const int64_t blkE = b_last < nblocks ? b_last : nblocks;
-    int nblk = 0, bo = 0;  // blocks of the lane's block-row, its first block's index in the group
-    if (br < nbr) {
-        const int64_t b_end = b_hi < nblocks ? b_hi : nblocks;
-        nblk = (int)(b_end > b_lo ? b_end - b_lo : 0);
-        bo = (int)(b_lo - blk0);
-    }
-    const int64_t g0 = blk0 * H, g1 = (blkE > blk0 ? blkE : blk0) * H;  // the group's header bytes
-    const int align = (int)(g0 & 3);
-    const int v0 = g.v0, nv = g.nv;
-    const bool staged = nv <= sv && (g1 - g0) + align <= shb;
-    if (!staged) {
-        // too large for the stage: global columns, direct writes
-        walk_group<R, VS, false, false>(g.rb, g.re, col, 0, [&](int k, int start, int tt, int first, int n,
-                                                                 unsigned mask, int src0) {
-            if (k >= nblk) return;  // inconsistent pointers: never write past the block-row
-            unsigned char* h = hdr + (blk0 + bo + k) * H;
-            if (tt == 0) __builtin_memcpy(h, &start, 4);
-            __builtin_memcpy(h + 4 + tt * MB, &mask, MB);
-            for (int j = 0; j < n; ++j) vout[first + j] = vin[src0 + j];
+    // blocks of the lane's block-row: never written past, whatever the pointers
+    const int64_t b_end = b_hi < nblocks ? b_hi : nblocks;
+    const int nblk = br < nbr && b_end > b_lo ? (int)(b_end - b_lo) : 0;
+    unsigned char* h = hdr + (int64_t)b_lo * H;
+    for (int lo = 0; lo < kGroupRows;) {
+        const RowRun p = row_run<R>(g, lo, sv, lane);
+        lo += p.rows;
+        const int v0 = p.v0, nv = p.nv;
+        if (nv == 0) continue;
+        if (nv > sv) {
+            // too large for the stage: global columns, direct writes
+            walk_group<R, VS, false>(p.rb, p.re, col, [&](int k, int start, int tt, int first, int n, unsigned mask,
+                                                          int src0) {
+                if (k >= nblk) return;
+                store_header<R, VS, MB>(h + (int64_t)k * H, (unsigned)start, mask, tt);
+                for (int j = 0; j < n; ++j) vout[first + j] = vin[src0 + j];
+            });
+            continue;
+        }
+        (void)stage_columns(col + v0, scol, nv, lane);
+        bool unused = false;
+        const unsigned first = mark_rows<false>(scol, p.rb - v0, p.re - v0, nv, lane, &unused);
+        W v[U];
+        auto load = [&](int i0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = i0 + lane + 64 * u;
+                v[u] = vin[v0 + (i < nv ? i : nv - 1)];
+            }
+        };
+        load(0);  // in flight across the walk
+        int at = __shfl(p.rb, lane - t, 64) - v0;  // destination of the block-row's next value
+        walk_staged<R, VS, (R > 1)>(scol, p.rb - v0, first, nv, [&](int k, bool more, unsigned start, int n,
+                                                                   unsigned mask, int src) {
+            if (more && k < nblk) store_header<R, VS, MB>(h + (unsigned)(k * H), start, mask, t);
+            if constexpr (R > 1) {
+                const int to = at + group_excl_scan<R>(n, t);
+                at += group_sum<R>(n);
+                if (n > 0) scol[src] = kMovedBase + (unsigned)(to - src + kMovedZero);
+            }
         });
-        return;
-    }
-    if (nv == 0) return;
-    // the group's first 64 kPrefetch columns and values in one round trip
-    int c[kPrefetch];
-    W v[kPrefetch];
-    prefetch_words(col + v0, nv, lane, c);
-    prefetch_words(vin + v0, nv, lane, v);
-    stage_columns(col + v0, scol, nv, lane, c);
-    walk_group<R, VS, true, false>(g.rb, g.re, scol, v0, [&](int k, int start, int tt, int first, int n,
-                                                             unsigned mask, int src0) {
-        if (k >= nblk) return;
-        unsigned char* h = shdr + align + (bo + k) * H;
-        if (tt == 0) __builtin_memcpy(h, &start, 4);
-        __builtin_memcpy(h + 4 + tt * MB, &mask, MB);
-#pragma unroll
-        for (int j = 0; j < VS; ++j)
-            if (j < n) scol[src0 - v0 + j] = first - v0 + j;
-    });
-    wave_sync();
-    // headers: whole dwords of the destination as dword stores, the partial
-    // first and last dwords byte by byte (their other bytes are another
-    // group's)
-    {
-        const int64_t w0 = g0 >> 2, w1 = (g1 + 3) >> 2;  // destination dwords touched
-        unsigned* hw = reinterpret_cast<unsigned*>(hdr);
-        const unsigned* sw = reinterpret_cast<const unsigned*>(shdr);
-        for (int64_t w = w0 + lane; w < w1; w += 64) {
-            const int li = (int)(w - w0);
-            const int64_t bb = w * 4;  // first destination byte of this dword
-            if (bb >= g0 && bb + 4 <= g1) {
-                hw[w] = sw[li];
-            } else {
-                for (int q = 0; q < 4; ++q)
-                    if (bb + q >= g0 && bb + q < g1) hdr[bb + q] = shdr[li * 4 + q];
-            }
-        }
-    }
-    // values: the prefetched ones from registers, the rest read in CSR order
-    // (8 loads in flight per lane); each written to its block-order position
-#pragma unroll
-    for (int u = 0; u < kPrefetch; ++u) {
-        const int i = lane + 64 * u;
-        if (i < nv) vout[v0 + scol[i]] = v[u];
-    }
-    {
-        constexpr int U = 8;
-        for (int i0 = 64 * kPrefetch; i0 < nv; i0 += 64 * U) {
-            W w[U];
+        wave_sync();
+        int carry = 0;  // distance of the last part begun before the chunk
+        for (int i0 = 0; i0 < nv; i0 += 64 * U) {
+            if (i0 > 0) load(i0);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
+                if (i0 + 64 * u >= nv) break;
                 const int i = i0 + lane + 64 * u;
-                w[u] = i < nv ? vin[v0 + i] : W(0);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = i0 + lane + 64 * u;
-                if (i < nv) vout[v0 + scol[i]] = w[u];
+                int d = 0;
+                if constexpr (R > 1) {
+                    const unsigned e = i < nv ? scol[i] : 0u;
+                    const unsigned long long starts = ballot64(e >= kMovedBase);
+                    // the last part begun at or before this lane
+                    const unsigned long long upto = starts & ((2ull << lane) - 1ull);
+                    const int from = upto ? 63 - __builtin_clzll(upto) : 0;
+                    const int mine = __builtin_amdgcn_ds_bpermute(from << 2, (int)(e - kMovedBase)) - kMovedZero;
+                    d = upto ? mine : carry;
+                    carry = __builtin_amdgcn_readlane(d, 63);
+                }
+                if (i < nv) vout[v0 + i + d] = v[u];
             }
         }
+        wave_sync();
     }
 }
 
@@ -456,7 +518,7 @@ void launch_count(int64_t nrows, int64_t nbr, const int* rowptr, const int* col,
                   hipStream_t s) {
     const int64_t groups = (nbr + group_blockrows<R>() - 1) / group_blockrows<R>();
     const int sv = stage_values(nnz, groups);
-    const size_t shm = (size_t)(sv + kStagePad + row_start_words(sv)) * 4;
+    const size_t shm = (size_t)(sv + kStagePad) * 4;
     hipLaunchKernelGGL((k_convert_count<R, VS>), dim3((unsigned)groups), dim3(64), shm, s, nrows, nbr,
                        rowptr, col, out, err, sv);
 }
@@ -470,10 +532,9 @@ int launch_fill_r(int r, int64_t nrows, int64_t nbr, const int* rowptr, const in
     do {                                                                                                       \
         const int64_t groups = (nbr + group_blockrows<R>() - 1) / group_blockrows<R>();                        \
         const int sv = stage_values(nnz, groups);                                                              \
-        const int shb = stage_header_bytes(nblocks, 4 + R * MB, groups);                                       \
-        const size_t shm = (size_t)(sv + kStagePad) * 4 + (size_t)shb + 16;                                    \
+        const size_t shm = (size_t)(sv + kStagePad) * 4;                                                       \
         hipLaunchKernelGGL((k_convert_fill<W, R, VS, MB>), dim3((unsigned)groups), dim3(64), shm, s, nrows, nbr, \
-                           rowptr, col, vi, bptr, nblocks, hdr, vo, sv, shb);                                  \
+                           rowptr, col, vi, bptr, nblocks, hdr, vo, sv);                                       \
     } while (0)
     switch (r) {
     case 1: SPC5_FILL_LAUNCH(1); break;

@@ -282,7 +282,7 @@ __global__ void k_tile_scatter(const int* __restrict__ valptr, const int* __rest
 template <int R, int MB, int VS>
 void launch_blockrow_values(const spc5_hip_mat& m, int* cnt, int* err, hipStream_t s) {
     const unsigned g = (unsigned)((m.nbr + 255) / 256);  // 4 waves of 64 block-rows per workgroup
-    const unsigned every = g * 4 > 1024 ? g * 4 / 1024 : 1;  // about 1,000 sampled groups
+    const unsigned every = g * 4 > 64 ? g * 4 / 64 : 1;  // 64 .. 127 sampled groups (their sums are atomics)
     hipLaunchKernelGGL((k_blockrow_values<R, MB, VS>), dim3(g), dim3(256), 0, s, m.bptr, m.hdr, m.nbr, m.ncols, cnt,
                        err, m.value_type == SPC5_HIP_F64 ? 8 : 4, every);
 }
