@@ -215,6 +215,17 @@ int spc5_hip_convert_fill(int value_bytes, int vs, int mask_bytes, int r, int64_
                           const int* d_rowsSize, unsigned char* d_headers_out, void* d_values_out,
                           void* stream);
 
+/* The same two calls where the caller knows the sizes: nnz, the entries the
+ * column array holds (no row pointer may exceed it), and for the fill pass the
+ * block count the count pass returned.  They read neither back, so the count
+ * pass waits for the device once and the fill pass does not wait. */
+int spc5_hip_convert_count_sized(int vs, int r, int64_t nrows, int64_t nnz, const int* d_rowptr, const int* d_colidx,
+                                 int* d_rowsSize_out, int64_t* nblocks, void* stream);
+int spc5_hip_convert_fill_sized(int value_bytes, int vs, int mask_bytes, int r, int64_t nrows, int64_t nnz,
+                                int64_t nblocks, const int* d_rowptr, const int* d_colidx, const void* d_values_in,
+                                const int* d_rowsSize, unsigned char* d_headers_out, void* d_values_out,
+                                void* stream);
+
 /* The count pass without any allocation: same arguments, results and
  * errors as spc5_hip_convert_count.  No counterpart in the reference; it is
  * for callers that cannot allocate (serving loops, harnesses that forbid

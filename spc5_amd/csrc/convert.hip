@@ -22,16 +22,6 @@ namespace spc5 {
 
 namespace {
 
-// Checks a CSR row pointer: starts at 0, non-decreasing.
-__global__ void k_check_rowptr(const int* __restrict__ rowptr, int64_t nrows, int* err) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > nrows) return;
-    bool bad = false;
-    if (i == 0) bad = rowptr[0] != 0;
-    if (i < nrows) bad |= rowptr[i + 1] < rowptr[i];
-    if (bad) atomicOr(err, 1);
-}
-
 // Groups: one wave converts kGroupRows = 64 consecutive rows, one lane per
 // row; the r lanes of a block-row form a lane group.  The group's column
 // indices are staged in LDS with coalesced loads, the first entry of every row
@@ -368,22 +358,28 @@ __device__ __forceinline__ RowRun row_run(const GroupRows& g, int lo, int sv, in
     return p;
 }
 
-// Blocks per block-row (the count pass).  A violation of the column
-// precondition sets bit 0 of *err; the fill pass is then never run.  Dynamic
-// LDS: sv staged column indices and kStagePad words of pad.
+// Blocks per block-row (the count pass); cnt_out[nbr] = 0.  A row pointer that
+// does not start at 0, decreases or passes nnz sets err[0], a violation of the
+// column precondition err[1]; the fill pass is then never run, and a wave whose
+// row pointers fail reads no column.  Dynamic LDS: sv staged column indices and
+// kStagePad words of pad.
 template <int R, int VS>
 __global__ __launch_bounds__(64) void k_convert_count(int64_t nrows, int64_t nbr, const int* __restrict__ rowptr,
-                                                      const int* __restrict__ col, int* __restrict__ cnt_out,
-                                                      int* __restrict__ err, int sv) {
+                                                      const int* __restrict__ col, int64_t nnz,
+                                                      int* __restrict__ cnt_out, int* __restrict__ err, int sv) {
     constexpr int BR = group_blockrows<R>();
     extern __shared__ __align__(16) unsigned char smem[];
     unsigned* scol = reinterpret_cast<unsigned*>(smem);
     const int lane = threadIdx.x;
     const int64_t br0 = (int64_t)blockIdx.x * BR;
     const GroupRows g = group_rows(rowptr, br0 * R, nrows, lane);
+    if (br0 + BR >= nbr && lane == 0) cnt_out[nbr] = 0;
+    const bool broken = g.rb < 0 || g.re < g.rb || (int64_t)g.re > nnz || (br0 == 0 && lane == 0 && g.rb != 0);
+    const bool any_broken = ballot64(broken) != 0;
+    if (any_broken && lane == 0) atomicOr(err, 1);
     int nb = 0;
     bool bad = false;
-    for (int lo = 0; lo < kGroupRows;) {
+    for (int lo = any_broken ? kGroupRows : 0; lo < kGroupRows;) {
         const RowRun p = row_run<R>(g, lo, sv, lane);
         lo += p.rows;
         if (p.nv == 0) continue;
@@ -400,7 +396,7 @@ __global__ __launch_bounds__(64) void k_convert_count(int64_t nrows, int64_t nbr
     }
     const int64_t br = br0 + lane / R;
     if (lane % R == 0 && br < nbr) cnt_out[br] = nb;
-    if (bad) atomicOr(err, 1);
+    if (bad) atomicOr(err + 1, 1);
 }
 
 // Header of one block, the lanes of its block-row together: lane t = 0 writes
@@ -520,7 +516,7 @@ void launch_count(int64_t nrows, int64_t nbr, const int* rowptr, const int* col,
     const int sv = stage_values(nnz, groups);
     const size_t shm = (size_t)(sv + kStagePad) * 4;
     hipLaunchKernelGGL((k_convert_count<R, VS>), dim3((unsigned)groups), dim3(64), shm, s, nrows, nbr,
-                       rowptr, col, out, err, sv);
+                       rowptr, col, nnz, out, err, sv);
 }
 
 template <class W, int VS, int MB>
@@ -611,11 +607,11 @@ int read_words(const int* d_words, int* h, int n, hipStream_t s) {
     return SPC5_HIP_OK;
 }
 
-// Count pass shared by spc5_hip_convert_count and its no-allocation variant:
-// row pointer check, block count per block-row, exclusive scan into
-// d_rowsSize_out[0..nbr], total into *nblocks.  Allocates nothing itself.
-int convert_count_impl(int vs, int r, int64_t nrows, const int* d_rowptr, const int* d_colidx, int* d_rowsSize_out,
-                       int64_t* nblocks, const CountScratch& ws, hipStream_t s) {
+// Count pass of every entry point: block count per block-row, exclusive scan
+// into d_rowsSize_out[0..nbr], total into *nblocks.  nnz bounds the row
+// pointers and sizes the stage.  Allocates nothing and waits once.
+int convert_count_impl(int vs, int r, int64_t nrows, int64_t nnz, const int* d_rowptr, const int* d_colidx,
+                       int* d_rowsSize_out, int64_t* nblocks, const CountScratch& ws, hipStream_t s) {
     *nblocks = 0;
     const int64_t nbr = (nrows + r - 1) / r;
     if (scan_partials_needed(nbr + 1) > ws.partial_cap) {
@@ -623,40 +619,27 @@ int convert_count_impl(int vs, int r, int64_t nrows, const int* d_rowptr, const 
                   std::to_string(ws.partial_cap * 2048 - 1) + ")");
         return SPC5_HIP_ERR_INVALID;
     }
-    // flags and total start at zero: a fill kernel, not a memset node
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, ws.words, (int64_t)3, 0);
-    SPC5_HIP_TRY(hipGetLastError());
-    {
-        const unsigned g = (unsigned)((nrows + 1 + 255) / 256);
-        hipLaunchKernelGGL(k_check_rowptr, dim3(g), dim3(256), 0, s, d_rowptr, nrows, ws.words);
-        SPC5_HIP_TRY(hipGetLastError());
-    }
-    // the flag and the value count (which sizes the count pass's stage)
-    int bad_rowptr = 0, nnz = 0;
-    SPC5_HIP_TRY(hipMemcpyAsync(&bad_rowptr, ws.words, sizeof(int), hipMemcpyDeviceToHost, s));
-    SPC5_HIP_TRY(hipMemcpyAsync(&nnz, d_rowptr + nrows, sizeof(int), hipMemcpyDeviceToHost, s));
-    SPC5_HIP_TRY(hipStreamSynchronize(s));
-    // the count pass reads columns at the row pointers: only once they are valid
-    if (bad_rowptr) {
-        set_error("CSR row pointer must start at 0 and be non-decreasing");
-        return SPC5_HIP_ERR_INVALID;
-    }
     // A matrix without entries may come without a column array (an empty
     // tensor's storage); the count pass then reads no column.
     SPC5_CHECK_ARG(nbr == 0 || d_colidx != nullptr || nnz == 0, "colidx is null");
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, d_rowsSize_out + nbr, (int64_t)1, 0);
+    // flags and total start at zero: a fill kernel, not a memset node
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, ws.words, (int64_t)3, 0);
     SPC5_HIP_TRY(hipGetLastError());
+    if (nbr == 0) {
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, d_rowsSize_out, (int64_t)1, 0);
+        SPC5_HIP_TRY(hipGetLastError());
+    }
     if (nbr > 0) {
         const int key = r * 100 + vs;
         switch (key) {
-        case 108: launch_count<1, 8>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words + 1, nnz, s); break;
-        case 208: launch_count<2, 8>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words + 1, nnz, s); break;
-        case 408: launch_count<4, 8>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words + 1, nnz, s); break;
-        case 808: launch_count<8, 8>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words + 1, nnz, s); break;
-        case 116: launch_count<1, 16>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words + 1, nnz, s); break;
-        case 216: launch_count<2, 16>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words + 1, nnz, s); break;
-        case 416: launch_count<4, 16>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words + 1, nnz, s); break;
-        case 816: launch_count<8, 16>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words + 1, nnz, s); break;
+        case 108: launch_count<1, 8>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words, nnz, s); break;
+        case 208: launch_count<2, 8>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words, nnz, s); break;
+        case 408: launch_count<4, 8>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words, nnz, s); break;
+        case 808: launch_count<8, 8>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words, nnz, s); break;
+        case 116: launch_count<1, 16>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words, nnz, s); break;
+        case 216: launch_count<2, 16>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words, nnz, s); break;
+        case 416: launch_count<4, 16>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words, nnz, s); break;
+        case 816: launch_count<8, 16>(nrows, nbr, d_rowptr, d_colidx, d_rowsSize_out, ws.words, nnz, s); break;
         }
         SPC5_HIP_TRY(hipGetLastError());
     }
@@ -665,11 +648,29 @@ int convert_count_impl(int vs, int r, int64_t nrows, const int* d_rowptr, const 
     int h[3] = {0, 0, 0};
     rc = read_words(ws.words, h, 3, s);
     if (rc) return rc;
+    if (h[0]) {
+        set_error("CSR row pointer must start at 0 and be non-decreasing");
+        return SPC5_HIP_ERR_INVALID;
+    }
     if (h[1]) {
         set_error("CSR columns must be non-negative and strictly increasing inside each row");
         return SPC5_HIP_ERR_INVALID;
     }
     *nblocks = h[2];
+    return SPC5_HIP_OK;
+}
+
+// The entry count of a CSR matrix whose caller did not give it: its last row
+// pointer (waits).
+int read_nnz(int64_t nrows, const int* d_rowptr, int64_t* nnz, hipStream_t s) {
+    int n = 0;
+    const int rc = read_words(d_rowptr + nrows, &n, 1, s);
+    if (rc) return rc;
+    if (n < 0 || (nrows == 0 && n != 0)) {
+        set_error("CSR row pointer must start at 0 and be non-decreasing");
+        return SPC5_HIP_ERR_INVALID;
+    }
+    *nnz = n;
     return SPC5_HIP_OK;
 }
 
@@ -692,11 +693,12 @@ using namespace spc5;
 
 extern "C" {
 
-int spc5_hip_convert_count(int vs, int r, int64_t nrows, const int* d_rowptr, const int* d_colidx,
-                           int* d_rowsSize_out, int64_t* nblocks, void* stream) {
+int spc5_hip_convert_count_sized(int vs, int r, int64_t nrows, int64_t nnz, const int* d_rowptr, const int* d_colidx,
+                                 int* d_rowsSize_out, int64_t* nblocks, void* stream) {
     int rc = check_convert_count_args(vs, r, nrows, d_rowptr, d_rowsSize_out, nblocks);
     if (rc) return rc;
     *nblocks = 0;
+    SPC5_CHECK_ARG(nnz >= 0 && nnz <= INT32_MAX, "nnz out of range");
     hipStream_t s = as_stream(stream);
     const int64_t nbr = (nrows + r - 1) / r;
     CountScratch ws;
@@ -705,11 +707,21 @@ int spc5_hip_convert_count(int vs, int r, int64_t nrows, const int* d_rowptr, co
     SPC5_HIP_TRY(buf.alloc(sizeof(int) * (size_t)(kScratchWords + ws.partial_cap)));
     ws.words = buf.as<int>();
     ws.partials = ws.words + kScratchWords;
-    rc = convert_count_impl(vs, r, nrows, d_rowptr, d_colidx, d_rowsSize_out, nblocks, ws, s);
+    rc = convert_count_impl(vs, r, nrows, nnz, d_rowptr, d_colidx, d_rowsSize_out, nblocks, ws, s);
     // the buffer is freed on return: every launch that uses it has ended
-    // (each path out of the pass ends with a stream synchronisation)
-    SPC5_HIP_TRY(hipStreamSynchronize(s));
+    if (rc) SPC5_HIP_TRY(hipStreamSynchronize(s));
     return rc;
+}
+
+int spc5_hip_convert_count(int vs, int r, int64_t nrows, const int* d_rowptr, const int* d_colidx,
+                           int* d_rowsSize_out, int64_t* nblocks, void* stream) {
+    int rc = check_convert_count_args(vs, r, nrows, d_rowptr, d_rowsSize_out, nblocks);
+    if (rc) return rc;
+    *nblocks = 0;
+    int64_t nnz = 0;
+    rc = read_nnz(nrows, d_rowptr, &nnz, as_stream(stream));
+    if (rc) return rc;
+    return spc5_hip_convert_count_sized(vs, r, nrows, nnz, d_rowptr, d_colidx, d_rowsSize_out, nblocks, stream);
 }
 
 int spc5_hip_convert_count_noalloc(int vs, int r, int64_t nrows, const int* d_rowptr, const int* d_colidx,
@@ -722,7 +734,40 @@ int spc5_hip_convert_count_noalloc(int vs, int r, int64_t nrows, const int* d_ro
     if (rc) return rc;
     ws.partials = ws.words + kScratchWords;
     ws.partial_cap = kScratchInts - kScratchWords;
-    return convert_count_impl(vs, r, nrows, d_rowptr, d_colidx, d_rowsSize_out, nblocks, ws, as_stream(stream));
+    hipStream_t s = as_stream(stream);
+    const int64_t nbr = (nrows + r - 1) / r;
+    if (scan_partials_needed(nbr + 1) > ws.partial_cap)  // refused before any device work
+        return convert_count_impl(vs, r, nrows, 0, d_rowptr, d_colidx, d_rowsSize_out, nblocks, ws, s);
+    int64_t nnz = 0;
+    rc = read_nnz(nrows, d_rowptr, &nnz, s);
+    if (rc) return rc;
+    return convert_count_impl(vs, r, nrows, nnz, d_rowptr, d_colidx, d_rowsSize_out, nblocks, ws, s);
+}
+
+int spc5_hip_convert_fill_sized(int value_bytes, int vs, int mask_bytes, int r, int64_t nrows, int64_t nnz,
+                                int64_t nblocks, const int* d_rowptr, const int* d_colidx, const void* d_values_in,
+                                const int* d_rowsSize, unsigned char* d_headers_out, void* d_values_out,
+                                void* stream) {
+    SPC5_CHECK_ARG(value_bytes == 8 || value_bytes == 4 || value_bytes == 2, "value_bytes must be 8, 4 or 2");
+    SPC5_CHECK_ARG(nrows >= 0 && nrows <= INT32_MAX, "nrows out of range");
+    SPC5_CHECK_ARG(nnz >= 0 && nnz <= INT32_MAX && nblocks >= 0 && nblocks <= INT32_MAX, "sizes out of range");
+    SPC5_CHECK_ARG(d_rowptr != nullptr && d_rowsSize != nullptr, "null pointer");
+    hipStream_t s = as_stream(stream);
+    const int64_t nbr = (nrows + r - 1) / r;
+    if (nbr == 0 || nblocks == 0) return SPC5_HIP_OK;
+    SPC5_CHECK_ARG(d_headers_out != nullptr && d_values_out != nullptr && d_values_in != nullptr,
+                   "null output/value pointer");
+    switch (value_bytes) {
+    case 8:
+        return launch_fill_w<unsigned long long>(vs, mask_bytes, r, nrows, nbr, d_rowptr, d_colidx, d_values_in,
+                                                 d_rowsSize, nblocks, nnz, d_headers_out, d_values_out, s);
+    case 4:
+        return launch_fill_w<unsigned int>(vs, mask_bytes, r, nrows, nbr, d_rowptr, d_colidx, d_values_in,
+                                           d_rowsSize, nblocks, nnz, d_headers_out, d_values_out, s);
+    default:
+        return launch_fill_w<unsigned short>(vs, mask_bytes, r, nrows, nbr, d_rowptr, d_colidx, d_values_in,
+                                             d_rowsSize, nblocks, nnz, d_headers_out, d_values_out, s);
+    }
 }
 
 int spc5_hip_convert_fill(int value_bytes, int vs, int mask_bytes, int r, int64_t nrows, const int* d_rowptr,
@@ -738,20 +783,8 @@ int spc5_hip_convert_fill(int value_bytes, int vs, int mask_bytes, int r, int64_
     SPC5_HIP_TRY(hipMemcpyAsync(&nb, d_rowsSize + nbr, sizeof(int), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipMemcpyAsync(&nnz, d_rowptr + nrows, sizeof(int), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipStreamSynchronize(s));
-    if (nb == 0) return SPC5_HIP_OK;
-    SPC5_CHECK_ARG(d_headers_out != nullptr && d_values_out != nullptr && d_values_in != nullptr,
-                   "null output/value pointer");
-    switch (value_bytes) {
-    case 8:
-        return launch_fill_w<unsigned long long>(vs, mask_bytes, r, nrows, nbr, d_rowptr, d_colidx, d_values_in,
-                                                 d_rowsSize, nb, nnz, d_headers_out, d_values_out, s);
-    case 4:
-        return launch_fill_w<unsigned int>(vs, mask_bytes, r, nrows, nbr, d_rowptr, d_colidx, d_values_in,
-                                           d_rowsSize, nb, nnz, d_headers_out, d_values_out, s);
-    default:
-        return launch_fill_w<unsigned short>(vs, mask_bytes, r, nrows, nbr, d_rowptr, d_colidx, d_values_in,
-                                             d_rowsSize, nb, nnz, d_headers_out, d_values_out, s);
-    }
+    return spc5_hip_convert_fill_sized(value_bytes, vs, mask_bytes, r, nrows, nnz, nb, d_rowptr, d_colidx, d_values_in,
+                                       d_rowsSize, d_headers_out, d_values_out, stream);
 }
 
 }  // extern "C"

@@ -161,27 +161,18 @@ __global__ __launch_bounds__(kWavesPerGroup * 64) void k_access_probe(
 
 // ---- plan kernels --------------------------------------------------------
 
-// Checks the block-row pointers: 0-based, non-decreasing, ending at nblocks.
-__global__ void k_check_bptr(const int* __restrict__ bptr, int64_t nbr, int64_t nblocks, int* err) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > nbr) return;
-    const int v = bptr[i];
-    bool bad = v < 0 || (int64_t)v > nblocks;
-    if (i == 0) bad |= v != 0;
-    if (i == nbr) bad |= (int64_t)v != nblocks;
-    if (i < nbr) bad |= bptr[i + 1] < v;
-    if (bad) atomicOr(err, 1);
-}
-
-// Values per block-row (popcount of every mask) and a column range check.
-// One wave per 64 block-rows (the pointers already checked): the lanes read
+// Values per block-row (popcount of every mask), with a check of the block-row
+// pointers (0-based, non-decreasing, ending at nblocks: err bit 0; a wave whose
+// pointers fail reads no header) and of the columns (bit 1).
+// One wave per 64 block-rows: the lanes read
 // the group's headers in block order, coalesced, find each block's block-row
 // by a binary search of the 65 group pointers in LDS and add its popcount to
 // that block-row's LDS counter.
 template <int R, int MB, int VS>
 __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__ bptr,
                                                          const unsigned char* __restrict__ hdr, int64_t nbr,
-                                                         int64_t ncols, int* __restrict__ cnt_out, int* err,
+                                                         int64_t nblocks, int64_t ncols, int* __restrict__ cnt_out,
+                                                         int* err,
                                                          int xbytes, unsigned every) {
     constexpr int H = 4 + R * MB;
     using MW = MaskWords<R * MB>;
@@ -191,6 +182,7 @@ __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int64_t br0 = ((int64_t)blockIdx.x * 4 + w) * 64;
     if (br0 >= nbr) return;  // whole wave: nothing below synchronises across waves
+    if (br0 + 64 >= nbr && lane == 0) cnt_out[nbr] = 0;  // the scan's last entry
     int* sp = sptr[w];
     int* sc = scnt[w];
     {
@@ -201,6 +193,16 @@ __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__
         sline[w][lane] = 0u;
     }
     wave_sync();
+    {
+        const int lo = sp[lane], hi = sp[lane + 1];
+        bool broken = lo < 0 || hi < lo || (int64_t)hi > nblocks;
+        if (lane == 0) broken |= (br0 == 0 && lo != 0) || (br0 + 64 >= nbr && (int64_t)sp[64] != nblocks);
+        if (ballot64(broken)) {
+            if (br0 + lane < nbr) cnt_out[br0 + lane] = 0;
+            if (lane == 0) atomicOr(err, 1);
+            return;
+        }
+    }
     const int b0 = sp[0], bE = sp[64];
     // One group in `every` also counts the distinct 128-byte lines of x that
     // its first 64 blocks start in (a hash into 2,048 bits): err[1] sums the
@@ -248,34 +250,60 @@ __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__
     }
 }
 
-// Tiles never cross a multiple of maxbr block-rows; each such run of
-// block-rows is cut into ceil(values / target) pieces of about equal values.
-__device__ __forceinline__ bool tile_starts(const int* valptr, int64_t br, int64_t nbr, int target, int maxbr) {
-    const int64_t first = br / maxbr * maxbr;
-    if (br == first) return true;
-    const int64_t v0 = valptr[first], all = valptr[first + maxbr < nbr ? first + maxbr : nbr] - v0;
-    if (all <= target) return false;
-    const int64_t pieces = (all + target - 1) / target;
-    return (valptr[br] - v0) * pieces / all != (valptr[br - 1] - v0) * pieces / all;
+// Tiles never cross a multiple of maxbr <= 64 block-rows (a chunk); a chunk is
+// cut into ceil(values / target) pieces of about equal values.  One wave per
+// chunk, one block-row per lane; returns the lanes whose block-row starts a
+// tile.
+__device__ __forceinline__ unsigned long long chunk_tiles(const int* __restrict__ valptr, int64_t chunk, int64_t nbr,
+                                                          int target, int maxbr, int lane, int& v) {
+    const int64_t first = chunk * maxbr;
+    const int n = (int)(nbr - first < maxbr ? nbr - first : maxbr);
+    v = valptr[first + (lane < n ? lane : n)];
+    const int v0 = __builtin_amdgcn_readfirstlane(v), all = valptr[first + n] - v0;
+    int64_t piece = 0;
+    if (all > target) piece = (int64_t)(v - v0) * ((all + (int64_t)target - 1) / target) / all;
+    const int at = (int)piece;  // at most the chunk's values / target
+    const int before = wave_prev_lane(at, -1);
+    return ballot64(lane < n && at != before);
 }
 
-__global__ void k_tile_flags(const int* __restrict__ valptr, int64_t nbr, int target, int maxbr,
-                             int* __restrict__ flags) {
-    const int64_t br = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (br >= nbr) return;
-    flags[br] = tile_starts(valptr, br, nbr, target, maxbr) ? 1 : 0;
-}
+constexpr int kChunkWaves = 4;
 
-__global__ void k_tile_scatter(const int* __restrict__ valptr, const int* __restrict__ bptr, int64_t nbr, int target,
-                               int maxbr, const int* __restrict__ idx, int64_t ntiles, int4* __restrict__ tiles) {
-    const int64_t br = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (br > nbr) return;
-    if (br == nbr) {
-        tiles[ntiles] = make_int4((int)nbr, bptr[nbr], valptr[nbr], 0);
+// WRITE false: tiles per chunk to `at` (at[nchunks] = 0).  WRITE true: `at` is
+// the scanned count; the tiles' records are written, and the results the host
+// reads are gathered: out[0..2] = err, out[3] = values, out[4] = tiles.
+template <bool WRITE>
+__global__ __launch_bounds__(64 * kChunkWaves) void k_tiles(const int* __restrict__ valptr,
+                                                           const int* __restrict__ bptr, int64_t nbr, int target,
+                                                           int maxbr, int64_t nchunks, int* __restrict__ at,
+                                                           int4* __restrict__ tiles, int64_t room,
+                                                           const int* __restrict__ err, int* __restrict__ out) {
+    const int lane = threadIdx.x & 63;
+    const int64_t c = (int64_t)blockIdx.x * kChunkWaves + (threadIdx.x >> 6);
+    if (c > nchunks) return;
+    if (c == nchunks) {
+        if (lane != 0) return;
+        if constexpr (WRITE) {
+            const int n = at[nchunks], nv = valptr[nbr];
+            if (n >= 0 && n < room) tiles[n] = make_int4((int)nbr, bptr[nbr], nv, 0);
+            out[0] = err ? err[0] : 0;
+            out[1] = err ? err[1] : 0;
+            out[2] = err ? err[2] : 0;
+            out[3] = nv;
+            out[4] = n;
+        } else {
+            at[nchunks] = 0;
+        }
         return;
     }
-    if (tile_starts(valptr, br, nbr, target, maxbr)) {
-        tiles[idx[br]] = make_int4((int)br, bptr[br], valptr[br], 0);
+    int v;
+    const unsigned long long starts = chunk_tiles(valptr, c, nbr, target, maxbr, lane, v);
+    if constexpr (WRITE) {
+        const int64_t br = c * maxbr + lane;
+        const int to = at[c] + lanes_below(starts);
+        if (((starts >> lane) & 1ull) && to < room) tiles[to] = make_int4((int)br, bptr[br], v, 0);
+    } else {
+        if (lane == 0) at[c] = __popcll(starts);
     }
 }
 
@@ -283,8 +311,8 @@ template <int R, int MB, int VS>
 void launch_blockrow_values(const spc5_hip_mat& m, int* cnt, int* err, hipStream_t s) {
     const unsigned g = (unsigned)((m.nbr + 255) / 256);  // 4 waves of 64 block-rows per workgroup
     const unsigned every = g * 4 > 64 ? g * 4 / 64 : 1;  // 64 .. 127 sampled groups (their sums are atomics)
-    hipLaunchKernelGGL((k_blockrow_values<R, MB, VS>), dim3(g), dim3(256), 0, s, m.bptr, m.hdr, m.nbr, m.ncols, cnt,
-                       err, m.value_type == SPC5_HIP_F64 ? 8 : 4, every);
+    hipLaunchKernelGGL((k_blockrow_values<R, MB, VS>), dim3(g), dim3(256), 0, s, m.bptr, m.hdr, m.nbr, m.nblocks, m.ncols,
+                       cnt, err, m.value_type == SPC5_HIP_F64 ? 8 : 4, every);
 }
 
 template <class V, class X, class ACC, int R, int VS, int MB, bool SORT>
@@ -378,63 +406,105 @@ int launch_spmv_f64vec(const spc5_hip_mat& m, const double* x, double* y, hipStr
     return SPC5_HIP_ERR_INVALID;
 }
 
+namespace {
+
+// Scratch of one plan: what the host reads back, the counters of
+// k_blockrow_values, scan partials and the tile count of every chunk.
+struct PlanScratch {
+    DeviceBuffer buf;
+    int* out = nullptr;       // int[8]: see k_tiles
+    int* err = nullptr;       // int[8]: flags, sampled lines, sampled blocks
+    int* partials = nullptr;
+    int* chunks = nullptr;    // int[nchunks + 1]
+    int64_t nchunks = 0;
+    int maxbr = 1;
+    hipError_t alloc(const spc5_hip_mat& m, int maxrows) {
+        maxbr = maxrows / m.r > 0 ? maxrows / m.r : 1;
+        if (maxbr > 64) maxbr = 64;
+        nchunks = (m.nbr + maxbr - 1) / maxbr;
+        const int64_t np = scan_partials_needed(m.nbr + 1);
+        const hipError_t e = buf.alloc(sizeof(int) * (size_t)(16 + np + nchunks + 1));
+        out = buf.as<int>();
+        err = out + 8;
+        partials = err + 8;
+        chunks = partials + np;
+        return e;
+    }
+};
+
+// Enqueues the tile list of p.valptr (room for every tile is known beforehand:
+// a chunk has at most one piece more than its values / target).
+int enqueue_tiles(const spc5_hip_mat& m, Plan& p, int target, const PlanScratch& w, const int* err, hipStream_t s) {
+    p.target = target;
+    const int* valptr = p.valptr->as<int>();
+    p.tiles = std::make_shared<DeviceBuffer>();
+    const int64_t room = m.nnz / target + w.nchunks + 1;
+    SPC5_HIP_TRY(p.tiles->alloc(sizeof(int4) * (size_t)room));
+    const unsigned g = (unsigned)((w.nchunks + 1 + kChunkWaves - 1) / kChunkWaves);
+    hipLaunchKernelGGL(k_tiles<false>, dim3(g), dim3(64 * kChunkWaves), 0, s, valptr, m.bptr, m.nbr, target, w.maxbr,
+                       w.nchunks, w.chunks, nullptr, (int64_t)0, nullptr, nullptr);
+    SPC5_HIP_TRY(hipGetLastError());
+    const int rc = scan_exclusive_i32_ws(w.chunks, w.nchunks + 1, nullptr, w.partials, s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_tiles<true>, dim3(g), dim3(64 * kChunkWaves), 0, s, valptr, m.bptr, m.nbr, target, w.maxbr,
+                       w.nchunks, w.chunks, p.tiles->as<int4>(), room, err, w.out);
+    SPC5_HIP_TRY(hipGetLastError());
+    return SPC5_HIP_OK;
+}
+
+}  // namespace
+
+// Everything is enqueued at once and the host waits once, for the results (a
+// wait and a read-back cost about 30 us; checking the pointers first, counting
+// values, counting tiles and allocating for them took four).  Until then the
+// kernels only keep inside their buffers: waves with bad pointers read no
+// header, and no tile is written past the room for the handle's nnz.
 int build_plan(spc5_hip_mat& m, hipStream_t s) {
     Plan& p = m.plan;
     p.ntiles = 0;
     if (m.nbr == 0) return SPC5_HIP_OK;
-    DeviceBuffer err;
-    SPC5_HIP_TRY(err.alloc(3 * sizeof(int)));  // flags, sampled lines, sampled blocks
-    SPC5_HIP_TRY(hipMemsetAsync(err.p, 0, 3 * sizeof(int), s));
-    {
-        const unsigned g = (unsigned)((m.nbr + 1 + 255) / 256);
-        hipLaunchKernelGGL(k_check_bptr, dim3(g), dim3(256), 0, s, m.bptr, m.nbr, m.nblocks, err.as<int>());
-        SPC5_HIP_TRY(hipGetLastError());
-        int herr = 0;
-        SPC5_HIP_TRY(hipMemcpyAsync(&herr, err.p, sizeof(int), hipMemcpyDeviceToHost, s));
-        SPC5_HIP_TRY(hipStreamSynchronize(s));
-        if (herr) {
-            set_error("rowsSize is not a 0-based non-decreasing block pointer array ending at nblocks");
-            return SPC5_HIP_ERR_INVALID;
-        }
-    }
+    PlanScratch w;
+    SPC5_HIP_TRY(w.alloc(m, tile_rows(m.r)));
+    SPC5_HIP_TRY(hipMemsetAsync(w.err, 0, 8 * sizeof(int), s));
     p.valptr = std::make_shared<DeviceBuffer>();
     SPC5_HIP_TRY(p.valptr->alloc(sizeof(int) * (size_t)(m.nbr + 1)));
     int* valptr = p.valptr->as<int>();
-    SPC5_HIP_TRY(hipMemsetAsync(valptr + m.nbr, 0, sizeof(int), s));
     const int key = m.r * 100 + m.mb * 10 + (m.vs == 16 ? 1 : 0);
     switch (key) {
-    case 110: launch_blockrow_values<1, 1, 8>(m, valptr, err.as<int>(), s); break;
-    case 210: launch_blockrow_values<2, 1, 8>(m, valptr, err.as<int>(), s); break;
-    case 410: launch_blockrow_values<4, 1, 8>(m, valptr, err.as<int>(), s); break;
-    case 810: launch_blockrow_values<8, 1, 8>(m, valptr, err.as<int>(), s); break;
-    case 121: launch_blockrow_values<1, 2, 16>(m, valptr, err.as<int>(), s); break;
-    case 221: launch_blockrow_values<2, 2, 16>(m, valptr, err.as<int>(), s); break;
-    case 421: launch_blockrow_values<4, 2, 16>(m, valptr, err.as<int>(), s); break;
-    case 821: launch_blockrow_values<8, 2, 16>(m, valptr, err.as<int>(), s); break;
+    case 110: launch_blockrow_values<1, 1, 8>(m, valptr, w.err, s); break;
+    case 210: launch_blockrow_values<2, 1, 8>(m, valptr, w.err, s); break;
+    case 410: launch_blockrow_values<4, 1, 8>(m, valptr, w.err, s); break;
+    case 810: launch_blockrow_values<8, 1, 8>(m, valptr, w.err, s); break;
+    case 121: launch_blockrow_values<1, 2, 16>(m, valptr, w.err, s); break;
+    case 221: launch_blockrow_values<2, 2, 16>(m, valptr, w.err, s); break;
+    case 421: launch_blockrow_values<4, 2, 16>(m, valptr, w.err, s); break;
+    case 821: launch_blockrow_values<8, 2, 16>(m, valptr, w.err, s); break;
     default: set_error("unsupported (r, VS, mask bytes)"); return SPC5_HIP_ERR_INVALID;
     }
     SPC5_HIP_TRY(hipGetLastError());
-    DeviceBuffer dtotal;
-    SPC5_HIP_TRY(dtotal.alloc(sizeof(int)));
-    // Counts are < 2^31 each; the scan is checked against nnz below.
-    int rc = scan_exclusive_i32(valptr, m.nbr + 1, dtotal.as<int>(), s);
+    int rc = scan_exclusive_i32_ws(valptr, m.nbr + 1, nullptr, w.partials, s);
     if (rc) return rc;
-    int hstat[3] = {0, 0, 0}, hnnz = 0;
-    const int& herr = hstat[0];
-    SPC5_HIP_TRY(hipMemcpyAsync(hstat, err.p, 3 * sizeof(int), hipMemcpyDeviceToHost, s));
-    SPC5_HIP_TRY(hipMemcpyAsync(&hnnz, valptr + m.nbr, sizeof(int), hipMemcpyDeviceToHost, s));
+    rc = enqueue_tiles(m, p, default_tile_values(m.nnz), w, w.err, s);
+    if (rc) return rc;
+    int h[5];
+    SPC5_HIP_TRY(hipMemcpyAsync(h, w.out, sizeof(h), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipStreamSynchronize(s));
-    if (herr) {
+    if (h[0] & 1) {
+        set_error("rowsSize is not a 0-based non-decreasing block pointer array ending at nblocks");
+        return SPC5_HIP_ERR_INVALID;
+    }
+    if (h[0]) {
         set_error("a block touches a column outside [0, ncols)");
         return SPC5_HIP_ERR_INVALID;
     }
-    if ((int64_t)hnnz != m.nnz) {
-        set_error("nnz (" + std::to_string(m.nnz) + ") differs from the mask popcount (" + std::to_string(hnnz) + ")");
+    if ((int64_t)h[3] != m.nnz) {
+        set_error("nnz (" + std::to_string(m.nnz) + ") differs from the mask popcount (" + std::to_string(h[3]) + ")");
         return SPC5_HIP_ERR_INVALID;
     }
-    m.scatter = hstat[2] > 0 ? (double)hstat[1] / hstat[2] : 0.0;
+    p.ntiles = h[4];
+    m.scatter = h[2] > 0 ? (double)h[1] / h[2] : 0.0;
     m.lane_body = lane_block_wins(m);
-    return build_tiles(m, p, tile_rows(m.r), default_tile_values(m.nnz), s);
+    return SPC5_HIP_OK;
 }
 
 // Which tile a product runs: lane-block (one block per lane, spmv_lane.hpp)
@@ -489,28 +559,14 @@ int build_tiles(const spc5_hip_mat& m, Plan& p, int maxrows, int target, hipStre
     p.target = target;
     if (m.nbr == 0) return SPC5_HIP_OK;
     if (!p.valptr) p.valptr = m.plan.valptr;
-    const int* valptr = p.valptr->as<int>();
-    const int maxbr = maxrows / m.r > 0 ? maxrows / m.r : 1;
-    int rc;
-    DeviceBuffer dtotal;
-    SPC5_HIP_TRY(dtotal.alloc(sizeof(int)));
-    DeviceBuffer flags;
-    SPC5_HIP_TRY(flags.alloc(sizeof(int) * (size_t)(m.nbr + 1)));
-    const unsigned g = (unsigned)((m.nbr + 1 + 255) / 256);
-    hipLaunchKernelGGL(k_tile_flags, dim3(g), dim3(256), 0, s, valptr, m.nbr, p.target, maxbr, flags.as<int>());
-    SPC5_HIP_TRY(hipGetLastError());
-    rc = scan_exclusive_i32(flags.as<int>(), m.nbr, dtotal.as<int>(), s);
+    PlanScratch w;
+    SPC5_HIP_TRY(w.alloc(m, maxrows));
+    const int rc = enqueue_tiles(m, p, target, w, nullptr, s);
     if (rc) return rc;
-    int hn = 0;
-    SPC5_HIP_TRY(hipMemcpyAsync(&hn, dtotal.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    int n = 0;
+    SPC5_HIP_TRY(hipMemcpyAsync(&n, w.out + 4, sizeof(int), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipStreamSynchronize(s));
-    p.ntiles = hn;
-    p.tiles = std::make_shared<DeviceBuffer>();
-    SPC5_HIP_TRY(p.tiles->alloc(sizeof(int4) * (size_t)(hn + 1)));
-    hipLaunchKernelGGL(k_tile_scatter, dim3(g), dim3(256), 0, s, valptr, m.bptr, m.nbr, p.target, maxbr,
-                       flags.as<int>(), (int64_t)hn, p.tiles->as<int4>());
-    SPC5_HIP_TRY(hipGetLastError());
-    SPC5_HIP_TRY(hipStreamSynchronize(s));
+    p.ntiles = n;
     return SPC5_HIP_OK;
 }
 

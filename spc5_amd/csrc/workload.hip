@@ -98,7 +98,9 @@ int spc5_hip_synth_banded_count(int64_t n, int64_t bw, uint64_t thr, uint64_t se
     SPC5_HIP_TRY(hipGetLastError());
     DeviceBuffer total;
     SPC5_HIP_TRY(total.alloc(sizeof(int)));
-    const int rc = scan_exclusive_i32(d_rowptr, n + 1, total.as<int>(), s);
+    DeviceBuffer partials;
+    SPC5_HIP_TRY(partials.alloc(sizeof(int) * (size_t)scan_partials_needed(n + 1)));
+    const int rc = scan_exclusive_i32_ws(d_rowptr, n + 1, total.as<int>(), partials.as<int>(), s);
     if (rc) return rc;
     int h = 0;
     SPC5_HIP_TRY(hipMemcpyAsync(&h, total.p, sizeof(int), hipMemcpyDeviceToHost, s));

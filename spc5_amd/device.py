@@ -48,6 +48,11 @@ def _need_cuda(t, name, dtype=None):
         raise Spc5Error(f"{name} must be contiguous")
 
 
+def _entries(col) -> int:
+    """Entries of a CSR column array, as far as 32-bit row pointers reach."""
+    return min(col.numel(), 2 ** 31 - 1)
+
+
 def convert_csr(rowptr, col, values, r: int, vs: int | None = None, stream=None):
     """GPU converter: CSR device tensors -> (rows_size[ceil(N/r)+1], headers, values).
 
@@ -62,14 +67,14 @@ def convert_csr(rowptr, col, values, r: int, vs: int | None = None, stream=None)
     rows_size = torch.empty(nbr + 1, dtype=torch.int32, device=dev)
     nb = C.c_int64(0)
     s = stream_ptr(stream)
-    check(lib().spc5_hip_convert_count(vs, r, n, _ptr(rowptr), _ptr(col), _ptr(rows_size), C.byref(nb), s),
-          "spc5_hip_convert_count")
+    check(lib().spc5_hip_convert_count_sized(vs, r, n, _entries(col), _ptr(rowptr), _ptr(col), _ptr(rows_size),
+                                             C.byref(nb), s), "spc5_hip_convert_count")
     nblocks = nb.value
     hdr = torch.empty(nblocks * (4 + r * mask_bytes(vs)), dtype=torch.uint8, device=dev)
     vout = torch.empty_like(values)
-    check(lib().spc5_hip_convert_fill(values.element_size(), vs, mask_bytes(vs), r, n, _ptr(rowptr), _ptr(col),
-                                      _ptr(values), _ptr(rows_size), _ptr(hdr), _ptr(vout), s),
-          "spc5_hip_convert_fill")
+    check(lib().spc5_hip_convert_fill_sized(values.element_size(), vs, mask_bytes(vs), r, n, _entries(col), nblocks,
+                                            _ptr(rowptr), _ptr(col), _ptr(values), _ptr(rows_size), _ptr(hdr),
+                                            _ptr(vout), s), "spc5_hip_convert_fill")
     return rows_size, hdr, vout, nblocks
 
 
@@ -80,8 +85,8 @@ def block_count(rowptr, col, r: int, vs: int = 8, stream=None) -> int:
     n = rowptr.numel() - 1
     tmp = torch.empty((n + r - 1) // r + 1, dtype=torch.int32, device=rowptr.device)
     nb = C.c_int64(0)
-    check(lib().spc5_hip_convert_count(vs, r, n, _ptr(rowptr), _ptr(col), _ptr(tmp), C.byref(nb),
-                                       stream_ptr(stream)), "spc5_hip_convert_count")
+    check(lib().spc5_hip_convert_count_sized(vs, r, n, _entries(col), _ptr(rowptr), _ptr(col), _ptr(tmp), C.byref(nb),
+                                             stream_ptr(stream)), "spc5_hip_convert_count")
     return nb.value
 
 
