@@ -186,6 +186,13 @@ int spc5_hip_spmv(spc5_hip_mat_t h, const void* d_x, void* d_y, void* stream);
 int spc5_hip_coo_to_csr(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, int sorted, const int* d_i,
                         const int* d_j, const void* d_v, int* d_rowptr, int* d_col, void* d_val, void* stream);
 
+/* The same in a workspace the caller provides (256-byte aligned, at least
+ * spc5_hip_coo_workspace_bytes; NULL: allocated for the call). */
+int64_t spc5_hip_coo_workspace_bytes(int64_t nrows, int64_t nnz, int sorted);
+int spc5_hip_coo_to_csr_ws(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, int sorted, const int* d_i,
+                           const int* d_j, const void* d_v, int* d_rowptr, int* d_col, void* d_val, void* d_workspace,
+                           int64_t workspace_bytes, void* stream);
+
 /* MatrixMarket coordinate files (real, integer or pattern; general,
  * symmetric or skew-symmetric), read as examples/load_mm_and_compare.cpp
  * loadMM (287-428) reads them: 0-based indices, pattern values 1, the

@@ -2,10 +2,11 @@
 //
 // spc5_hip_coo_to_csr does what the reference's COO_unsorted_to_CSR /
 // COO_sorted_to_CSR do (src/spc5.hpp:77-114) with the GPU: entries are
-// ordered by (row, column) with a stable radix sort of 64-bit keys
-// (row << 32 | column; hipCUB), the row pointers come from a binary search
-// of every row's first key in the sorted keys, and columns and values are
-// gathered through the sort's permutation.  Duplicate (row, column) entries
+// ordered by (row, column), stably.  Short rows are counted, filled and ranked
+// (see "rows of few entries"); otherwise a radix sort of 64-bit keys
+// (row << 32 | column; hipCUB) orders them, the row pointers come from a binary
+// search of every row's first key in the sorted keys, and columns and values
+// are gathered through the sort's permutation.  Duplicate (row, column) entries
 // are kept, in input order, as the reference keeps them.  With `sorted` set
 // the sort is skipped and the order is checked instead (the reference
 // trusts it).  Every index is range-checked.
@@ -72,10 +73,149 @@ __global__ void k_coo_gather(const unsigned long long* __restrict__ keys, const 
     val[t] = v[perm ? perm[t] : t];
 }
 
+// ---- rows of few entries -----------------------------------------------------
+//
+// Most matrices have short rows, and ordering (row, column) keys of 64 bits
+// with a radix sort reads and writes every entry once per 8 key bits.  Here the
+// rows are the buckets: entries count themselves into their row (the count a
+// counter returns is the entry's place in it), the scanned counts are the row
+// pointers, every entry writes (column, input position) to its place, and then
+// finds its rank among its row's keys by comparing with each of them, which
+// gives the stable order whatever order the counters were reached in.  Three
+// passes over the entries and one comparison per pair of entries of a row: the
+// pairs bound it, so rows of more than kShortRow entries go to the radix sort
+// (coo_short_rows decides on the mean; a longer row found on the way sends the
+// whole matrix there).  1.25 M entries in 50 K rows: 462 us with the radix
+// sort, 199 us; 3.2 M in 100 K rows 1,467 and 385 us.
+constexpr int kShortRow = 1024;
+
+// Counts per row (rowptr, cleared before) and every entry's place in its row.
+__global__ __launch_bounds__(256) void k_coo_count(const int* __restrict__ ri, const int* __restrict__ cj, int64_t nnz,
+                                                   int64_t nrows, int64_t ncols, int* __restrict__ count,
+                                                   int* __restrict__ place, int* __restrict__ err) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nnz) return;
+    const int r = ri[t], c = cj[t];
+    if (r < 0 || (int64_t)r >= nrows || c < 0 || (int64_t)c >= ncols) {
+        atomicOr(err, 1);
+        place[t] = -1;
+        return;
+    }
+    place[t] = atomicAdd(&count[r], 1);
+}
+
+// keys[row pointer + place] = (column, input position).
+__global__ __launch_bounds__(256) void k_coo_place(const int* __restrict__ ri, const int* __restrict__ cj, int64_t nnz,
+                                                   const int* __restrict__ rowptr, const int* __restrict__ place,
+                                                   unsigned long long* __restrict__ keys, int* __restrict__ err) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nnz) return;
+    const int p = place[t];
+    if (p < 0) return;
+    if (p >= kShortRow) atomicOr(err, 4);
+    keys[(int64_t)rowptr[ri[t]] + p] = ((unsigned long long)(unsigned)cj[t] << 32) | (unsigned)t;
+}
+
+// Every entry to its rank in its row.  Does nothing after an error or a long row.
+template <class T>
+__global__ __launch_bounds__(256) void k_coo_rank(const int* __restrict__ ri, int64_t nnz,
+                                                  const int* __restrict__ rowptr,
+                                                  const unsigned long long* __restrict__ keys,
+                                                  const T* __restrict__ v, const int* __restrict__ err,
+                                                  int* __restrict__ col, T* __restrict__ val) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= nnz || *err != 0) return;
+    const unsigned long long mine = keys[e];
+    const unsigned t = (unsigned)mine;
+    const int r = ri[t];
+    const T value = v[t];
+    const int b = rowptr[r], n = rowptr[r + 1] - b;
+    const unsigned long long* k = keys + b;
+    int rank = 0, i = 0;
+    for (; i + 4 <= n; i += 4) {
+        const unsigned long long k0 = k[i], k1 = k[i + 1], k2 = k[i + 2], k3 = k[i + 3];
+        rank += (k0 < mine ? 1 : 0) + (k1 < mine ? 1 : 0) + (k2 < mine ? 1 : 0) + (k3 < mine ? 1 : 0);
+    }
+    for (; i < n; ++i) rank += k[i] < mine ? 1 : 0;
+    col[(int64_t)b + rank] = (int)(mine >> 32);
+    val[(int64_t)b + rank] = value;
+}
+
+// Whether the rows are short on average.
+bool coo_short_rows(int64_t nrows, int64_t nnz) { return nnz > 0 && nnz / 96 <= nrows; }
+
+size_t align256(size_t b) { return (b + 255) / 256 * 256; }
+
+// Workspace of the short-row path: flags, scan partials, places, keys.
+size_t coo_short_bytes(int64_t nrows, int64_t nnz) {
+    return 256 + align256(sizeof(int) * (size_t)scan_partials_needed(nrows + 1)) + align256(sizeof(int) * (size_t)nnz) +
+           sizeof(unsigned long long) * (size_t)nnz;
+}
+
 unsigned grid_of(int64_t n) { return (unsigned)((n + 255) / 256); }
 
+// The short-row path in a workspace of coo_short_bytes; *flags: as `err` of the
+// kernels (4: a long row was found and nothing was written but the row
+// pointers).
+int coo_short(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, const int* d_i, const int* d_j,
+              const void* d_v, int* d_rowptr, int* d_col, void* d_val, void* ws, int* flags, hipStream_t s) {
+    unsigned char* w = reinterpret_cast<unsigned char*>(ws);
+    int* err = reinterpret_cast<int*>(w);
+    int* partials = reinterpret_cast<int*>(w + 256);
+    w += 256 + align256(sizeof(int) * (size_t)scan_partials_needed(nrows + 1));
+    int* place = reinterpret_cast<int*>(w);
+    unsigned long long* keys = reinterpret_cast<unsigned long long*>(w + align256(sizeof(int) * (size_t)nnz));
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, s, err, (int64_t)1, 0);
+    hipLaunchKernelGGL(k_fill_i32, dim3(grid_of(nrows + 1)), dim3(256), 0, s, d_rowptr, nrows + 1, 0);
+    hipLaunchKernelGGL(k_coo_count, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, d_j, nnz, nrows, ncols, d_rowptr, place,
+                       err);
+    SPC5_HIP_TRY(hipGetLastError());
+    const int rc = scan_exclusive_i32_ws(d_rowptr, nrows + 1, nullptr, partials, s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_coo_place, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, d_j, nnz, d_rowptr, place, keys, err);
+    if (value_bytes == 8)
+        hipLaunchKernelGGL(k_coo_rank<double>, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, nnz, d_rowptr, keys,
+                           reinterpret_cast<const double*>(d_v), err, d_col, reinterpret_cast<double*>(d_val));
+    else
+        hipLaunchKernelGGL(k_coo_rank<float>, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, nnz, d_rowptr, keys,
+                           reinterpret_cast<const float*>(d_v), err, d_col, reinterpret_cast<float*>(d_val));
+    SPC5_HIP_TRY(hipGetLastError());
+    SPC5_HIP_TRY(hipMemcpyAsync(flags, err, sizeof(int), hipMemcpyDeviceToHost, s));
+    SPC5_HIP_TRY(hipStreamSynchronize(s));
+    return SPC5_HIP_OK;
+}
+
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return na > 0 && nb > 0 && x < y + nb && y < x + na;
+}
+
+int coo_range_error() {
+    set_error("COO index out of range (row not in [0, nrows) or column not in [0, ncols))");
+    return SPC5_HIP_ERR_INVALID;
+}
+
 int coo_to_csr(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, bool sorted, const int* d_i,
-               const int* d_j, const void* d_v, int* d_rowptr, int* d_col, void* d_val, hipStream_t s) {
+               const int* d_j, const void* d_v, int* d_rowptr, int* d_col, void* d_val, void* ws, hipStream_t s) {
+    // The short-row path reads the rows to the end, so outputs over inputs take
+    // the radix sort, which reads rows and columns first.
+    const size_t in = sizeof(int) * (size_t)nnz, vb = (size_t)value_bytes * (size_t)nnz;
+    const size_t rb = sizeof(int) * (size_t)(nrows + 1);
+    const bool apart = !overlap(d_rowptr, rb, d_i, in) && !overlap(d_rowptr, rb, d_j, in) &&
+                       !overlap(d_rowptr, rb, d_v, vb) && !overlap(d_col, in, d_i, in) &&
+                       !overlap(d_col, in, d_v, vb) && !overlap(d_val, vb, d_i, in) && !overlap(d_val, vb, d_v, vb);
+    if (!sorted && apart && coo_short_rows(nrows, nnz)) {
+        DeviceBuffer own;
+        if (!ws) {
+            SPC5_HIP_TRY(own.alloc(coo_short_bytes(nrows, nnz)));
+            ws = own.p;
+        }
+        int flags = 0;
+        const int rc = coo_short(value_bytes, nrows, ncols, nnz, d_i, d_j, d_v, d_rowptr, d_col, d_val, ws, &flags, s);
+        if (rc) return rc;
+        if (flags & 1) return coo_range_error();
+        if (!(flags & 4)) return SPC5_HIP_OK;
+    }
     DeviceBuffer err;
     SPC5_HIP_TRY(err.alloc(sizeof(int)));
     SPC5_HIP_TRY(hipMemsetAsync(err.p, 0, sizeof(int), s));
@@ -126,10 +266,7 @@ int coo_to_csr(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, bool 
     int herr = 0;
     SPC5_HIP_TRY(hipMemcpyAsync(&herr, err.p, sizeof(int), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipStreamSynchronize(s));
-    if (herr & 1) {
-        set_error("COO index out of range (row not in [0, nrows) or column not in [0, ncols))");
-        return SPC5_HIP_ERR_INVALID;
-    }
+    if (herr & 1) return coo_range_error();
     if (herr & 2) {
         set_error("COO entries not sorted by (row, column)");
         return SPC5_HIP_ERR_INVALID;
@@ -243,16 +380,30 @@ int64_t mm_walk(const MMFile& mm, Emit&& emit) {
 
 extern "C" {
 
-int spc5_hip_coo_to_csr(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, int sorted, const int* d_i,
-                        const int* d_j, const void* d_v, int* d_rowptr, int* d_col, void* d_val, void* stream) {
+int64_t spc5_hip_coo_workspace_bytes(int64_t nrows, int64_t nnz, int sorted) {
+    return !sorted && nrows >= 0 && coo_short_rows(nrows, nnz) ? (int64_t)coo_short_bytes(nrows, nnz) : 0;
+}
+
+int spc5_hip_coo_to_csr_ws(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, int sorted, const int* d_i,
+                           const int* d_j, const void* d_v, int* d_rowptr, int* d_col, void* d_val, void* d_workspace,
+                           int64_t workspace_bytes, void* stream) {
     SPC5_CHECK_ARG(value_bytes == 8 || value_bytes == 4, "value_bytes must be 8 or 4");
     SPC5_CHECK_ARG(nrows >= 0 && ncols >= 0 && nnz >= 0, "negative size");
     SPC5_CHECK_ARG(nrows < ((int64_t)1 << 31) && ncols < ((int64_t)1 << 31) && nnz < ((int64_t)1 << 31),
                    "sizes must fit the 32-bit CSR arrays");
     SPC5_CHECK_ARG(d_rowptr != nullptr, "null rowptr");
     SPC5_CHECK_ARG(nnz == 0 || (d_i && d_j && d_v && d_col && d_val), "null COO or CSR array");
-    return coo_to_csr(value_bytes, nrows, ncols, nnz, sorted != 0, d_i, d_j, d_v, d_rowptr, d_col, d_val,
+    SPC5_CHECK_ARG(d_workspace == nullptr || ((uintptr_t)d_workspace % 256 == 0 &&
+                                              workspace_bytes >= spc5_hip_coo_workspace_bytes(nrows, nnz, sorted)),
+                   "workspace misaligned or too small");
+    return coo_to_csr(value_bytes, nrows, ncols, nnz, sorted != 0, d_i, d_j, d_v, d_rowptr, d_col, d_val, d_workspace,
                       as_stream(stream));
+}
+
+int spc5_hip_coo_to_csr(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, int sorted, const int* d_i,
+                        const int* d_j, const void* d_v, int* d_rowptr, int* d_col, void* d_val, void* stream) {
+    return spc5_hip_coo_to_csr_ws(value_bytes, nrows, ncols, nnz, sorted, d_i, d_j, d_v, d_rowptr, d_col, d_val, nullptr,
+                                  0, stream);
 }
 
 int spc5_hip_mm_info(const char* path, int64_t* nrows, int64_t* ncols, int64_t* nentries) {

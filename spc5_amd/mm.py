@@ -49,9 +49,13 @@ def coo_to_csr(i, j, v, nrows: int, ncols: int, sorted: bool = False, stream=Non
     rowptr = torch.empty(nrows + 1, dtype=torch.int32, device=v.device)
     col = torch.empty(max(nnz, 1), dtype=torch.int32, device=v.device)
     val = torch.empty(max(nnz, 1), dtype=v.dtype, device=v.device)
-    check(lib().spc5_hip_coo_to_csr(v.element_size(), nrows, ncols, nnz, 1 if sorted else 0, i.data_ptr(),
-                                    j.data_ptr(), v.data_ptr(), rowptr.data_ptr(), col.data_ptr(), val.data_ptr(),
-                                    stream_ptr(stream)), "spc5_hip_coo_to_csr")
+    # the call waits for its stream, so the workspace outlives its use
+    need = lib().spc5_hip_coo_workspace_bytes(nrows, nnz, 1 if sorted else 0)
+    ws = torch.empty(need + 255, dtype=torch.uint8, device=v.device) if need else None
+    at = (ws.data_ptr() + 255) // 256 * 256 if need else None
+    check(lib().spc5_hip_coo_to_csr_ws(v.element_size(), nrows, ncols, nnz, 1 if sorted else 0, i.data_ptr(),
+                                       j.data_ptr(), v.data_ptr(), rowptr.data_ptr(), col.data_ptr(), val.data_ptr(),
+                                       at, need, stream_ptr(stream)), "spc5_hip_coo_to_csr")
     return rowptr, col[:nnz], val[:nnz]
 
 
