@@ -161,14 +161,14 @@ int spc5_hip_mat_load(const char* path, spc5_hip_mat_t* out);
  * batch created afterwards uses the new tiles.  No counterpart in the
  * reference (the work split of the GPU kernel). */
 #define SPC5_HIP_OPT_TILE_VALUES 3
-/* SPMM_X16 (0 or 1; default 1 for double vectors, 0 for float): in
- * spc5_hip_spmm each lane requests 16 bytes of an X row (two doubles or four
- * floats, adjacent columns) instead of one element, where X allows it
- * (16-byte aligned X, a leading dimension, k and column chunk that are
- * multiples of the element count); otherwise one element per lane.  Fewer
- * lanes then share a record, which halves (double) or quarters (float) the
- * address work per column.  Results agree with one element per lane to
- * rounding.  No counterpart in the reference. */
+/* SPMM_X16 (0 or 1): in spc5_hip_spmm each lane requests 16 bytes of an X row
+ * (two doubles or four floats, adjacent columns, at any element's address)
+ * instead of one element.  Fewer lanes then share a record, which halves
+ * (double) or quarters (float) the address work per column.  Column chunks
+ * narrower than a request take one element per lane.  Unless set: on for
+ * double vectors, with column records from 3 r columns per chunk.
+ * Results agree with one element per lane to rounding.  No counterpart in the
+ * reference. */
 #define SPC5_HIP_OPT_SPMM_X16 4
 int spc5_hip_mat_set_option(spc5_hip_mat_t h, int option, int64_t value);
 

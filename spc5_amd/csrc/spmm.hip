@@ -9,10 +9,10 @@
 // as in the SpMV tile (headers prefetched, values read once, coalesced, from
 // the value stream) and every value becomes a 16-byte LDS record (value,
 // column, tile-local row), or with column records every set column of a
-// block one record (k_spmm_cols).  The wave then splits into groups of
-// KC / CPL lanes, each lane taking CPL adjacent columns of the chunk (one
-// element, or 16 bytes of the X row with SPC5_HIP_OPT_SPMM_X16); each group
-// walks a contiguous run of the batch's records, requests the X rows of U
+// block one record (k_spmm_cols).  The wave then splits into groups of as many
+// lanes as the chunk's columns need (spmm_lanes), each lane taking CPL adjacent
+// columns (one element, or 16 bytes of the X row, SPC5_HIP_OPT_SPMM_X16); each
+// group walks a contiguous run of the batch's records, requests the X rows of U
 // records at a time (one contiguous kt-wide row segment per record; with
 // 64-column chunks of float or bfloat16 X and one column per lane the whole
 // wave is one group and the records are broadcast to scalar registers) and
@@ -65,9 +65,9 @@ using SpmmFloatAcc = std::conditional<SPC5_SPMM_FLOAT_ACC_DOUBLE != 0, double, f
 // chunks measured slower with it).  Double X keeps vector records: the
 // scalar form measured 2 % slower there (its 512-byte X rows, not
 // occupancy, set the pace).
-template <int KC, class X, int CPL = 1>
+template <bool ONE, class X>
 constexpr int spmm_cap() {
-    return KC == 64 && CPL == 1 && sizeof(X) < 8 ? SPC5_SPMM_CAP64_NARROW : SPC5_SPMM_CAP;
+    return ONE && sizeof(X) < 8 ? SPC5_SPMM_CAP64_NARROW : SPC5_SPMM_CAP;
 }
 // a batch must hold the largest block (r = 8, VS = 16: 128 values)
 static_assert(SPC5_SPMM_CAP >= 128 && SPC5_SPMM_CAP % 64 == 0, "SPC5_SPMM_CAP: a multiple of 64, at least 128");
@@ -103,9 +103,9 @@ int spmm_max_rows(int kt) {
     return rows;
 }
 
-template <class ACC, int KC, class X, int CPL>
+template <class ACC, bool ONE, class X>
 size_t spmm_smem_bytes(int maxrows, int kt, int r) {
-    return sizeof(SpmmRec<ACC>) * spmm_cap<KC, X, CPL>() + sizeof(ACC) * (size_t)maxrows * kt +
+    return sizeof(SpmmRec<ACC>) * spmm_cap<ONE, X>() + sizeof(ACC) * (size_t)maxrows * kt +
            sizeof(int) * (maxrows / r + 1);
 }
 
@@ -120,9 +120,8 @@ __device__ __forceinline__ X spmm_x(const X* __restrict__ xcol, const X* __restr
 }
 
 // CPL adjacent X columns of one record: one X value, or (CPL = 16 /
-// sizeof(X)) one 16-byte load of two doubles or four floats; the caller has
-// checked that every X row start and every lane's first column are then
-// 16-byte aligned.
+// sizeof(X)) one 16-byte load of two doubles or four floats, at any element's
+// address.
 template <int CPL, bool WIDE, class X, class ACC>
 __device__ __forceinline__ void spmm_xs(const X* __restrict__ xcol, const X* __restrict__ x, int col, int64_t ldx,
                                         unsigned lane_off, ACC* out) {
@@ -132,16 +131,15 @@ __device__ __forceinline__ void spmm_xs(const X* __restrict__ xcol, const X* __r
         static_assert(CPL * sizeof(X) == 16, "one 16-byte load per lane");
         const X* p = WIDE ? xcol + (int64_t)col * ldx
                           : reinterpret_cast<const X*>(reinterpret_cast<const char*>(x) + ((unsigned)col + lane_off));
-        const uint4 w = *reinterpret_cast<const uint4*>(p);
         X v[CPL];
-        __builtin_memcpy(v, &w, 16);
+        __builtin_memcpy(v, p, 16);
 #pragma unroll
         for (int e = 0; e < CPL; ++e) out[e] = (ACC)v[e];
     }
 }
 
 // The value of lane l (a compile-time or uniform lane index) on every lane.
-__device__ __forceinline__ float read_lane(float v, int l) {
+[[maybe_unused]] __device__ __forceinline__ float read_lane(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 __device__ __forceinline__ double read_lane(double v, int l) {
@@ -174,25 +172,53 @@ __device__ __forceinline__ bool spmm_item(int64_t ntiles, int k, int kt, int64_t
     return (int64_t)ch * kt < k;  // false for the padding after the last chunk
 }
 
+// How a wave's lanes share a chunk of ktc columns: groups of lpr lanes, lane
+// l of a group taking the CPL columns from jl on.  The last lane of a group
+// takes the chunk's last CPL columns, of which the first `skip` are its
+// neighbour's (computed and not written), so every request stays inside the
+// row whatever ktc is.  Lanes left over hold a group past the last and no record.
+// Groups as wide as the columns need, not the next power of two, and 16-byte
+// requests at any alignment: on the clustered 300 K-row matrix at beta(2,16)
+// in float, k = 7 went 93 -> 89 us (with 16 bytes 86) and k = 33 242 -> 215
+// (with 16 bytes 124).
+struct SpmmLanes {
+    int grp, groups, jl, skip;
+};
+template <int CPL, bool ONE>
+__device__ __forceinline__ SpmmLanes spmm_lanes(int ktc, int lane) {
+    SpmmLanes w;
+    if constexpr (ONE) {
+        // one group; lanes past the chunk repeat its last column
+        w.groups = 1;
+        w.grp = 0;
+        w.jl = lane < ktc ? lane : ktc - 1;
+        w.skip = lane < ktc ? 0 : 1;
+        return w;
+    }
+    const int lpr = (ktc + CPL - 1) / CPL;
+    w.groups = 64 / lpr;
+    w.grp = lane / lpr;
+    const int first = (lane - w.grp * lpr) * CPL;
+    w.jl = first < ktc - CPL ? first : ktc - CPL;
+    w.skip = first - w.jl;
+    return w;
+}
+
 // WIDE: X spans 4 GiB or more (or rows of 16 MiB or more), so records hold
 // columns and X is addressed with 64-bit arithmetic; otherwise they hold
 // 32-bit byte offsets of the X rows, computed with 24-bit multiplies.
 // CPL: adjacent X columns per lane (1, or 16 / sizeof(X): one 16-byte X
-// request), so KC / CPL lanes share a record.
-template <class V, class X, class ACC, int R, int VS, int MB, int KC, bool WIDE, int CPL>
+// request).  ONE: every chunk takes 64 lanes a record (one group, CPL = 1).
+// U: records whose X rows are requested together.
+template <class V, class X, class ACC, int R, int VS, int MB, bool WIDE, int CPL, bool ONE, int U>
 __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr, const unsigned char* __restrict__ hdr,
                                                     const V* __restrict__ val, const X* __restrict__ x, int64_t ldx,
                                                     X* __restrict__ y, int64_t ldy, int k, int kt,
                                                     const int4* __restrict__ tiles,
                                                     int64_t ntiles, int64_t nrows, int maxrows, ACC alpha, ACC beta) {
-    constexpr int CAP = spmm_cap<KC, X, CPL>();
+    constexpr int CAP = spmm_cap<ONE, X>();
     constexpr int K = CAP / 64;
     constexpr int NW = MaskWords<R * MB>::kWords;
-    constexpr int LPR = KC / CPL;  // lanes per record
-    constexpr int G = 64 / LPR;    // record groups per wave
-    // records whose X rows are requested together (half as many with
-    // several columns per lane and more than two groups per wave)
-    constexpr int U = (LPR == 64 ? SPC5_SPMM_U64 : SPC5_SPMM_U) / (CPL > 1 && G > 2 ? 2 : 1);
     using Rec = SpmmRec<ACC>;
     extern __shared__ __align__(16) unsigned char smem[];
     Rec* rec = reinterpret_cast<Rec*>(smem);                            // [CAP]
@@ -204,11 +230,10 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
     if (!spmm_item(ntiles, k, kt, t, c0)) return;
     const int ktc = (k - c0) < kt ? (k - c0) : kt;
     const int lane = lane_id();
-    const int grp = lane / LPR;
-    const int jl = (lane % LPR) * CPL;  // the lane's first column in the chunk
-    const bool colok = jl < ktc;        // ktc is a multiple of CPL
-    const X* __restrict__ xcol = x + c0 + (colok ? jl : 0);
-    const unsigned lane_off = (unsigned)(c0 + (colok ? jl : 0)) * (unsigned)sizeof(X);  // byte offset in an X row
+    const SpmmLanes part = spmm_lanes<CPL, ONE>(ktc, lane);
+    const int grp = part.grp, jl = part.jl;
+    const X* __restrict__ xcol = x + c0 + jl;
+    const unsigned lane_off = (unsigned)(c0 + jl) * (unsigned)sizeof(X);  // byte offset in an X row
     const unsigned row_bytes = (unsigned)ldx * (unsigned)sizeof(X);
     const int4 first = tiles[t], last = tiles[t + 1];
     const int br0 = first.x, br1 = last.x;
@@ -274,7 +299,7 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
         }
         wave_sync();
         // group grp walks records [qa, qb)
-        const int per = (total + G - 1) / G;
+        const int per = ONE ? total : (total + part.groups - 1) / part.groups;
         int q = grp * per;
         const int qb = q + per < total ? q + per : total;
         ACC run[CPL];
@@ -283,14 +308,15 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
         int prow = -1;
         // the running sums of row prow go to the tile's LDS sums
         auto close = [&]() {
-            if (prow >= 0 && colok) {
+            if (prow >= 0) {
 #pragma unroll
-                for (int e = 0; e < CPL; ++e) atomicAdd(&acc[prow * kt + jl + e], run[e]);
+                for (int e = 0; e < CPL; ++e)
+                    if (e >= part.skip) atomicAdd(&acc[prow * kt + jl + e], run[e]);
             }
 #pragma unroll
             for (int e = 0; e < CPL; ++e) run[e] = (ACC)0;
         };
-        if constexpr (KC == 64 && CPL == 1 && !WIDE && sizeof(X) < 8) {
+        if constexpr (ONE && !WIDE && sizeof(X) < 8) {
             // One group: every record is the same on all lanes.  Lane u reads
             // record q + u (one LDS read for U records) and the fields are
             // broadcast to scalars, so the records take no vector registers
@@ -394,9 +420,6 @@ constexpr int spmm_col_cap_val() { return R == 2 ? 256 : (R == 4 ? 384 : 512); }
 // record sequence of its tile in block-row order, so it writes each finished
 // block-row of Y directly (no LDS row x column sums, tiles of up to kMaxRows
 // rows).
-template <int KC, int CPL>
-constexpr bool spmm_col_direct() { return KC == 64 && CPL == 1; }
-
 
 template <class ACC, int R>
 size_t spmm_col_smem_bytes(int maxrows, int kt, bool direct) {
@@ -416,9 +439,9 @@ __device__ __forceinline__ unsigned block_columns(const unsigned long long* mw) 
     return cm;
 }
 
-// KC: the chunk's columns rounded up to a power of two; CPL: adjacent
-// columns per lane (1, or 16 / sizeof(X)), so KC / CPL lanes share a record.
-template <class V, class X, class ACC, int R, int VS, int MB, int KC, bool WIDE, int CPL>
+// CPL, U: as k_spmm_tiles.  DIRECT: every chunk takes 64 lanes a record (one
+// group, CPL = 1), finished block-rows go straight to Y.
+template <class V, class X, class ACC, int R, int VS, int MB, bool WIDE, int CPL, bool DIRECT, int U>
 __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, const unsigned char* __restrict__ hdr,
                                                    const V* __restrict__ val, const X* __restrict__ x, int64_t ldx,
                                                    X* __restrict__ y, int64_t ldy, int k, int kt,
@@ -428,15 +451,6 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
     constexpr int CAP = spmm_col_cap_val<R>();
     constexpr int K = CAP / 64;
     constexpr int NW = MaskWords<R * MB>::kWords;
-    constexpr int LPR = KC / CPL;        // lanes per record
-    constexpr int G = 64 / LPR;          // record groups per wave
-    // X rows requested together.  With several columns per lane and more
-    // than two groups per wave, half as many: k = 64 in double on the
-    // 27-point stencil at beta(4,8) took 3.16 ms with 32-column chunks and 4
-    // requests (3.53 ms with 8), and 2.95 ms with 64-column chunks (two
-    // groups) and 8 requests (3.12 ms with 4).
-    constexpr int U = (R <= 2 ? 16 : 8) / (CPL > 1 && G > 2 ? 2 : 1);
-    constexpr bool DIRECT = spmm_col_direct<KC, CPL>();
     using Rec = SpmmColRec<ACC, R>;
     static_assert(sizeof(Rec) % 16 == 0, "16-byte aligned records");
     extern __shared__ __align__(16) unsigned char smem[];
@@ -450,11 +464,10 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
     if (!spmm_item(ntiles, k, kt, t, c0)) return;
     const int ktc = (k - c0) < kt ? (k - c0) : kt;
     const int lane = lane_id();
-    const int grp = lane / LPR;
-    const int jl = (lane % LPR) * CPL;  // the lane's first column in the chunk
-    const bool colok = jl < ktc;        // ktc is a multiple of CPL
-    const X* __restrict__ xcol = x + c0 + (colok ? jl : 0);
-    const unsigned lane_off = (unsigned)(c0 + (colok ? jl : 0)) * (unsigned)sizeof(X);
+    const SpmmLanes part = spmm_lanes<CPL, DIRECT>(ktc, lane);
+    const int grp = part.grp, jl = part.jl;
+    const X* __restrict__ xcol = x + c0 + jl;
+    const unsigned lane_off = (unsigned)(c0 + jl) * (unsigned)sizeof(X);
     const unsigned row_bytes = (unsigned)ldx * (unsigned)sizeof(X);
     const int4 first = tiles[t], last = tiles[t + 1];
     const int br0 = first.x, br1 = last.x;
@@ -490,7 +503,7 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
 #pragma unroll
             for (int tr = 0; tr < R; ++tr) {
                 const int rr = brow * R + tr;
-                yv[tr] = (beta != (ACC)0 && brow >= 0 && rr < nrow_t && colok) ? y[(row0 + rr) * ldy + c0 + jl]
+                yv[tr] = (beta != (ACC)0 && brow >= 0 && rr < nrow_t && part.skip == 0) ? y[(row0 + rr) * ldy + c0 + jl]
                                                                                  : (X)0;
             }
         }
@@ -499,7 +512,7 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
 #pragma unroll
         for (int tr = 0; tr < R; ++tr) {
             const int rr = brow * R + tr;
-            if (rr < nrow_t && colok) {
+            if (rr < nrow_t && part.skip == 0) {
                 X* yp = &y[(row0 + rr) * ldy + c0 + jl];
                 const ACC s = have ? run[tr][0] : (ACC)0;
                 const ACC yo = beta == (ACC)0 ? (ACC)0 : (have ? (ACC)yv[tr] : (ACC)*yp);
@@ -520,11 +533,12 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
                 skip_to(pb);
                 write_blockrow(pb, true);
                 done = pb + 1;
-            } else if (colok) {
+            } else {
 #pragma unroll
                 for (int tr = 0; tr < R; ++tr)
 #pragma unroll
-                    for (int e = 0; e < CPL; ++e) atomicAdd(&acc[(pb * R + tr) * kt + jl + e], run[tr][e]);
+                    for (int e = 0; e < CPL; ++e)
+                        if (e >= part.skip) atomicAdd(&acc[(pb * R + tr) * kt + jl + e], run[tr][e]);
             }
         }
 #pragma unroll
@@ -607,7 +621,7 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
         }
         wave_sync();
         // group grp walks records [q, qb)
-        const int per = (nrec + G - 1) / G;
+        const int per = DIRECT ? nrec : (nrec + part.groups - 1) / part.groups;
         int q = grp * per;
         const int qb = q + per < nrec ? q + per : nrec;
         for (; q + U <= qb; q += U) {
@@ -663,6 +677,16 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
     }
 }
 
+// 16-byte X requests where the option is not set: double only.  With column
+// records they start at 3 r columns: below, a group's few lanes hold 2 r running
+// sums each and add them to the tile's sums once per block-row and batch
+// (clustered 300 K rows, beta(4,8): k = 3 207 us, 139 with one column a lane;
+// k = 16 173 us, 199 with one).
+template <class X>
+bool spmm_x16_default(bool cols, int r, int kt) {
+    return sizeof(X) == 8 && (!cols || kt >= 3 * r);
+}
+
 struct SpmmPlans {
     std::mutex mu;
     std::map<const spc5_hip_mat*, std::map<int, Plan>> plans;
@@ -679,94 +703,104 @@ unsigned spmm_grid(int64_t ntiles, int k, int kt) {
     return (unsigned)((items + 7) / 8 * 8);
 }
 
-template <class V, class X, class ACC, int VS, int MB, int KC, bool WIDE, int CPL>
-int launch_spmm_cols(const spc5_hip_mat& m, const Plan& p, int maxrows, const void* x, int64_t ldx, void* y,
-                     int64_t ldy, int k, int kt, double alpha, double beta, hipStream_t s) {
-    const dim3 grid(spmm_grid(p.ntiles, k, kt));
-    const int4* tl = p.tiles->as<int4>();
-    const V* val = reinterpret_cast<const V*>(m.values);
-    const X* xx = reinterpret_cast<const X*>(x);
-    X* yy = reinterpret_cast<X*>(y);
-#define SPC5_SPMM_COLS(R)                                                                                          \
-    {                                                                                                              \
-        const size_t shm = spmm_col_smem_bytes<ACC, R>(maxrows, kt, spmm_col_direct<KC, CPL>());                  \
-        hipLaunchKernelGGL((k_spmm_cols<V, X, ACC, R, VS, MB, KC, WIDE, CPL>), grid, dim3(64), shm, s, m.bptr, m.hdr, \
-                           val,                                                                                    \
-                           xx, ldx, yy, ldy, k, kt, tl, p.ntiles, m.nrows, maxrows, (ACC)alpha, (ACC)beta);       \
-    }
-    switch (m.r) {
-    case 2: SPC5_SPMM_COLS(2); break;
-    case 4: SPC5_SPMM_COLS(4); break;
-    case 8: SPC5_SPMM_COLS(8); break;
-    default: set_error("column records need r = 2, 4 or 8"); return SPC5_HIP_ERR_INVALID;
-    }
-#undef SPC5_SPMM_COLS
-    SPC5_HIP_TRY(hipGetLastError());
-    return SPC5_HIP_OK;
+// One launch: everything the kernels need besides the matrix.
+struct SpmmArgs {
+    const Plan* p;
+    int maxrows;
+    const void* x;
+    int64_t ldx;
+    void* y;
+    int64_t ldy;
+    int k, kt;
+    double alpha, beta;
+    hipStream_t s;
+};
+
+template <class V, class X, class ACC, int R, int VS, int MB, bool WIDE, int CPL, bool ONE, int U>
+void launch_spmm_cols(const spc5_hip_mat& m, const SpmmArgs& a) {
+    hipLaunchKernelGGL((k_spmm_cols<V, X, ACC, R, VS, MB, WIDE, CPL, ONE, U>), dim3(spmm_grid(a.p->ntiles, a.k, a.kt)),
+                       dim3(64), (spmm_col_smem_bytes<ACC, R>(a.maxrows, a.kt, ONE)), a.s, m.bptr, m.hdr,
+                       reinterpret_cast<const V*>(m.values), reinterpret_cast<const X*>(a.x), a.ldx,
+                       reinterpret_cast<X*>(a.y), a.ldy, a.k, a.kt, a.p->tiles->as<int4>(), a.p->ntiles, m.nrows,
+                       a.maxrows, (ACC)a.alpha, (ACC)a.beta);
 }
 
-template <class V, class X, class ACC, int VS, int MB, int KC, bool WIDE, int CPL>
-int launch_spmm_vals(const spc5_hip_mat& m, const Plan& p, int maxrows, const void* x, int64_t ldx, void* y,
-                     int64_t ldy, int k, int kt, double alpha, double beta, hipStream_t s) {
-    const dim3 grid(spmm_grid(p.ntiles, k, kt));
-    const size_t shm = spmm_smem_bytes<ACC, KC, X, CPL>(maxrows, kt, m.r);
-    const int4* tl = p.tiles->as<int4>();
-    const V* val = reinterpret_cast<const V*>(m.values);
-    const X* xx = reinterpret_cast<const X*>(x);
-    X* yy = reinterpret_cast<X*>(y);
-#define SPC5_SPMM_LAUNCH(R)                                                                                   \
-    hipLaunchKernelGGL((k_spmm_tiles<V, X, ACC, R, VS, MB, KC, WIDE, CPL>), grid, dim3(64), shm, s, m.bptr, m.hdr, \
-                       val, xx, ldx, yy, ldy, k, kt, tl, p.ntiles, m.nrows, maxrows, (ACC)alpha, (ACC)beta)
-    switch (m.r) {
-    case 1: SPC5_SPMM_LAUNCH(1); break;
-    case 2: SPC5_SPMM_LAUNCH(2); break;
-    case 4: SPC5_SPMM_LAUNCH(4); break;
-    default: SPC5_SPMM_LAUNCH(8); break;
-    }
-#undef SPC5_SPMM_LAUNCH
-    SPC5_HIP_TRY(hipGetLastError());
-    return SPC5_HIP_OK;
+template <class V, class X, class ACC, int R, int VS, int MB, bool WIDE, int CPL, bool ONE, int U>
+void launch_spmm_vals(const spc5_hip_mat& m, const SpmmArgs& a) {
+    hipLaunchKernelGGL((k_spmm_tiles<V, X, ACC, R, VS, MB, WIDE, CPL, ONE, U>),
+                       dim3(spmm_grid(a.p->ntiles, a.k, a.kt)), dim3(64),
+                       (spmm_smem_bytes<ACC, ONE, X>(a.maxrows, a.kt, R)), a.s, m.bptr, m.hdr,
+                       reinterpret_cast<const V*>(m.values), reinterpret_cast<const X*>(a.x), a.ldx,
+                       reinterpret_cast<X*>(a.y), a.ldy, a.k, a.kt, a.p->tiles->as<int4>(), a.p->ntiles, m.nrows,
+                       a.maxrows, (ACC)a.alpha, (ACC)a.beta);
 }
 
-template <class V, class X, class ACC, int VS, int MB, int KC, bool WIDE>
-int launch_spmm_kc(const spc5_hip_mat& m, const Plan& p, int maxrows, const void* x, int64_t ldx, void* y,
-                   int64_t ldy, int k, int kt, double alpha, double beta, bool vec, hipStream_t s) {
+// The kernel for one r: column or value records; 16-byte requests (vec), one
+// column per lane with 64 lanes a record (one), or with fewer.
+// X rows requested together: 16 (values) with one group of 64 lanes, 8 with
+// narrower ones; with several columns per lane half as many where more than two
+// groups share the wave (k = 64 in double on the 27-point stencil at beta(4,8):
+// 3.16 ms with 32-column chunks and 4 requests, 3.53 ms with 8; 2.95 ms with
+// 64-column chunks, two groups, and 8 requests, 3.12 ms with 4).
+template <class V, class X, class ACC, int R, int VS, int MB, bool WIDE>
+void launch_spmm_r(const spc5_hip_mat& m, const SpmmArgs& a, bool cols, bool vec, bool one) {
     constexpr int CPL = 16 / (int)sizeof(X);
-    const bool cols = m.spmm_cols && m.r > 1;
-    if constexpr (KC >= CPL) {
-        if (vec)
-            return cols ? launch_spmm_cols<V, X, ACC, VS, MB, KC, WIDE, CPL>(m, p, maxrows, x, ldx, y, ldy, k, kt,
-                                                                            alpha, beta, s)
-                        : launch_spmm_vals<V, X, ACC, VS, MB, KC, WIDE, CPL>(m, p, maxrows, x, ldx, y, ldy, k, kt,
-                                                                            alpha, beta, s);
+    constexpr bool kTwo = 32 * CPL <= kSpmmMaxKt;
+    const bool two = kTwo && (a.kt + CPL - 1) / CPL > 21;  // at most two groups
+    if constexpr (R > 1) {
+        if (cols) {
+            constexpr int U = R <= 2 ? 16 : 8;
+            if constexpr (kTwo) {
+                if (vec && two) return launch_spmm_cols<V, X, ACC, R, VS, MB, WIDE, CPL, false, U>(m, a);
+            }
+            if (vec)
+                launch_spmm_cols<V, X, ACC, R, VS, MB, WIDE, CPL, false, U / 2>(m, a);
+            else if (one)
+                launch_spmm_cols<V, X, ACC, R, VS, MB, WIDE, 1, true, U>(m, a);
+            else
+                launch_spmm_cols<V, X, ACC, R, VS, MB, WIDE, 1, false, U>(m, a);
+            return;
+        }
     }
-    return cols ? launch_spmm_cols<V, X, ACC, VS, MB, KC, WIDE, 1>(m, p, maxrows, x, ldx, y, ldy, k, kt, alpha, beta, s)
-                : launch_spmm_vals<V, X, ACC, VS, MB, KC, WIDE, 1>(m, p, maxrows, x, ldx, y, ldy, k, kt, alpha, beta, s);
+    if constexpr (kTwo) {
+        if (vec && two) return launch_spmm_vals<V, X, ACC, R, VS, MB, WIDE, CPL, false, SPC5_SPMM_U>(m, a);
+    }
+    if (vec)
+        launch_spmm_vals<V, X, ACC, R, VS, MB, WIDE, CPL, false, SPC5_SPMM_U / 2>(m, a);
+    else if (one)
+        launch_spmm_vals<V, X, ACC, R, VS, MB, WIDE, 1, true, SPC5_SPMM_U64>(m, a);
+    else
+        launch_spmm_vals<V, X, ACC, R, VS, MB, WIDE, 1, false, SPC5_SPMM_U>(m, a);
+}
+
+template <class V, class X, class ACC, int VS, int MB, bool WIDE>
+int launch_spmm_w(const spc5_hip_mat& m, const SpmmArgs& a, bool cols, bool vec, bool one) {
+    switch (m.r) {
+    case 1: launch_spmm_r<V, X, ACC, 1, VS, MB, WIDE>(m, a, cols, vec, one); break;
+    case 2: launch_spmm_r<V, X, ACC, 2, VS, MB, WIDE>(m, a, cols, vec, one); break;
+    case 4: launch_spmm_r<V, X, ACC, 4, VS, MB, WIDE>(m, a, cols, vec, one); break;
+    default: launch_spmm_r<V, X, ACC, 8, VS, MB, WIDE>(m, a, cols, vec, one); break;
+    }
+    SPC5_HIP_TRY(hipGetLastError());
+    return SPC5_HIP_OK;
 }
 
 template <class V, class X, class ACC, int VS, int MB>
 int launch_spmm_t(const spc5_hip_mat& m, const void* x, int64_t ldx, void* y, int64_t ldy, int k, int kt,
                   double alpha, double beta, hipStream_t s) {
-    int kc = 1;  // lanes per record: the smallest power of two holding the chunk's kt columns
-    while (kc < kt) kc <<= 1;
-    // With SPMM_X16, records take 16 / sizeof(X) adjacent columns per lane
-    // (one 16-byte X load) when every chunk's width is a multiple of that
-    // and every X row and chunk start is 16-byte aligned.  A record's X
-    // request then takes a half (double) or a quarter (float) of the lanes,
-    // and the address path and the LDS record reads cost that much less per
-    // column: k = 64 in double on the 27-point stencil (160^3, beta(4,8),
-    // column records) went from 3.65 to 2.95 ms.  For float X it wins or
-    // loses by r and chunk (column records with 64-column chunks: 2.37 ->
-    // 2.74 ms at beta(4,8), 2.28 ms at beta(2,8)), so it is off by default
-    // there.
+    const bool cols = m.spmm_cols && m.r > 1;
+    // With SPMM_X16, a record's X request takes a half (double) or a quarter
+    // (float) of the lanes, and the address path and the LDS record reads cost
+    // that much less per column: k = 64 in double on the 27-point stencil
+    // (160^3, beta(4,8), column records) went from 3.65 to 2.95 ms.  It needs
+    // a whole request in every chunk.
     const int cpl = 16 / (int)sizeof(X);
-    const bool x16 = m.spmm_x16 < 0 ? sizeof(X) == 8 : m.spmm_x16 == 1;
-    const bool vec = x16 && kc >= cpl && k % cpl == 0 && kt % cpl == 0 && ldx % cpl == 0 &&
-                     ((uintptr_t)x & 15u) == 0;
-    // column records with 64-column chunks of one column per lane write Y
-    // directly: whole SpMV-sized tiles
-    const bool direct = m.spmm_cols && m.r > 1 && kc == 64 && !vec;
-    const int maxrows = direct ? kMaxRows : spmm_max_rows<ACC>(kt);
+    const bool x16 = m.spmm_x16 < 0 ? spmm_x16_default<X>(cols, m.r, kt) : m.spmm_x16 == 1;
+    const bool vec = x16 && kt >= cpl && (k % kt == 0 || k % kt >= cpl);
+    // one column per lane and the whole wave on one record; with column
+    // records it writes Y directly, on whole SpMV-sized tiles
+    const bool one = !vec && kt > 32 && (k % kt == 0 || k % kt > 32);
+    const int maxrows = cols && one ? kMaxRows : spmm_max_rows<ACC>(kt);
     Plan* p = nullptr;
     {
         SpmmPlans& sp = spmm_plans();
@@ -793,21 +827,9 @@ int launch_spmm_t(const spc5_hip_mat& m, const void* x, int64_t ldx, void* y, in
     // row is under 16 MiB (the 24-bit multiply of the expansion)
     const uint64_t row_bytes = (uint64_t)ldx * sizeof(X);
     const bool wide = row_bytes >= (1ull << 24) || (uint64_t)m.ncols * row_bytes > 0xffffffffull;
-#define SPC5_SPMM_KC(KC)                                                                                         \
-    return wide ? launch_spmm_kc<V, X, ACC, VS, MB, KC, true>(m, *p, maxrows, x, ldx, y, ldy, k, kt, alpha, beta, \
-                                                               vec, s)                                            \
-                : launch_spmm_kc<V, X, ACC, VS, MB, KC, false>(m, *p, maxrows, x, ldx, y, ldy, k, kt, alpha, beta,  \
-                                                                vec, s)
-    switch (kc) {
-    case 64: SPC5_SPMM_KC(64);
-    case 32: SPC5_SPMM_KC(32);
-    case 16: SPC5_SPMM_KC(16);
-    case 8: SPC5_SPMM_KC(8);
-    case 4: SPC5_SPMM_KC(4);
-    case 2: SPC5_SPMM_KC(2);
-    default: SPC5_SPMM_KC(1);
-    }
-#undef SPC5_SPMM_KC
+    const SpmmArgs a{p, maxrows, x, ldx, y, ldy, k, kt, alpha, beta, s};
+    return wide ? launch_spmm_w<V, X, ACC, VS, MB, true>(m, a, cols, vec, one)
+                : launch_spmm_w<V, X, ACC, VS, MB, false>(m, a, cols, vec, one);
 }
 
 }  // namespace

@@ -204,9 +204,9 @@ class DeviceMatrix:
     @property
     def spmm_x16(self) -> bool:
         """Multi-right-hand-side products request 16 bytes of an X row per
-        lane (two doubles or four floats) where X's layout allows it; on by
-        default for double vectors (see SPC5_HIP_OPT_SPMM_X16 in
-        include/spc5_hip.h)."""
+        lane (two doubles or four floats).  As set; until set, True for
+        double vectors, while the library decides by type, record kind and
+        column chunk (see SPC5_HIP_OPT_SPMM_X16 in include/spc5_hip.h)."""
         return getattr(self, "_spmm_x16", self.vec_dtype == torch.float64)
 
     @spmm_x16.setter
