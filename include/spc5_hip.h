@@ -166,7 +166,8 @@ int spc5_hip_mat_load(const char* path, spc5_hip_mat_t* out);
  * instead of one element.  Fewer lanes then share a record, which halves
  * (double) or quarters (float) the address work per column.  Column chunks
  * narrower than a request take one element per lane.  Unless set: on for
- * double vectors, with column records from 3 r columns per chunk.
+ * double vectors (with column records from 3 r columns per chunk), and for
+ * float vectors with value records from 5 columns (r > 1: up to 48).
  * Results agree with one element per lane to rounding.  No counterpart in the
  * reference. */
 #define SPC5_HIP_OPT_SPMM_X16 4

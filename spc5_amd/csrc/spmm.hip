@@ -204,6 +204,17 @@ __device__ __forceinline__ SpmmLanes spmm_lanes(int ktc, int lane) {
     return w;
 }
 
+// Records a group walks of a batch of n.  From 8 groups on an odd number: the
+// groups read one record each at a time, and at an even distance many of
+// their 16-byte reads meet in the same LDS banks (k = 2 in float, 32 groups
+// 128 bytes apart: 64 -> 53 us on the clustered 300 K-row matrix; k = 8 in
+// float with 16-byte requests: 83 -> 67 us).  Fewer groups meet in few banks
+// anyway, and keep the even split.
+__device__ __forceinline__ int spmm_run(int n, int groups) {
+    const int per = (n + groups - 1) / groups;
+    return groups >= 8 ? per | 1 : per;
+}
+
 // WIDE: X spans 4 GiB or more (or rows of 16 MiB or more), so records hold
 // columns and X is addressed with 64-bit arithmetic; otherwise they hold
 // 32-bit byte offsets of the X rows, computed with 24-bit multiplies.
@@ -269,8 +280,8 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
         const int incl = wave_incl_scan(cnt);
         const int ntake = __popcll(ballot64(valid && incl <= CAP));
         const int total = __builtin_amdgcn_readlane(incl, ntake - 1);
-        ACC a[K];
-        load_values<V, ACC, K>(val, v, total, lane, a);
+        typename ValueBuf<V>::Raw a[K];  // converted where the records take them (next to the load it would wait)
+        load_values_buf<V, K>(val, v, total, lane, a);
         const int jcur = b + lane;
         const int bn = b + ntake;
         load_header_clamped<R, MB>(hdr, bn + lane, b1 - 1, cs, mw);
@@ -295,11 +306,11 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
             const int q = lane + 64 * kk;
-            if (q < total) rec[q].v = a[kk];
+            if (q < total) rec[q].v = ValueBuf<V>::template acc<ACC>(a[kk]);
         }
         wave_sync();
         // group grp walks records [qa, qb)
-        const int per = ONE ? total : (total + part.groups - 1) / part.groups;
+        const int per = ONE ? total : spmm_run(total, part.groups);
         int q = grp * per;
         const int qb = q + per < total ? q + per : total;
         ACC run[CPL];
@@ -316,68 +327,76 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
 #pragma unroll
             for (int e = 0; e < CPL; ++e) run[e] = (ACC)0;
         };
-        if constexpr (ONE && !WIDE && sizeof(X) < 8) {
-            // One group: every record is the same on all lanes.  Lane u reads
-            // record q + u (one LDS read for U records) and the fields are
-            // broadcast to scalars, so the records take no vector registers
-            // and each X row request is a scalar base plus the lane's offset.
-            static_assert(U <= 64 && (U & (U - 1)) == 0, "U: a power of two up to 64");
-            for (; q + U <= qb; q += U) {
-                const Rec mine = rec[q + (lane & (U - 1))];
-                unsigned cu[U];
-                int ru[U];
-                ACC vu[U];
+        // UU records from q on; with PART only the first qb - q of them are
+        // there (the others repeat the last record's request and add nothing):
+        // the remainder of a run waits for one round of requests, where one
+        // record at a time waited up to U - 1 times (clustered 300 K rows,
+        // beta(2,16) float, k = 5, one column a lane: 80 -> 71 us; stencil
+        // 64^3, beta(2,8), k = 64, column records: 226 -> 198 us).
+        auto step = [&](auto uu, auto part_step) {
+            constexpr int UU = decltype(uu)::value;
+            constexpr bool PART = decltype(part_step)::value;
+            if constexpr (ONE && !WIDE && sizeof(X) < 8) {
+                // One group: every record is the same on all lanes.  Lane u
+                // reads record q + u (one LDS read for UU records) and the
+                // fields are broadcast to scalars, so the records take no
+                // vector registers and each X row request is a scalar base
+                // plus the lane's offset.
+                static_assert(UU <= 64 && (UU & (UU - 1)) == 0, "UU: a power of two up to 64");
+                const int left = __builtin_amdgcn_readfirstlane(qb - q);
+                const int mu = lane & (UU - 1);
+                const Rec mine = rec[q + (!PART || mu < left ? mu : left - 1)];
+                unsigned cu[UU];
+                int ru[UU];
+                ACC vu[UU];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
+                for (int u = 0; u < UU; ++u) {
                     cu[u] = (unsigned)__builtin_amdgcn_readlane(mine.col, u);
                     ru[u] = __builtin_amdgcn_readlane(mine.row, u);
                     vu[u] = read_lane(mine.v, u);
                 }
-                ACC xv[U];
+                ACC xv[UU];
 #pragma unroll
-                for (int u = 0; u < U; ++u)
+                for (int u = 0; u < UU; ++u)
                     xv[u] = (ACC) * reinterpret_cast<const X*>(reinterpret_cast<const char*>(x) + cu[u] + lane_off);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
+                for (int u = 0; u < UU; ++u) {
                     if (ru[u] != prow) {
                         close();
                         prow = ru[u];
                     }
-                    run[0] += vu[u] * xv[u];
+                    const ACC sum = run[0] + vu[u] * xv[u];
+                    run[0] = !PART || u < left ? sum : run[0];
                 }
-            }
-        } else {
-            for (; q + U <= qb; q += U) {
-                Rec rr[U];
+            } else {
+                Rec rr[UU];
 #pragma unroll
-                for (int u = 0; u < U; ++u) rr[u] = rec[q + u];
-                // All U record reads are issued before the first use waits.
+                for (int u = 0; u < UU; ++u) rr[u] = rec[!PART || q + u < qb ? q + u : qb - 1];
+                // All UU record reads are issued before the first use waits.
                 __builtin_amdgcn_sched_barrier(0);
-                ACC xv[U][CPL];
+                ACC xv[UU][CPL];
 #pragma unroll
-                for (int u = 0; u < U; ++u) spmm_xs<CPL, WIDE>(xcol, x, rr[u].col, ldx, lane_off, xv[u]);
+                for (int u = 0; u < UU; ++u) spmm_xs<CPL, WIDE>(xcol, x, rr[u].col, ldx, lane_off, xv[u]);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
+                for (int u = 0; u < UU; ++u) {
                     if (rr[u].row != prow) {
                         close();
                         prow = rr[u].row;
                     }
 #pragma unroll
-                    for (int e = 0; e < CPL; ++e) run[e] += rr[u].v * xv[u][e];
+                    for (int e = 0; e < CPL; ++e) {
+                        const ACC sum = run[e] + rr[u].v * xv[u][e];
+                        run[e] = !PART || q + u < qb ? sum : run[e];
+                    }
                 }
             }
-        }
-        for (; q < qb; ++q) {
-            const Rec r1 = rec[q];
-            ACC xv[CPL];
-            spmm_xs<CPL, WIDE>(xcol, x, r1.col, ldx, lane_off, xv);
-            if (r1.row != prow) {
-                close();
-                prow = r1.row;
-            }
-#pragma unroll
-            for (int e = 0; e < CPL; ++e) run[e] += r1.v * xv[e];
-        }
+            q += UU;
+        };
+        while (q + U <= qb) step(std::integral_constant<int, U>{}, std::false_type{});
+        if (q + U / 2 < qb)
+            step(std::integral_constant<int, U>{}, std::true_type{});
+        else if (q < qb)
+            step(std::integral_constant<int, U / 2>{}, std::true_type{});
         close();
         v += total;
         b = bn;
@@ -573,8 +592,8 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
         const int ntake = __popcll(ballot64(valid && incl <= CAP && inclr <= CAPR));
         const int total = __builtin_amdgcn_readlane(incl, ntake - 1);
         const int nrec = __builtin_amdgcn_readlane(inclr, ntake - 1);
-        ACC a[K];
-        load_values<V, ACC, K>(val, v, total, lane, a);
+        typename ValueBuf<V>::Raw a[K];  // converted where the records take them (next to the load it would wait)
+        load_values_buf<V, K>(val, v, total, lane, a);
         const int jcur = b + lane;
         const int bn = b + ntake;
         load_header_clamped<R, MB>(hdr, bn + lane, b1 - 1, cs, mw);
@@ -617,45 +636,45 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
             const int q = lane + 64 * kk;
-            if (q < total) *reinterpret_cast<ACC*>(reinterpret_cast<unsigned char*>(rec) + slot[q]) = a[kk];
+            if (q < total)
+                *reinterpret_cast<ACC*>(reinterpret_cast<unsigned char*>(rec) + slot[q]) = ValueBuf<V>::template acc<ACC>(a[kk]);
         }
         wave_sync();
         // group grp walks records [q, qb)
-        const int per = DIRECT ? nrec : (nrec + part.groups - 1) / part.groups;
+        const int per = DIRECT ? nrec : spmm_run(nrec, part.groups);
         int q = grp * per;
         const int qb = q + per < nrec ? q + per : nrec;
-        for (; q + U <= qb; q += U) {
-            int cu[U], bu[U];
+        auto step = [&](auto uu, auto part_step) {  // as k_spmm_tiles
+            constexpr int UU = decltype(uu)::value;
+            constexpr bool PART = decltype(part_step)::value;
+            int cu[UU], bu[UU];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int2 hb = *reinterpret_cast<const int2*>(&rec[q + u]);
+            for (int u = 0; u < UU; ++u) {
+                const int2 hb = *reinterpret_cast<const int2*>(&rec[!PART || q + u < qb ? q + u : qb - 1]);
                 cu[u] = hb.x;
                 bu[u] = hb.y;
             }
-            // all U X rows are requested before the first use waits
+            // all UU X rows are requested before the first use waits
             __builtin_amdgcn_sched_barrier(0);
-            ACC xv[U][CPL];
+            ACC xv[UU][CPL];
 #pragma unroll
-            for (int u = 0; u < U; ++u) spmm_xs<CPL, WIDE>(xcol, x, cu[u], ldx, lane_off, xv[u]);
+            for (int u = 0; u < UU; ++u) spmm_xs<CPL, WIDE>(xcol, x, cu[u], ldx, lane_off, xv[u]);
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
+            for (int u = 0; u < UU; ++u) {
                 if (bu[u] != pb) flush(bu[u]);
+                if (PART && q + u >= qb) break;
 #pragma unroll
                 for (int tr = 0; tr < R; ++tr)
 #pragma unroll
                     for (int e = 0; e < CPL; ++e) run[tr][e] += rec[q + u].v[tr] * xv[u][e];
             }
-        }
-        for (; q < qb; ++q) {
-            const int2 hb = *reinterpret_cast<const int2*>(&rec[q]);
-            ACC xv[CPL];
-            spmm_xs<CPL, WIDE>(xcol, x, hb.x, ldx, lane_off, xv);
-            if (hb.y != pb) flush(hb.y);
-#pragma unroll
-            for (int tr = 0; tr < R; ++tr)
-#pragma unroll
-                for (int e = 0; e < CPL; ++e) run[tr][e] += rec[q].v[tr] * xv[e];
-        }
+            q += UU;
+        };
+        while (q + U <= qb) step(std::integral_constant<int, U>{}, std::false_type{});
+        if (q + U / 2 < qb)
+            step(std::integral_constant<int, U>{}, std::true_type{});
+        else if (q < qb)
+            step(std::integral_constant<int, U / 2>{}, std::true_type{});
         // groups end their runs with the batch (each batch splits anew);
         // one group keeps its block-row open across batches
         if constexpr (!DIRECT) flush(-1);
@@ -677,14 +696,20 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
     }
 }
 
-// 16-byte X requests where the option is not set: double only.  With column
-// records they start at 3 r columns: below, a group's few lanes hold 2 r running
-// sums each and add them to the tile's sums once per block-row and batch
-// (clustered 300 K rows, beta(4,8): k = 3 207 us, 139 with one column a lane;
-// k = 16 173 us, 199 with one).
+// 16-byte X requests where the option is not set.  Value records: from 5
+// columns in float, always in double (clustered 300 K rows, beta(2,16) float,
+// one column a lane and 16 bytes: k = 4 55 / 65 us, k = 5 71 / 63, k = 16
+// 93 / 79; beta(2,8) double: k = 3 52 / 54, k = 5 63 / 63, k = 16 112 / 90).
+// Past 48 columns in float only at r = 1 (k = 64: 214 / 172): with r > 1 the
+// scalar records win where rows of a block alternate quickly (stencil 64^3,
+// beta(4,16): 162 / 192; clustered 228 / 190).  Column records: double from 3 r columns; below, a group's
+// few lanes hold 2 r running sums each and add them to the tile's sums once
+// per block-row and batch (beta(4,8): k = 8 153 / 165 us, k = 16 189 / 174);
+// float keeps one column a lane (beta(4,16), stencil 64^3: k = 32 107 / 120).
 template <class X>
 bool spmm_x16_default(bool cols, int r, int kt) {
-    return sizeof(X) == 8 && (!cols || kt >= 3 * r);
+    if (cols) return sizeof(X) == 8 && kt >= 3 * r;
+    return sizeof(X) == 8 || (kt >= 5 && (kt <= 48 || r == 1));
 }
 
 struct SpmmPlans {
