@@ -4,9 +4,9 @@
 //
 // CG iteration, scalars kept on the device (no host round trip):
 //   K1  q = A p            (SpMV, y = A x epilogue; each tile writes its
-//                           partial of p.q) -> pq = sum of the partials
-//   K2  r -= alpha q       (alpha = rr / pq); per-workgroup partials of r.r
-//                           -> rr_new
+//                           partial of p.q)
+//   K2  pq = sum of the tiles' partials; r -= alpha q  (alpha = rr / pq);
+//                           per-workgroup partials of r.r -> rr_new
 //   K3  x += alpha p, p = r + beta p   (beta = rr_new / rr)
 // rr and rr_new alternate between two device slots from one iteration to
 // the next.  Reductions never use global atomics: partials are summed in a
@@ -42,22 +42,32 @@ namespace {
 
 // Workgroups of the first stage of the p.q reduction (see k_reduce_stage).
 constexpr int kSumGroups = 64;
+// The iteration's vector kernels: at most one workgroup of 8 waves per CU, so
+// that few workgroups read the partials again and few partials are left.
+constexpr int kCgThreads = 512;
+constexpr int kCgGroups = 256;
+// Most tiles whose p.q partials every workgroup of K2 sums itself: a launch and
+// its gap less per iteration (4.6 us of kernel for 13.8 K tiles) for 4 us at
+// most in K2, where 64 sums of a first stage take 1 us.
+constexpr int64_t kCgPartials = 16384;
 
 // Device scalars of CG.  Iteration i reads r.r from rr[i & 1] and writes
 // the new r.r to rr[(i + 1) & 1], so no kernel has to rotate them.  pq_stage
-// holds the first-stage sums of the product's p.q partials.
+// holds the first-stage sums of the product's p.q partials (many tiles),
+// rr_part the partials of r.r.
 struct CgScalars {
     double rr[2];
     double pq;
     double pad;
     double pq_stage[kSumGroups];
+    double rr_part[kCgGroups];
 };
 
 constexpr int kVecThreads = 256;
 #ifndef SPC5_VEC_GROUPS
 #define SPC5_VEC_GROUPS 2048
 #endif
-constexpr int kMaxVecGroups = SPC5_VEC_GROUPS;  // most workgroups of a vector kernel (and partials)
+constexpr int kMaxVecGroups = SPC5_VEC_GROUPS;  // most workgroups of the other vector kernels (and partials)
 
 __device__ __forceinline__ double block_sum(double v, double* s_part) {
     v = wave_sum_f64(v);
@@ -169,7 +179,8 @@ __global__ __launch_bounds__(kVecThreads) void k_add_scaled_f32(double* __restri
 // CU): workgroup w sums the contiguous range [w c, (w+1) c) of the n
 // partials, c = ceil(n / kSumGroups), in a fixed order (thread t adds
 // elements t, t + kVecThreads, ... of the range, 4 loads in flight; then the
-// wave and workgroup sums) into out[w].  k_cg_r adds the kSumGroups sums.
+// wave and workgroup sums) into out[w].  k_cg_r adds the kSumGroups sums.  Only
+// for products of more than kCgPartials tiles.
 __global__ __launch_bounds__(kVecThreads) void k_reduce_stage(const double* __restrict__ part, int64_t n,
                                                               double* __restrict__ out) {
     __shared__ double s_part[kVecThreads / 64];
@@ -191,89 +202,179 @@ __global__ __launch_bounds__(kVecThreads) void k_reduce_stage(const double* __re
     if (threadIdx.x == 0) out[blockIdx.x] = acc;
 }
 
-// K2: p.q = sum of the kSumGroups first-stage sums (workgroup 0 stores it in
-// sc->pq for K3); r -= alpha q; partials of r.r (par: parity of the
-// iteration)
+// E elements (16 bytes) of a vector from any element on.
 template <class X>
-__global__ __launch_bounds__(kVecThreads) void k_cg_r(X* __restrict__ r, const X* __restrict__ q, int64_t n,
-                                                      CgScalars* __restrict__ sc, int par, double* __restrict__ part) {
-    static_assert(kSumGroups == 64, "one first-stage sum per lane");
-    __shared__ double s_part[kVecThreads / 64];
-    // every wave adds the same 64 sums by the same xor butterfly: one value
-    // in every lane of every workgroup
-    const double pq = wave_sum_f64(sc->pq_stage[threadIdx.x & 63]);
-    if (blockIdx.x == 0 && threadIdx.x == 0) sc->pq = pq;
-    const X alpha = (X)(sc->rr[par] / pq);
-    double p = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * kVecThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kVecThreads) {
-        const X ri = r[i] - alpha * q[i];
-        r[i] = ri;
-        p += (double)ri * (double)ri;
-    }
-    p = block_sum(p, s_part);
-    if (threadIdx.x == 0) part[blockIdx.x] = p;
-}
+struct CgVec {
+    static constexpr int E = 16 / (int)sizeof(X);
+    X v[E];
+    __device__ __forceinline__ void load(const X* p) { __builtin_memcpy(v, p, 16); }
+    __device__ __forceinline__ void store(X* p) const { __builtin_memcpy(p, v, 16); }
+};
 
-// sum of part[0..m) (m <= kMaxVecGroups) in a fixed order, the same value in
-// every thread of every workgroup that calls it: thread t adds part[t],
-// part[t + kVecThreads], ...; the xor butterfly leaves identical sums in all
-// lanes (each step adds the same two values in either order), and every
-// thread adds the wave sums in wave order.  Replaces a separate reduction
-// launch: the partials stay in L2 and each workgroup reads them itself.
+// sum of part[0..m) in a fixed order, the same value in every thread of every
+// workgroup that calls it: thread t adds part[t], part[t + kCgThreads], ...
+// (8 loads in flight); the xor butterfly leaves identical sums in all lanes
+// (each step adds the same two values in either order), and every thread adds
+// the wave sums in wave order.
 __device__ __forceinline__ double sum_partials_all(const double* __restrict__ part, unsigned m,
                                                    double* __restrict__ s_part) {
-    constexpr int kLoads = kMaxVecGroups / kVecThreads;
-    static_assert(kMaxVecGroups % kVecThreads == 0 && kMaxVecGroups >= kVecThreads,
-                  "SPC5_VEC_GROUPS must be a positive multiple of the vector workgroup size");
-    double v[kLoads];
-#pragma unroll
-    for (int k = 0; k < kLoads; ++k) {
-        const unsigned i = (unsigned)k * kVecThreads + threadIdx.x;
-        const unsigned off = (i < m ? i : m - 1) * (unsigned)sizeof(double);
-        v[k] = *(const double*)((const char*)part + off);
-    }
+    constexpr int kLoads = 8;
     double acc = 0.0;
+    for (unsigned i0 = 0; i0 < m; i0 += kLoads * kCgThreads) {
+        double v[kLoads];
 #pragma unroll
-    for (int k = 0; k < kLoads; ++k) acc += (unsigned)k * kVecThreads + threadIdx.x < m ? v[k] : 0.0;
+        for (int k = 0; k < kLoads; ++k) {
+            const unsigned i = i0 + (unsigned)k * kCgThreads + threadIdx.x;
+            v[k] = part[i < m ? i : m - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k) acc += i0 + (unsigned)k * kCgThreads + threadIdx.x < m ? v[k] : 0.0;
+    }
     acc = wave_sum_f64(acc);
     if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = acc;
     __syncthreads();
     double t = 0.0;
 #pragma unroll
-    for (int w = 0; w < kVecThreads / 64; ++w) t += s_part[w];
+    for (int w = 0; w < kCgThreads / 64; ++w) t += s_part[w];
     return t;
+}
+
+// sum of the m <= kCgGroups partials of r.r in a fixed order, on every wave.
+__device__ __forceinline__ double sum_rr(const CgScalars* __restrict__ sc, unsigned m) {
+    constexpr int kLoads = kCgGroups / 64;
+    double v[kLoads], acc = 0.0;
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+        const unsigned i = (unsigned)k * 64 + (threadIdx.x & 63);
+        v[k] = sc->rr_part[i < m ? i : m - 1];
+    }
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) acc += (unsigned)k * 64 + (threadIdx.x & 63) < m ? v[k] : 0.0;
+    return wave_sum_f64(acc);
+}
+
+// This thread's share of the first n / E whole vectors: f(i, V...) with the
+// vectors at element i of every pointer loaded, the next round's loads issued
+// before.  `ready()` is called once, with the first loads in flight: what it
+// waits for (the sums a kernel starts with) overlaps them.  Then g(i) for the
+// element of the remainder this thread holds, if any.
+template <class X, int N, class Ready, class F, class G>
+__device__ __forceinline__ void cg_elements(int64_t n, const X* const (&in)[N], Ready&& ready, F&& f, G&& g) {
+    constexpr int E = CgVec<X>::E;
+    const int64_t nv = n / E;
+    const int64_t first = (int64_t)blockIdx.x * kCgThreads + threadIdx.x;
+    const int64_t step = (int64_t)gridDim.x * kCgThreads;
+    CgVec<X> v[N];
+    auto load = [&](int64_t i) {
+        if (nv > 0) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) v[k].load(in[k] + (i < nv ? i : nv - 1) * E);
+        }
+    };
+    load(first);
+    ready();
+    for (int64_t i = first; i < nv; i += step) {
+        CgVec<X> c[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) c[k] = v[k];
+        if (i + step < nv) load(i + step);
+        f(i * E, c);
+    }
+    if (first < n - nv * E) g(nv * E + first);
+}
+
+// K2: p.q = sum of m partials (the tiles', or the first stage's; workgroup 0
+// stores it in sc->pq for K3); r -= alpha q; partials of r.r (par: parity of
+// the iteration).  Bound by launch and latency up to some 100 K rows, then HBM.
+template <class X>
+__global__ __launch_bounds__(kCgThreads) void k_cg_r(X* r, const X* __restrict__ q, int64_t n,
+                                                     CgScalars* __restrict__ sc, int par,
+                                                     const double* __restrict__ pq_part, unsigned m) {
+    __shared__ double s_part[kCgThreads / 64], s_rr[kCgThreads / 64];
+    X alpha;
+    double p = 0.0;
+    const X* const in[2] = {r, q};
+    cg_elements<X, 2>(
+        n, in,
+        [&] {
+            const double pq = sum_partials_all(pq_part, m, s_part);
+            if (blockIdx.x == 0 && threadIdx.x == 0) sc->pq = pq;
+            alpha = (X)(sc->rr[par] / pq);
+        },
+        [&](int64_t i, CgVec<X>(&v)[2]) {
+#pragma unroll
+            for (int e = 0; e < CgVec<X>::E; ++e) {
+                v[0].v[e] -= alpha * v[1].v[e];
+                p += (double)v[0].v[e] * (double)v[0].v[e];
+            }
+            v[0].store(r + i);
+        },
+        [&](int64_t i) {
+            const X ri = r[i] - alpha * q[i];
+            r[i] = ri;
+            p += (double)ri * (double)ri;
+        });
+    p = wave_sum_f64(p);
+    if ((threadIdx.x & 63) == 0) s_rr[threadIdx.x >> 6] = p;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < kCgThreads / 64; ++w) t += s_rr[w];
+        sc->rr_part[blockIdx.x] = t;
+    }
 }
 
 // K3: rr' = sum of the m partials of r.r left by K2 (workgroup 0 stores it in
 // sc->rr[par ^ 1]); x += alpha p; p = r + beta p
 template <class X>
-__global__ __launch_bounds__(kVecThreads) void k_cg_xp(X* __restrict__ x, X* __restrict__ p, const X* __restrict__ r,
-                                                       int64_t n, CgScalars* __restrict__ sc, int par,
-                                                       const double* __restrict__ part, unsigned m) {
-    __shared__ double s_part[kVecThreads / 64];
-    const double rr = sc->rr[par];
-    const double rr_new = sum_partials_all(part, m, s_part);
-    if (blockIdx.x == 0 && threadIdx.x == 0) sc->rr[par ^ 1] = rr_new;
-    const X alpha = (X)(rr / sc->pq);
-    const X beta = (X)(rr_new / rr);
-    for (int64_t i = (int64_t)blockIdx.x * kVecThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kVecThreads) {
-        const X pi = p[i];
-        x[i] += alpha * pi;
-        p[i] = r[i] + beta * pi;
-    }
+__global__ __launch_bounds__(kCgThreads) void k_cg_xp(X* x, X* p, const X* __restrict__ r,
+                                                      int64_t n, CgScalars* __restrict__ sc, int par, unsigned m) {
+    X alpha, beta;
+    const X* const in[3] = {x, p, r};
+    cg_elements<X, 3>(
+        n, in,
+        [&] {
+            const double rr = sc->rr[par];
+            const double rr_new = sum_rr(sc, m);
+            if (blockIdx.x == 0 && threadIdx.x == 0) sc->rr[par ^ 1] = rr_new;
+            alpha = (X)(rr / sc->pq);
+            beta = (X)(rr_new / rr);
+        },
+        [&](int64_t i, CgVec<X>(&v)[3]) {
+#pragma unroll
+            for (int e = 0; e < CgVec<X>::E; ++e) {
+                v[0].v[e] += alpha * v[1].v[e];
+                v[1].v[e] = v[2].v[e] + beta * v[1].v[e];
+            }
+            v[0].store(x + i);
+            v[1].store(p + i);
+        },
+        [&](int64_t i) {
+            const X pi = p[i];
+            x[i] += alpha * pi;
+            p[i] = r[i] + beta * pi;
+        });
 }
 
 // K3 split in two around a reliable update: rr' as in K3; x += alpha p ...
 template <class X>
-__global__ __launch_bounds__(kVecThreads) void k_cg_x(X* __restrict__ x, const X* __restrict__ p, int64_t n,
-                                                      CgScalars* __restrict__ sc, int par,
-                                                      const double* __restrict__ part, unsigned m) {
-    __shared__ double s_part[kVecThreads / 64];
-    const double rr_new = sum_partials_all(part, m, s_part);
-    if (blockIdx.x == 0 && threadIdx.x == 0) sc->rr[par ^ 1] = rr_new;
-    const X alpha = (X)(sc->rr[par] / sc->pq);
-    for (int64_t i = (int64_t)blockIdx.x * kVecThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kVecThreads)
-        x[i] += alpha * p[i];
+__global__ __launch_bounds__(kCgThreads) void k_cg_x(X* x, const X* __restrict__ p, int64_t n,
+                                                     CgScalars* __restrict__ sc, int par, unsigned m) {
+    X alpha;
+    const X* const in[2] = {x, p};
+    cg_elements<X, 2>(
+        n, in,
+        [&] {
+            const double rr_new = sum_rr(sc, m);
+            if (blockIdx.x == 0 && threadIdx.x == 0) sc->rr[par ^ 1] = rr_new;
+            alpha = (X)(sc->rr[par] / sc->pq);
+        },
+        [&](int64_t i, CgVec<X>(&v)[2]) {
+#pragma unroll
+            for (int e = 0; e < CgVec<X>::E; ++e) v[0].v[e] += alpha * v[1].v[e];
+            v[0].store(x + i);
+        },
+        [&](int64_t i) { x[i] += alpha * p[i]; });
 }
 
 // ... and p = r + beta p
@@ -368,6 +469,26 @@ unsigned vec_grid(int64_t n) {
     return (unsigned)g;
 }
 
+// Workgroups of K2 and K3.
+unsigned cg_grid(int64_t n, int64_t elem_bytes) {
+    const int64_t vecs = std::max<int64_t>(1, n * elem_bytes / 16);
+    return (unsigned)std::min<int64_t>(kCgGroups, (vecs + kCgThreads - 1) / kCgThreads);
+}
+
+// K2 after a product of `ntiles` tiles, whose p.q partials are in `part`.
+template <class X>
+void launch_cg_r(X* r, const X* q, int64_t n, CgScalars* sc, int par, const double* part, int64_t ntiles,
+                 hipStream_t t) {
+    const unsigned g = cg_grid(n, sizeof(X));
+    if (ntiles <= kCgPartials) {
+        hipLaunchKernelGGL(k_cg_r<X>, dim3(g), dim3(kCgThreads), 0, t, r, q, n, sc, par, part, (unsigned)ntiles);
+        return;
+    }
+    hipLaunchKernelGGL(k_reduce_stage, dim3(kSumGroups), dim3(kVecThreads), 0, t, part, ntiles, sc->pq_stage);
+    hipLaunchKernelGGL(k_cg_r<X>, dim3(g), dim3(kCgThreads), 0, t, r, q, n, sc, par, (const double*)sc->pq_stage,
+                       (unsigned)kSumGroups);
+}
+
 // *d_out = a.b (partials in `part`, at least vec_grid(n) doubles)
 template <class X>
 int dot(const X* a, const X* b, int64_t n, double* part, double* d_out, hipStream_t s) {
@@ -391,7 +512,7 @@ int read_scalar(const double* d, double* h, hipStream_t s) {
 template <class X>
 int cg_run(const spc5_hip_mat& A, X* x, X* r, X* p, X* q, CgScalars* sc, double* part, int64_t n, int check,
            int maxit, double stop2, int& it, double& hrr, hipStream_t s) {
-    const unsigned g = vec_grid(n);
+    const unsigned g = cg_grid(n, sizeof(X));
     Epilogue ek1;
     ek1.alpha = 1.0;
     ek1.beta = 0.0;
@@ -400,10 +521,8 @@ int cg_run(const spc5_hip_mat& A, X* x, X* r, X* p, X* q, CgScalars* sc, double*
     auto iteration = [&](hipStream_t t, int par) -> int {
         int e;
         if ((e = launch_spmv(A, p, q, t, ek1))) return e;
-        hipLaunchKernelGGL(k_reduce_stage, dim3(kSumGroups), dim3(kVecThreads), 0, t, part, A.plan.ntiles,
-                           sc->pq_stage);
-        hipLaunchKernelGGL(k_cg_r<X>, dim3(g), dim3(kVecThreads), 0, t, r, q, n, sc, par, part);
-        hipLaunchKernelGGL(k_cg_xp<X>, dim3(g), dim3(kVecThreads), 0, t, x, p, r, n, sc, par, part, g);
+        launch_cg_r<X>(r, q, n, sc, par, part, A.plan.ntiles, t);
+        hipLaunchKernelGGL(k_cg_xp<X>, dim3(g), dim3(kCgThreads), 0, t, x, p, r, n, sc, par, g);
         SPC5_HIP_TRY(hipGetLastError());
         return SPC5_HIP_OK;
     };
@@ -540,7 +659,7 @@ int mixed_cg_impl(const spc5_hip_mat& A64, const spc5_hip_mat& Alo, const double
     double* part = vpart.as<double>();
     double* d_bb = vtmp.as<double>();
     double* d_rr = d_bb + 1;
-    const unsigned g = vec_grid(n);
+    const unsigned g = vec_grid(n), gc = cg_grid(n, sizeof(XV));
     int rc;
     Epilogue eres;  // r64 = b - A64 x64 (r64 holds a copy of b)
     eres.alpha = -1.0;
@@ -586,13 +705,11 @@ int mixed_cg_impl(const spc5_hip_mat& A64, const spc5_hip_mat& Alo, const double
     auto iteration = [&](hipStream_t t, int par, bool last) -> int {
         int e;
         if ((e = spmv_lo(t))) return e;
-        hipLaunchKernelGGL(k_reduce_stage, dim3(kSumGroups), dim3(kVecThreads), 0, t, part, Alo.plan.ntiles,
-                           sc->pq_stage);
-        hipLaunchKernelGGL(k_cg_r<XV>, dim3(g), dim3(kVecThreads), 0, t, r, q, n, sc, par, part);
+        launch_cg_r<XV>(r, q, n, sc, par, part, Alo.plan.ntiles, t);
         if (!last)
-            hipLaunchKernelGGL(k_cg_xp<XV>, dim3(g), dim3(kVecThreads), 0, t, d, p, r, n, sc, par, part, g);
+            hipLaunchKernelGGL(k_cg_xp<XV>, dim3(gc), dim3(kCgThreads), 0, t, d, p, r, n, sc, par, gc);
         else
-            hipLaunchKernelGGL(k_cg_x<XV>, dim3(g), dim3(kVecThreads), 0, t, d, p, n, sc, par, part, g);
+            hipLaunchKernelGGL(k_cg_x<XV>, dim3(gc), dim3(kCgThreads), 0, t, d, p, n, sc, par, gc);
         SPC5_HIP_TRY(hipGetLastError());
         return SPC5_HIP_OK;
     };
