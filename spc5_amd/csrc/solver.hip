@@ -11,8 +11,10 @@
 // rr and rr_new alternate between two device slots from one iteration to
 // the next.  Reductions never use global atomics: partials are summed in a
 // fixed order by one workgroup, so a solve is bit-reproducible.  The host
-// reads rr every `check` iterations to stop; a chunk of `check` iterations
-// is recorded once into a hipGraph and replayed.
+// reads rr every `check` iterations to stop and launches the iterations in
+// between directly: a recorded chunk's launch hands its kernels over no faster,
+// and its stream, capture and instantiation cost every solve (24^3 stencil, 72
+// iterations: 1345 us recorded, 1215 direct; 96^3: 18.5 and 18.1 ms).
 //
 // Iterative refinement (IR-CG): x64 = 0, r64 = b; repeat
 //   r32 = r64 / ||r64||  (float);  solve A_lo d = r32 with float CG to a
@@ -32,7 +34,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <cstdlib>
 #include <vector>
 
 using namespace spc5;
@@ -427,52 +428,6 @@ __global__ void k_cg_init_scalars(CgScalars* sc, const double* __restrict__ rr) 
     sc->pad = 0.0;
 }
 
-// A fixed sequence of launches recorded once into a hipGraph on a private
-// stream and replayed on the caller's stream (fewer launch gaps per CG
-// iteration).  SPC5_CG_GRAPH=0 in the environment launches directly.
-class ChunkGraph {
-  public:
-    ChunkGraph() = default;
-    ChunkGraph(const ChunkGraph&) = delete;
-    ChunkGraph& operator=(const ChunkGraph&) = delete;
-    ~ChunkGraph() {
-        if (exec_) (void)hipGraphExecDestroy(exec_);
-        if (graph_) (void)hipGraphDestroy(graph_);
-        if (cs_) (void)hipStreamDestroy(cs_);
-    }
-    static bool enabled() {
-        const char* e = std::getenv("SPC5_CG_GRAPH");
-        return !(e && e[0] == '0');
-    }
-    // Runs fn(stream): recorded on the first call, replayed afterwards;
-    // without graphs, fn runs on s every time.
-    template <class F>
-    int run(hipStream_t s, F&& fn) {
-        if (!enabled()) return fn(s);
-        if (!exec_) {
-            SPC5_HIP_TRY(hipStreamCreateWithFlags(&cs_, hipStreamNonBlocking));
-            SPC5_HIP_TRY(hipStreamBeginCapture(cs_, hipStreamCaptureModeThreadLocal));
-            const int rc = fn(cs_);
-            hipGraph_t g = nullptr;
-            const hipError_t err = hipStreamEndCapture(cs_, &g);
-            if (rc) {
-                if (g) (void)hipGraphDestroy(g);
-                return rc;
-            }
-            SPC5_HIP_TRY(err);
-            graph_ = g;
-            SPC5_HIP_TRY(hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0));
-        }
-        SPC5_HIP_TRY(hipGraphLaunch(exec_, s));
-        return SPC5_HIP_OK;
-    }
-
-  private:
-    hipStream_t cs_ = nullptr;
-    hipGraph_t graph_ = nullptr;
-    hipGraphExec_t exec_ = nullptr;
-};
-
 unsigned vec_grid(int64_t n) {
     int64_t g = (n + kVecThreads - 1) / kVecThreads;
     if (g > kMaxVecGroups) g = kMaxVecGroups;
@@ -537,8 +492,7 @@ class HostScalars {
 
 // CG iterations on A from a given state: x, r, p (type X), r.r in
 // sc->rr[it & 1]; stops when r.r <= stop2 (read every `check` iterations)
-// or after maxit iterations in total.  it and hrr are updated.  Full chunks
-// start at an even iteration and are replayed from a hipGraph.
+// or after maxit iterations in total.  it and hrr are updated.
 template <class X>
 int cg_run(const spc5_hip_mat& A, X* x, X* r, X* p, X* q, CgScalars* sc, double* part, const HostScalars& host,
            int64_t n, int check, int maxit, double stop2, int& it, double& hrr, hipStream_t s) {
@@ -557,23 +511,11 @@ int cg_run(const spc5_hip_mat& A, X* x, X* r, X* p, X* q, CgScalars* sc, double*
         SPC5_HIP_TRY(hipGetLastError());
         return SPC5_HIP_OK;
     };
-    ChunkGraph chunk_graph;  // `check` iterations from an even one (parity returns to 0)
     int rc;
     while (hrr > stop2 && it < maxit) {
         const int chunk = (maxit - it) < check ? (maxit - it) : check;
-        if (chunk == check && check % 2 == 0 && it % 2 == 0) {
-            rc = chunk_graph.run(s, [&](hipStream_t t) -> int {
-                for (int c = 0; c < check; ++c) {
-                    const int e = iteration(t, c & 1, c + 1 == check);
-                    if (e) return e;
-                }
-                return SPC5_HIP_OK;
-            });
-            if (rc) return rc;
-        } else {
-            for (int c = 0; c < chunk; ++c)
-                if ((rc = iteration(s, (it + c) & 1, c + 1 == chunk))) return rc;
-        }
+        for (int c = 0; c < chunk; ++c)
+            if ((rc = iteration(s, (it + c) & 1, c + 1 == chunk))) return rc;
         it += chunk;
         if ((rc = host.read(0, &hrr, s))) return rc;
         if (!std::isfinite(hrr)) break;
@@ -750,22 +692,10 @@ int mixed_cg_impl(const spc5_hip_mat& A64, const spc5_hip_mat& Alo, const double
         SPC5_HIP_TRY(hipGetLastError());
         return SPC5_HIP_OK;
     };
-    ChunkGraph chunk_graph;  // `check` iterations, the last without its p update
     while (rr_true > stop2 && it < maxit && std::isfinite(rr_true)) {
         const int chunk = std::min(check, maxit - it);
-        if (chunk == check) {
-            rc = chunk_graph.run(s, [&](hipStream_t t) -> int {
-                for (int c = 0; c < check; ++c) {
-                    const int e = iteration(t, c & 1, c + 1 == check);
-                    if (e) return e;
-                }
-                return SPC5_HIP_OK;
-            });
-            if (rc) return rc;
-        } else {
-            for (int c = 0; c < chunk; ++c)
-                if ((rc = iteration(s, (it + c) & 1, c + 1 == chunk))) return rc;
-        }
+        for (int c = 0; c < chunk; ++c)
+            if ((rc = iteration(s, (it + c) & 1, c + 1 == chunk))) return rc;
         const int par = (it + chunk - 1) & 1;  // parity of the chunk's last iteration
         it += chunk;
         double rr_it = 0.0;
