@@ -513,12 +513,18 @@ int build_plan(spc5_hip_mat& m, hipStream_t s) {
 // the value-order tile costs about three times as many instructions per value
 // but gathers x with fewer distinct lines per request.  So the line is drawn
 // on `scatter`, the distinct 128-byte lines of x per block among 64 blocks in a
-// row: stencils, banded matrices and Laplacians have 0.04 .. 0.41, the
-// clustered matrix 0.52 .. 0.97 (value-order / lane-block, us):
+// row: stencils, narrow bands and Laplacians have 0.04 .. 0.41, bands wider
+// than 64 blocks 0.5 .. 0.64 (every block its own part of a line or two, read
+// once), the clustered matrix from 60,000 rows on 0.68 .. 0.97 (value-order /
+// lane-block, us):
 //   27-point stencil 128^3, scatter 0.2: float beta(2,16) 101 / 66, bfloat16
 //     beta(2,8) 95 / 53, double beta(2,8) 121 / 108
 //   banded 100,000 rows, half-width 130, scatter 0.14 .. 0.27: float beta(4,16)
 //     29 / 19, double beta(4,8) 28 / 21
+//   banded 60,000 rows, half-width 256 and 1,000, scatter 0.50 .. 0.64: double
+//     beta(4,8) 32 / 26 and 98 / 68, beta(1,8) 34 / 31 and 106 / 97, float
+//     beta(4,16) at 1,000 106 / 54
+//   clustered 40,000 rows, scatter 0.61 .. 0.63: 9 / 9 at every r
 //   clustered 1 M rows, scatter 0.8 .. 0.97: double beta(1,8) 88 / 102, float
 //     beta(2,16) 61 / 66, but bfloat16 beta(2,8) 66 / 55
 //   clustered 60,000 rows (x and matrix in the L2s): double beta(2,8) 10.5 /
@@ -529,7 +535,7 @@ bool lane_block_wins(const spc5_hip_mat& m) {
     if ((uint64_t)m.ncols * 8 > 0xffffffffull || m.ncols < 16) return false;  // 32-bit x offsets, a whole window
     const bool f64 = m.value_type == SPC5_HIP_F64;
     if (f64 && m.r == 8) return false;
-    if (m.scatter < 0.48) return true;
+    if (m.scatter < 0.65) return true;
     const bool small = m.nnz < (4 << 20);
     if (f64) return m.r <= 2 && small;
     if (m.value_type == SPC5_HIP_F32 && m.vs == 16) return m.r <= 4 && small;
