@@ -27,11 +27,16 @@ struct BatchEntry {
     const void* val;
     const void* x;
     void* y;
-    const int4* tiles;
     int64_t nrows;
     int64_t ncols;
     int r;
     int lanes;  // 1: lane-block tile
+};
+
+// One tile of the batch: its matrix, where it starts and where it ends
+// ({block-row, block, value, matrix} and the next tile's).
+struct alignas(32) BatchTile {
+    int4 first, last;
 };
 
 struct spc5_hip_batch {
@@ -44,12 +49,10 @@ struct spc5_hip_batch {
     int lanes = 0;          // only_r, and every matrix runs the lane-block tile
     int sorted = 0;         // only_r is 2 or 4, not all lane-block, and every matrix has row sorting on
     DeviceBuffer entries;   // BatchEntry[nmats]
-    DeviceBuffer tile_mat;  // int32[ntiles]: matrix of each tile
-    DeviceBuffer tile_loc;  // int32[ntiles]: tile index inside its matrix
+    // BatchTile[ntiles], copied: a matrix's plan may be rebuilt later
+    // (SPC5_HIP_OPT_TILE_VALUES).
+    DeviceBuffer tiles;
     std::vector<spc5_hip_mat_t> mats;  // borrowed handles
-    // The tile lists the batch was built from: a matrix's plan may be
-    // rebuilt later (SPC5_HIP_OPT_TILE_VALUES); the batch keeps its own.
-    std::vector<std::shared_ptr<DeviceBuffer>> tiles_kept;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipStream_t capture_stream = nullptr;
@@ -94,19 +97,25 @@ constexpr int batch_waves_per_eu(int only_r, bool wide_x, int value_bytes, bool 
 
 // The batch loop over tiles: tile t of the list runs body(matrix entry,
 // tile bounds) on its wave.
+// The record of a wave's next tile is loaded while the current one runs, so a
+// tile starts with its matrix's entry (shared by its neighbours) and not with
+// the chain matrix index -> matrix -> tile list -> bounds (96 banded matrices,
+// double beta(4,8), tiles of 500 values: 715 -> 698 us).
 template <class Body>
-__device__ __forceinline__ void batch_tiles(const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat,
-                                            const int* __restrict__ tile_loc, int64_t ntiles, Body&& body) {
+__device__ __forceinline__ void batch_tiles(const BatchEntry* __restrict__ mats, const BatchTile* __restrict__ tiles,
+                                            int64_t ntiles, Body&& body) {
     const int w = threadIdx.x >> 6;
     const int64_t stride = (int64_t)gridDim.x * kWavesPerGroup;
     // The tile index is the same on every lane (it comes from the wave index,
     // which the compiler cannot tell is uniform): read it as a scalar, so the
-    // matrix descriptor is loaded into scalar registers.
+    // records are loaded into scalar registers.
     const int64_t t0 = (int64_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerGroup + w));
+    if (t0 >= ntiles) return;
+    BatchTile next = tiles[t0];
     for (int64_t t = t0; t < ntiles; t += stride) {
-        const BatchEntry& m = mats[tile_mat[t]];
-        const int lt = tile_loc[t];
-        body(m, m.tiles[lt], m.tiles[lt + 1]);
+        const BatchTile cur = next;
+        next = tiles[t + stride < ntiles ? t + stride : t];
+        body(mats[cur.first.w], cur.first, cur.last);
         wave_sync();
     }
 }
@@ -115,8 +124,7 @@ __device__ __forceinline__ void batch_tiles(const BatchEntry* __restrict__ mats,
 // tile keep it.
 template <class V, class X, class ACC, int VS, int MB, int R>
 __global__ __launch_bounds__(kWavesPerGroup * 64, batch_waves_per_eu(R, sizeof(X) > sizeof(ACC), sizeof(V), true)) void
-k_spmv_batch_sorted(const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat,
-                    const int* __restrict__ tile_loc, int64_t ntiles) {
+k_spmv_batch_sorted(const BatchEntry* __restrict__ mats, const BatchTile* __restrict__ tiles, int64_t ntiles) {
     static_assert(R == 2 || R == 4, "row-sorted tiles exist for r = 2 and 4");
     __shared__ union {
         TileSmem<ACC, R, expand_cap<V>(), true> order;
@@ -124,7 +132,7 @@ k_spmv_batch_sorted(const BatchEntry* __restrict__ mats, const int* __restrict__
     } sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const Epilogue ep;
-    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
+    batch_tiles(mats, tiles, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
         if (m.lanes)
             spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w].lanes, m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
                                                  reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first,
@@ -139,12 +147,11 @@ k_spmv_batch_sorted(const BatchEntry* __restrict__ mats, const int* __restrict__
 // Every matrix has r = R and runs the lane-block tile.
 template <class V, class X, class ACC, int VS, int MB, int R>
 __global__ __launch_bounds__(kWavesPerGroup * 64, lane_waves_per_eu(R, VS, sizeof(X)) - 1) void k_spmv_batch_lanes(
-    const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat, const int* __restrict__ tile_loc,
-    int64_t ntiles) {
+    const BatchEntry* __restrict__ mats, const BatchTile* __restrict__ tiles, int64_t ntiles) {
     __shared__ LaneSmem<V, ACC, R, MB> sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const Epilogue ep;
-    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
+    batch_tiles(mats, tiles, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
         spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w], m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
                                              reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first, last,
                                              m.nrows, m.ncols, ep);
@@ -154,12 +161,11 @@ __global__ __launch_bounds__(kWavesPerGroup * 64, lane_waves_per_eu(R, VS, sizeo
 // Every matrix has r = R and runs the value-order tile.
 template <class V, class X, class ACC, int VS, int MB, int R>
 __global__ __launch_bounds__(kWavesPerGroup * 64, batch_waves_per_eu(R, sizeof(X) > sizeof(ACC), sizeof(V))) void
-k_spmv_batch(const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat, const int* __restrict__ tile_loc,
-             int64_t ntiles) {
+k_spmv_batch(const BatchEntry* __restrict__ mats, const BatchTile* __restrict__ tiles, int64_t ntiles) {
     __shared__ TileSmem<ACC, R, expand_cap<V>()> sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const Epilogue ep;
-    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
+    batch_tiles(mats, tiles, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
         spmv_tile<V, X, ACC, R, VS, MB>(sm[w], m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
                                         reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first, last,
                                         m.nrows, m.ncols, ep);
@@ -169,12 +175,11 @@ k_spmv_batch(const BatchEntry* __restrict__ mats, const int* __restrict__ tile_m
 // Any r and either tile per matrix.
 template <class V, class X, class ACC, int VS, int MB>
 __global__ __launch_bounds__(kWavesPerGroup * 64, batch_waves_per_eu(0, sizeof(X) > sizeof(ACC), sizeof(V))) void
-k_spmv_batch_mixed(const BatchEntry* __restrict__ mats, const int* __restrict__ tile_mat,
-                   const int* __restrict__ tile_loc, int64_t ntiles) {
+k_spmv_batch_mixed(const BatchEntry* __restrict__ mats, const BatchTile* __restrict__ tiles, int64_t ntiles) {
     __shared__ MixedSmem<V, ACC, MB> sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const Epilogue ep;
-    batch_tiles(mats, tile_mat, tile_loc, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
+    batch_tiles(mats, tiles, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
         const V* val = reinterpret_cast<const V*>(m.val);
         const X* x = reinterpret_cast<const X*>(m.x);
         X* y = reinterpret_cast<X*>(m.y);
@@ -191,11 +196,20 @@ k_spmv_batch_mixed(const BatchEntry* __restrict__ mats, const int* __restrict__ 
     });
 }
 
+// The tile records of one matrix.
+__global__ __launch_bounds__(256) void k_batch_records(const int4* __restrict__ tiles, int64_t ntiles, int mat,
+                                                       BatchTile* __restrict__ out) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= ntiles) return;
+    const int4 a = tiles[t];
+    out[t] = BatchTile{make_int4(a.x, a.y, a.z, mat), tiles[t + 1]};
+}
+
 template <class Kernel>
 void launch_batch_kernel(const spc5_hip_batch& b, Kernel k, hipStream_t s) {
     const unsigned groups = (unsigned)((b.waves + kWavesPerGroup - 1) / kWavesPerGroup);
     hipLaunchKernelGGL(k, dim3(groups), dim3(kWavesPerGroup * 64), 0, s, b.entries.as<const BatchEntry>(),
-                       b.tile_mat.as<const int>(), b.tile_loc.as<const int>(), b.ntiles);
+                       b.tiles.as<const BatchTile>(), b.ntiles);
 }
 
 template <class V, class X, class ACC, int VS, int MB>
@@ -253,7 +267,6 @@ int spc5_hip_batch_create(int nmats, const spc5_hip_mat_t* mats, const void* con
     b->vs = mats[0]->vs;
     b->nmats = nmats;
     std::vector<BatchEntry> ent((size_t)nmats);
-    std::vector<int> tmat, tloc;
     for (int i = 0; i < nmats; ++i) {
         const spc5_hip_mat* m = mats[i];
         SPC5_CHECK_ARG(m != nullptr, "null matrix handle");
@@ -265,19 +278,13 @@ int spc5_hip_batch_create(int nmats, const spc5_hip_mat_t* mats, const void* con
         e.val = m->values;
         e.x = d_x[i];
         e.y = d_y[i];
-        e.tiles = m->plan.ntiles ? m->plan.tiles->as<const int4>() : nullptr;
-        if (m->plan.ntiles) b->tiles_kept.push_back(m->plan.tiles);
         e.nrows = m->nrows;
         e.ncols = m->ncols;
         e.r = m->r;
         e.lanes = m->lane_body;
-        for (int64_t t = 0; t < m->plan.ntiles; ++t) {
-            tmat.push_back(i);
-            tloc.push_back((int)t);
-        }
         b->mats.push_back(const_cast<spc5_hip_mat*>(m));
     }
-    b->ntiles = (int64_t)tmat.size();
+    for (const spc5_hip_mat* m : b->mats) b->ntiles += m->plan.ntiles;
     SPC5_CHECK_ARG(b->ntiles <= 0x7ffffff0, "batch: more than 2^31 - 16 tiles");
     int dev = 0, ncu = 256;
     SPC5_HIP_TRY(hipGetDevice(&dev));
@@ -297,13 +304,18 @@ int spc5_hip_batch_create(int nmats, const spc5_hip_mat_t* mats, const void* con
     if (wv > b->ntiles) wv = std::max<int64_t>(b->ntiles, 1);
     b->waves = (int)wv;
     SPC5_HIP_TRY(b->entries.alloc(sizeof(BatchEntry) * (size_t)nmats));
-    SPC5_HIP_TRY(b->tile_mat.alloc(sizeof(int) * (size_t)std::max<int64_t>(b->ntiles, 1)));
-    SPC5_HIP_TRY(b->tile_loc.alloc(sizeof(int) * (size_t)std::max<int64_t>(b->ntiles, 1)));
+    SPC5_HIP_TRY(b->tiles.alloc(sizeof(BatchTile) * (size_t)std::max<int64_t>(b->ntiles, 1)));
     SPC5_HIP_TRY(hipMemcpy(b->entries.p, ent.data(), sizeof(BatchEntry) * (size_t)nmats, hipMemcpyHostToDevice));
-    if (b->ntiles) {
-        SPC5_HIP_TRY(hipMemcpy(b->tile_mat.p, tmat.data(), sizeof(int) * tmat.size(), hipMemcpyHostToDevice));
-        SPC5_HIP_TRY(hipMemcpy(b->tile_loc.p, tloc.data(), sizeof(int) * tloc.size(), hipMemcpyHostToDevice));
+    int64_t at = 0;
+    for (int i = 0; i < nmats; ++i) {
+        const Plan& p = mats[i]->plan;
+        if (p.ntiles)
+            hipLaunchKernelGGL(k_batch_records, dim3((unsigned)((p.ntiles + 255) / 256)), dim3(256), 0, nullptr,
+                               p.tiles->as<const int4>(), p.ntiles, i, b->tiles.as<BatchTile>() + at);
+        at += p.ntiles;
     }
+    SPC5_HIP_TRY(hipGetLastError());
+    SPC5_HIP_TRY(hipStreamSynchronize(nullptr));
     // Capture the persistent launch once; products replay the graph.
     SPC5_HIP_TRY(hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking));
     if (b->ntiles) {
