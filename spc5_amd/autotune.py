@@ -297,8 +297,8 @@ def tune_batch_tiles(mats, make_batch, candidates=(0, 2048, 4096, 8192, 16384), 
 
 
 def tune_batch_waves(make_batch, fractions=(0.5, 1.0, 2.0, 4.0), reps=5):
-    """Fastest persistent wave count of a batch: `make_batch(waves)` builds
-    a batch.Batch (waves = 0 is the kernel's resident count); candidates are
+    """Fastest wave count of a batch: `make_batch(waves)` builds
+    a batch.Batch (waves = 0 is the default count); candidates are
     fractions of that count and one wave per tile (the tiles then dealt out
     by the hardware's dispatcher, which measured fastest on 2,000 banded
     matrices with large tiles).  Returns (waves, {waves: seconds}); the

@@ -15,8 +15,8 @@ ONE_WAVE_PER_TILE = 2**31 - 1
 class Batch:
     """y_i += A_i x_i for all i in one launch.  Matrices may use different r
     but share value type and VS; the x_i / y_i tensors are kept alive here.
-    `waves`: persistent waves walking the tile list (0: the kernel's resident
-    count; ONE_WAVE_PER_TILE: one wave per tile)."""
+    `waves`: waves walking the tile list (0: 32 for every wave that is resident
+    at once; ONE_WAVE_PER_TILE: one wave per tile)."""
 
     def __init__(self, mats: list[DeviceMatrix], xs, ys, waves: int = 0):
         if not mats or not (len(mats) == len(xs) == len(ys)):

@@ -1,9 +1,9 @@
-// batch.hip -- many independent beta(r,VS) matrices in one persistent,
+// batch.hip -- many independent beta(r,VS) matrices in one
 // hipGraph-captured launch (the batching form; no counterpart in the
 // reference).
 //
-// The tiles of every matrix form one list (matrix index + local tile index
-// per entry, built once at batch creation).  A persistent grid of
+// The tiles of every matrix form one list (matrix index and tile bounds
+// per entry, built once at batch creation).  A grid of
 // `waves` waves walks the list with a static stride; each tile runs the
 // same tile routine as the single-matrix kernel, with the matrix's own r
 // (chosen per matrix, e.g. by the autotuner) selected at run time.  When
@@ -96,8 +96,7 @@ constexpr int batch_waves_per_eu(int only_r, bool wide_x, int value_bytes, bool 
     spmv_lane_tile<V, X, ACC, RR, VS, MB>(SMEM, m.bptr, m.hdr, val, x, y, first, last, m.nrows, m.ncols, ep)
 
 // The batch loop over tiles: tile t of the list runs body(matrix entry,
-// tile bounds) on its wave.
-// The record of a wave's next tile is loaded while the current one runs, so a
+// tile bounds) on its wave.  The record of a wave's next tile is loaded while the current one runs, so a
 // tile starts with its matrix's entry (shared by its neighbours) and not with
 // the chain matrix index -> matrix -> tile list -> bounds (96 banded matrices,
 // double beta(4,8), tiles of 500 values: 715 -> 698 us).
@@ -232,7 +231,16 @@ void launch_batch(const spc5_hip_batch& b, hipStream_t s) {
     }
 }
 
-// Waves per SIMD the batch's kernel runs at (sizes the persistent grid).
+// Waves launched by default for every one that is resident at once: with the
+// resident ones alone the last wave to finish its share of uneven tiles sets
+// the time, and none starts a tile while another waits for its first loads.
+// 96 banded matrices (1,000 to 200,000 rows, half-widths 4 to 256), us at 1, 4,
+// 8, 16, 32 rounds and one wave per tile: double beta(4,8) 695, 642, 615, 606,
+// 606, 612; beta(8,8) 1038, 909, 860, 833, 827, 835; 4 matrices beta(4,8) 49.1,
+// 42.8, 42.6, 41.9, 41.5, 41.0.
+constexpr int kWaveRounds = 32;
+
+// Waves per SIMD the batch's kernel runs at (sizes the grid).
 int batch_kernel_waves(const spc5_hip_batch& b) {
     const int vb = (int)value_bytes(b.value_type);
     if (b.lanes) return lane_waves_per_eu(b.only_r, b.vs, vb == 8 ? 8 : 4) - 1;
@@ -300,7 +308,7 @@ int spc5_hip_batch_create(int nmats, const spc5_hip_mat_t* mats, const void* con
     b->lanes = b->only_r && all_lanes ? 1 : 0;
     b->sorted = (b->only_r == 2 || b->only_r == 4) && !b->lanes && all_sorted ? 1 : 0;
     if (b->only_r && !b->lanes && !b->sorted && any_lanes) b->only_r = 0;  // both tiles: the mixed kernel
-    int64_t wv = waves > 0 ? waves : (int64_t)ncu * 4 * batch_kernel_waves(*b);
+    int64_t wv = waves > 0 ? waves : (int64_t)ncu * 4 * batch_kernel_waves(*b) * kWaveRounds;
     if (wv > b->ntiles) wv = std::max<int64_t>(b->ntiles, 1);
     b->waves = (int)wv;
     SPC5_HIP_TRY(b->entries.alloc(sizeof(BatchEntry) * (size_t)nmats));
@@ -316,7 +324,7 @@ int spc5_hip_batch_create(int nmats, const spc5_hip_mat_t* mats, const void* con
     }
     SPC5_HIP_TRY(hipGetLastError());
     SPC5_HIP_TRY(hipStreamSynchronize(nullptr));
-    // Capture the persistent launch once; products replay the graph.
+    // Capture the launch once; products replay the graph.
     SPC5_HIP_TRY(hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking));
     if (b->ntiles) {
         SPC5_HIP_TRY(hipStreamBeginCapture(b->capture_stream, hipStreamCaptureModeThreadLocal));
