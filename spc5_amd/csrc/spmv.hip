@@ -167,7 +167,10 @@ __global__ __launch_bounds__(kWavesPerGroup * 64) void k_access_probe(
 // One wave per 64 block-rows: the lanes read
 // the group's headers in block order, coalesced, find each block's block-row
 // by a binary search of the 65 group pointers in LDS and add its popcount to
-// that block-row's LDS counter.
+// that block-row's LDS counter.  Bound by the latency of the header loads and
+// the searches, so each lane takes four blocks a round, loads first
+// (clustered 1 M rows, double beta(4,8): 33 -> 21 us; 96 banded matrices of 1,000
+// to 200,000 rows, 24.9 -> 11.2 us at the median).
 template <int R, int MB, int VS>
 __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__ bptr,
                                                          const unsigned char* __restrict__ hdr, int64_t nbr,
@@ -209,34 +212,47 @@ __global__ __launch_bounds__(256) void k_blockrow_values(const int* __restrict__
     // lines, err[2] the blocks.
     const bool sample = (blockIdx.x * 4u + (unsigned)w) % every == 0;
     bool bad = false;
-    for (int b = b0 + lane; b < bE; b += 64) {
-        const unsigned char* h = hdr + (int64_t)b * H;
-        const int cs = load_i32_unaligned(h);
-        unsigned long long mw[MW::kWords];
-        MW::load(h + 4, mw);
-        if (sample && b < b0 + 64) {
-            const unsigned line = (unsigned)(((uint64_t)(unsigned)cs * (unsigned)xbytes) >> 7);
+    constexpr int U = 4;
+    for (int bb = b0 + lane; bb - lane < bE; bb += 64 * U) {
+        int cs[U];
+        unsigned long long mw[U][MW::kWords];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int b = bb + 64 * u < bE ? bb + 64 * u : bE - 1;
+            const unsigned char* h = hdr + (int64_t)b * H;
+            cs[u] = load_i32_unaligned(h);
+            MW::load(h + 4, mw[u]);
+        }
+        if (sample && bb < b0 + 64 && bb < bE) {
+            const unsigned line = (unsigned)(((uint64_t)(unsigned)cs[0] * (unsigned)xbytes) >> 7);
             const unsigned h = (line * 0x9e3779b1u) >> 21;
             atomicOr(&sline[w][h >> 5], 1u << (h & 31u));
         }
-        int c = 0;
-        unsigned rowor = 0;
-        for (int k = 0; k < MW::kWords; ++k) {
-            c += __popcll(mw[k]);
-            for (int q = 0; q < 64 / VS; ++q) rowor |= (unsigned)((mw[k] >> (q * VS)) & ((1ull << VS) - 1ull));
+        // the blocks' block-rows: the largest i with sp[i] <= b (sp[0] <= b < sp[64])
+        int lo[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) lo[u] = 0;
+#pragma unroll
+        for (int step = 32; step >= 1; step >>= 1) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) lo[u] += sp[lo[u] + step] <= bb + 64 * u ? step : 0;
         }
-        if (rowor != 0) {
-            const int hi = 31 - __builtin_clz(rowor);
-            bad |= cs < 0 || (int64_t)cs + hi >= ncols;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (bb + 64 * u >= bE) continue;
+            int c = 0;
+            unsigned rowor = 0;
+            for (int k = 0; k < MW::kWords; ++k) {
+                c += __popcll(mw[u][k]);
+                for (int q = 0; q < 64 / VS; ++q)
+                    rowor |= (unsigned)((mw[u][k] >> (q * VS)) & ((1ull << VS) - 1ull));
+            }
+            if (rowor != 0) {
+                const int hi = 31 - __builtin_clz(rowor);
+                bad |= cs[u] < 0 || (int64_t)cs[u] + hi >= ncols;
+            }
+            atomicAdd(&sc[lo[u]], c);
         }
-        // the block's block-row: the largest i with sp[i] <= b (sp[0] <= b < sp[64])
-        int lo = 0, up = 64;
-        while (up - lo > 1) {
-            const int mid = (lo + up) >> 1;
-            if (sp[mid] <= b) lo = mid;
-            else up = mid;
-        }
-        atomicAdd(&sc[lo], c);
     }
     wave_sync();
     if (br0 + lane < nbr) cnt_out[br0 + lane] = sc[lane];
