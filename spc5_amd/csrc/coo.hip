@@ -86,34 +86,144 @@ __global__ void k_coo_gather(const unsigned long long* __restrict__ keys, const 
 // pairs bound it, so rows of more than kShortRow entries go to the radix sort
 // (coo_short_rows decides on the mean; a longer row found on the way sends the
 // whole matrix there).  1.25 M entries in 50 K rows: 462 us with the radix
-// sort, 199 us; 3.2 M in 100 K rows 1,467 and 385 us.
+// sort, 155 us.
 constexpr int kShortRow = 1024;
 
 // Counts per row (rowptr, cleared before) and every entry's place in its row.
-__global__ __launch_bounds__(256) void k_coo_count(const int* __restrict__ ri, const int* __restrict__ cj, int64_t nnz,
-                                                   int64_t nrows, int64_t ncols, int* __restrict__ count,
-                                                   int* __restrict__ place, int* __restrict__ err) {
+// Counters in memory take an atomic per entry, 22 G/s at best and a third of it
+// where neighbouring entries share a row; for matrices of many entries see
+// k_coo_count_ranges.
+__global__ __launch_bounds__(256) void k_coo_count(const int* __restrict__ ri, int64_t nnz, int64_t nrows,
+                                                   int* __restrict__ count, int* __restrict__ place,
+                                                   int* __restrict__ err) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nnz) return;
-    const int r = ri[t], c = cj[t];
-    if (r < 0 || (int64_t)r >= nrows || c < 0 || (int64_t)c >= ncols) {
+    const int r = ri[t];
+    if (r < 0 || (int64_t)r >= nrows) {
         atomicOr(err, 1);
         place[t] = -1;
         return;
     }
-    place[t] = atomicAdd(&count[r], 1);
+    const int p = atomicAdd(&count[r], 1);
+    if (p >= kShortRow) atomicOr(err, 4);
+    place[t] = p;
 }
 
-// keys[row pointer + place] = (column, input position).
+// The counters in LDS: workgroup (c, g) takes chunk c of the entries and counts
+// those whose row lies in range g of kRangeRows rows, 16 bits a counter; a place
+// is then one in its chunk, and k_coo_bases turns the chunks' counts into each
+// chunk's first place per row.  Every range reads all rows again and the counts
+// pass through memory, so counters in memory stay for few entries (112 K: the
+// same 80 us) and for more than kMaxRanges ranges (at 31 ranges, 5 M shuffled
+// entries, the same 565 us).  Whole call, shuffled and in order: 260 K entries in
+// 20 K rows 98 / 90 -> 91 / 84 us, 1.25 M in 50 K 184 / 186 -> 155 / 114, 9.5 M in
+// 300 K 1037 / 1080 -> 916 / 513.
+constexpr int kRangeRows = 32768;
+constexpr int kMaxRanges = 32;
+constexpr int kRangeThreads = 1024;
+constexpr int64_t kChunkEntries = 16384;
+constexpr int64_t kRangeEntries = 1 << 17;
+
+struct CooChunks {
+    int64_t entries = 0;  // per chunk, a multiple of 256 (0: counters in memory)
+    int chunks = 0, ranges = 0;
+    int64_t words = 0;    // of two counters, per chunk
+    size_t bytes() const { return sizeof(unsigned) * (size_t)words * (size_t)chunks; }
+};
+CooChunks coo_chunks(int64_t nrows, int64_t nnz) {
+    CooChunks k;
+    if (nnz < kRangeEntries || nrows > (int64_t)kMaxRanges * kRangeRows) return k;
+    k.ranges = (int)((nrows + kRangeRows - 1) / kRangeRows);
+    const int64_t most = 512 / k.ranges;  // two workgroups per CU, and at most 32 MiB of counts
+    int64_t n = (nnz + kChunkEntries - 1) / kChunkEntries;
+    if (n > most) n = most;
+    k.entries = ((nnz + n - 1) / n + 255) / 256 * 256;
+    k.chunks = (int)((nnz + k.entries - 1) / k.entries);
+    k.words = (nrows + 1) / 2;
+    return k;
+}
+
+__global__ __launch_bounds__(kRangeThreads) void k_coo_count_ranges(const int* __restrict__ ri, int64_t nnz,
+                                                                    int64_t nrows, int64_t entries, int64_t words,
+                                                                    unsigned* __restrict__ counts,
+                                                                    int* __restrict__ place, int* __restrict__ err) {
+    constexpr int U = 4;
+    __shared__ unsigned h[kRangeRows / 2];
+    for (int i = threadIdx.x; i < kRangeRows / 2; i += kRangeThreads) h[i] = 0u;
+    __syncthreads();
+    const int64_t b = (int64_t)blockIdx.x * entries;
+    const int64_t e = b + entries < nnz ? b + entries : nnz;
+    const int64_t row0 = (int64_t)blockIdx.y * kRangeRows;
+    int bad = 0;
+    for (int64_t t0 = b + threadIdx.x; t0 < e; t0 += U * kRangeThreads) {
+        int r[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) r[u] = ri[t0 + u * kRangeThreads < e ? t0 + u * kRangeThreads : e - 1];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t t = t0 + u * kRangeThreads;
+            if (t >= e) continue;
+            if (r[u] < 0 || (int64_t)r[u] >= nrows) {
+                bad |= 1;
+            } else if (r[u] >= row0 && r[u] < row0 + kRangeRows) {
+                const unsigned l = (unsigned)(r[u] - row0), sh = 16u * (l & 1u);
+                const int p = (int)((atomicAdd(&h[l >> 1], 1u << sh) >> sh) & 0xffffu);
+                if (p >= kShortRow) bad |= 4;
+                place[t] = p;
+            }
+        }
+    }
+    if (bad) atomicOr(err, bad);
+    __syncthreads();
+    const int64_t w0 = row0 / 2;
+    unsigned* out = counts + (int64_t)blockIdx.x * words + w0;
+    for (int i = threadIdx.x; i < kRangeRows / 2 && w0 + i < words; i += kRangeThreads) out[i] = h[i];
+}
+
+// Counts of the chunks -> each chunk's first place in every row (in place), and
+// the rows' counts; rowptr[nrows] = 0.
+__global__ __launch_bounds__(256) void k_coo_bases(unsigned* __restrict__ counts, int64_t words, int chunks,
+                                                   int64_t nrows, int* __restrict__ rowptr, int* __restrict__ err) {
+    constexpr int U = 8;
+    const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (w >= words) return;
+    unsigned lo = 0, hi = 0;
+    for (int c0 = 0; c0 < chunks; c0 += U) {
+        unsigned n[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) n[u] = counts[(int64_t)(c0 + u < chunks ? c0 + u : chunks - 1) * words + w];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (c0 + u >= chunks) continue;
+            counts[(int64_t)(c0 + u) * words + w] = (lo & 0xffffu) | (hi << 16);
+            lo += n[u] & 0xffffu;
+            hi += n[u] >> 16;
+        }
+    }
+    if (lo > (unsigned)kShortRow || hi > (unsigned)kShortRow) atomicOr(err, 4);
+    rowptr[2 * w] = (int)lo;
+    if (2 * w + 1 < nrows) rowptr[2 * w + 1] = (int)hi;
+    if (w == 0) rowptr[nrows] = 0;
+}
+
+// keys[row pointer + place] = (column, input position).  Does nothing after an
+// error (the counts may then not add up).
 __global__ __launch_bounds__(256) void k_coo_place(const int* __restrict__ ri, const int* __restrict__ cj, int64_t nnz,
-                                                   const int* __restrict__ rowptr, const int* __restrict__ place,
-                                                   unsigned long long* __restrict__ keys, int* __restrict__ err) {
+                                                   int64_t ncols, const int* __restrict__ rowptr,
+                                                   const int* __restrict__ place, const unsigned* __restrict__ bases,
+                                                   int64_t words, int64_t entries,
+                                                   unsigned long long* __restrict__ keys,
+                                                   const int* __restrict__ counted, int* __restrict__ err) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nnz) return;
-    const int p = place[t];
-    if (p < 0) return;
-    if (p >= kShortRow) atomicOr(err, 4);
-    keys[(int64_t)rowptr[ri[t]] + p] = ((unsigned long long)(unsigned)cj[t] << 32) | (unsigned)t;
+    if (t >= nnz || *counted != 0) return;
+    const int r = ri[t], c = cj[t];
+    int p = place[t];
+    if (bases) {
+        const int64_t chunk = (int64_t)blockIdx.x * 256 / entries;  // entries is a multiple of 256
+        p += (int)((bases[chunk * words + (r >> 1)] >> (16 * (r & 1))) & 0xffffu);
+    }
+    if (c < 0 || (int64_t)c >= ncols) atomicOr(err, 1);
+    keys[(int64_t)rowptr[r] + p] = ((unsigned long long)(unsigned)c << 32) | (unsigned)t;
 }
 
 // Every entry to its rank in its row.  Does nothing after an error or a long row.
@@ -124,7 +234,7 @@ __global__ __launch_bounds__(256) void k_coo_rank(const int* __restrict__ ri, in
                                                   const T* __restrict__ v, const int* __restrict__ err,
                                                   int* __restrict__ col, T* __restrict__ val) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nnz || *err != 0) return;
+    if (e >= nnz || (err[0] | err[1]) != 0) return;
     const unsigned long long mine = keys[e];
     const unsigned t = (unsigned)mine;
     const int r = ri[t];
@@ -146,10 +256,11 @@ bool coo_short_rows(int64_t nrows, int64_t nnz) { return nnz > 0 && nnz / 96 <= 
 
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
-// Workspace of the short-row path: flags, scan partials, places, keys.
+// Workspace of the short-row path: flags (of the counts, of the columns), scan
+// partials, places, the chunks' counts, keys.
 size_t coo_short_bytes(int64_t nrows, int64_t nnz) {
     return 256 + align256(sizeof(int) * (size_t)scan_partials_needed(nrows + 1)) + align256(sizeof(int) * (size_t)nnz) +
-           sizeof(unsigned long long) * (size_t)nnz;
+           sizeof(unsigned long long) * (size_t)nnz + align256(coo_chunks(nrows, nnz).bytes());
 }
 
 unsigned grid_of(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -164,15 +275,25 @@ int coo_short(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, const 
     int* partials = reinterpret_cast<int*>(w + 256);
     w += 256 + align256(sizeof(int) * (size_t)scan_partials_needed(nrows + 1));
     int* place = reinterpret_cast<int*>(w);
-    unsigned long long* keys = reinterpret_cast<unsigned long long*>(w + align256(sizeof(int) * (size_t)nnz));
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, s, err, (int64_t)1, 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_of(nrows + 1)), dim3(256), 0, s, d_rowptr, nrows + 1, 0);
-    hipLaunchKernelGGL(k_coo_count, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, d_j, nnz, nrows, ncols, d_rowptr, place,
-                       err);
+    w += align256(sizeof(int) * (size_t)nnz);
+    const CooChunks k = coo_chunks(nrows, nnz);
+    unsigned* counts = k.entries ? reinterpret_cast<unsigned*>(w) : nullptr;
+    unsigned long long* keys = reinterpret_cast<unsigned long long*>(w + align256(k.bytes()));
+    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, s, err, (int64_t)2, 0);
+    if (k.entries) {
+        hipLaunchKernelGGL(k_coo_count_ranges, dim3((unsigned)k.chunks, (unsigned)k.ranges), dim3(kRangeThreads), 0, s,
+                           d_i, nnz, nrows, k.entries, k.words, counts, place, err);
+        hipLaunchKernelGGL(k_coo_bases, dim3(grid_of(k.words)), dim3(256), 0, s, counts, k.words, k.chunks, nrows,
+                           d_rowptr, err);
+    } else {
+        hipLaunchKernelGGL(k_fill_i32, dim3(grid_of(nrows + 1)), dim3(256), 0, s, d_rowptr, nrows + 1, 0);
+        hipLaunchKernelGGL(k_coo_count, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, nnz, nrows, d_rowptr, place, err);
+    }
     SPC5_HIP_TRY(hipGetLastError());
     const int rc = scan_exclusive_i32_ws(d_rowptr, nrows + 1, nullptr, partials, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_coo_place, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, d_j, nnz, d_rowptr, place, keys, err);
+    hipLaunchKernelGGL(k_coo_place, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, d_j, nnz, ncols, d_rowptr, place,
+                       (const unsigned*)counts, k.words, k.entries, keys, (const int*)err, err + 1);
     if (value_bytes == 8)
         hipLaunchKernelGGL(k_coo_rank<double>, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, nnz, d_rowptr, keys,
                            reinterpret_cast<const double*>(d_v), err, d_col, reinterpret_cast<double*>(d_val));
@@ -180,8 +301,10 @@ int coo_short(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, const 
         hipLaunchKernelGGL(k_coo_rank<float>, dim3(grid_of(nnz)), dim3(256), 0, s, d_i, nnz, d_rowptr, keys,
                            reinterpret_cast<const float*>(d_v), err, d_col, reinterpret_cast<float*>(d_val));
     SPC5_HIP_TRY(hipGetLastError());
-    SPC5_HIP_TRY(hipMemcpyAsync(flags, err, sizeof(int), hipMemcpyDeviceToHost, s));
+    int h[2] = {0, 0};
+    SPC5_HIP_TRY(hipMemcpyAsync(h, err, sizeof(h), hipMemcpyDeviceToHost, s));
     SPC5_HIP_TRY(hipStreamSynchronize(s));
+    *flags = h[0] | h[1];
     return SPC5_HIP_OK;
 }
 
