@@ -30,7 +30,7 @@ struct BatchEntry {
     int64_t nrows;
     int64_t ncols;
     int r;
-    int lanes;  // 1: lane-block tile
+    int lanes;  // 1 + stage level: lane-block tile
 };
 
 // One tile of the batch: its matrix, where it starts and where it ends
@@ -46,7 +46,7 @@ struct spc5_hip_batch {
     int64_t ntiles = 0;
     int waves = 0;
     int only_r = 0;         // the r shared by every matrix, 0 if they differ
-    int lanes = 0;          // only_r, and every matrix runs the lane-block tile
+    int lanes = 0;          // only_r, and every matrix runs the lane-block tile: 1 + their highest stage level
     int sorted = 0;         // only_r is 2 or 4, not all lane-block, and every matrix has row sorting on
     DeviceBuffer entries;   // BatchEntry[nmats]
     // BatchTile[ntiles], copied: a matrix's plan may be rebuilt later
@@ -73,14 +73,20 @@ union BatchSmem {
     TileSmem<ACC, 4, expand_cap<V>()> r4;
     TileSmem<ACC, 8, expand_cap<V>()> r8;
 };
+// The largest stage of the values (the matrices' own levels bound its use).
+template <class V, int R, int MB>
+constexpr int max_stage() {
+    return lane_stage_bytes(sizeof(V), R, 8 * MB, lane_levels(sizeof(V), R, 8 * MB) - 1);
+}
+
 // Any r and either tile.
 template <class V, class ACC, int MB>
 union MixedSmem {
     BatchSmem<V, ACC> order;
-    LaneSmem<V, ACC, 1, MB> l1;
-    LaneSmem<V, ACC, 2, MB> l2;
-    LaneSmem<V, ACC, 4, MB> l4;
-    LaneSmem<V, ACC, 8, MB> l8;
+    LaneSmem<V, ACC, 1, MB, max_stage<V, 1, MB>()> l1;
+    LaneSmem<V, ACC, 2, MB, max_stage<V, 2, MB>()> l2;
+    LaneSmem<V, ACC, 4, MB, max_stage<V, 4, MB>()> l4;
+    LaneSmem<V, ACC, 8, MB, max_stage<V, 8, MB>()> l8;
 };
 #define SPC5_BATCH_TILE(RR, SMEM) \
     spmv_tile<V, X, ACC, RR, VS, MB>(SMEM, m.bptr, m.hdr, val, x, y, first, last, m.nrows, m.ncols, ep)
@@ -93,7 +99,7 @@ constexpr int batch_waves_per_eu(int only_r, bool wide_x, int value_bytes, bool 
 }
 
 #define SPC5_BATCH_LANES(RR, SMEM) \
-    spmv_lane_tile<V, X, ACC, RR, VS, MB>(SMEM, m.bptr, m.hdr, val, x, y, first, last, m.nrows, m.ncols, ep)
+    spmv_lane_tile<V, X, ACC, RR, VS, MB>(SMEM, lane_stage_bytes(sizeof(V), RR, VS, m.lanes - 1), m.bptr, m.hdr, val, x, y, first, last, m.nrows, m.ncols, ep)
 
 // The batch loop over tiles: tile t of the list runs body(matrix entry,
 // tile bounds) on its wave.  The record of a wave's next tile is loaded while the current one runs, so a
@@ -127,13 +133,14 @@ k_spmv_batch_sorted(const BatchEntry* __restrict__ mats, const BatchTile* __rest
     static_assert(R == 2 || R == 4, "row-sorted tiles exist for r = 2 and 4");
     __shared__ union {
         TileSmem<ACC, R, expand_cap<V>(), true> order;
-        LaneSmem<V, ACC, R, MB> lanes;
+        LaneSmem<V, ACC, R, MB, max_stage<V, R, MB>()> lanes;
     } sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const Epilogue ep;
     batch_tiles(mats, tiles, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
         if (m.lanes)
-            spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w].lanes, m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
+            spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w].lanes, lane_stage_bytes(sizeof(V), R, VS, m.lanes - 1), m.bptr,
+                                                 m.hdr, reinterpret_cast<const V*>(m.val),
                                                  reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first,
                                                  last, m.nrows, m.ncols, ep);
         else
@@ -143,15 +150,16 @@ k_spmv_batch_sorted(const BatchEntry* __restrict__ mats, const BatchTile* __rest
     });
 }
 
-// Every matrix has r = R and runs the lane-block tile.
-template <class V, class X, class ACC, int VS, int MB, int R>
+// Every matrix has r = R and runs the lane-block tile, at LEVEL or below.
+template <class V, class X, class ACC, int VS, int MB, int R, int LEVEL>
 __global__ __launch_bounds__(kWavesPerGroup * 64, lane_waves_per_eu(R, VS, sizeof(X)) - 1) void k_spmv_batch_lanes(
     const BatchEntry* __restrict__ mats, const BatchTile* __restrict__ tiles, int64_t ntiles) {
-    __shared__ LaneSmem<V, ACC, R, MB> sm[kWavesPerGroup];
+    __shared__ LaneSmem<V, ACC, R, MB, lane_stage_bytes(sizeof(V), R, VS, LEVEL)> sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const Epilogue ep;
     batch_tiles(mats, tiles, ntiles, [&](const BatchEntry& m, int4 first, int4 last) {
-        spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w], m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
+        const int stage = lane_stage_bytes(sizeof(V), R, VS, LEVEL == 0 ? 0 : m.lanes - 1);
+        spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w], stage, m.bptr, m.hdr, reinterpret_cast<const V*>(m.val),
                                              reinterpret_cast<const X*>(m.x), reinterpret_cast<X*>(m.y), first, last,
                                              m.nrows, m.ncols, ep);
     });
@@ -211,6 +219,14 @@ void launch_batch_kernel(const spc5_hip_batch& b, Kernel k, hipStream_t s) {
                        b.tiles.as<const BatchTile>(), b.ntiles);
 }
 
+template <class V, class X, class ACC, int VS, int MB, int R, int LEVEL = 0>
+void launch_batch_lanes(const spc5_hip_batch& b, hipStream_t s) {
+    if constexpr (LEVEL + 1 < lane_levels(sizeof(V), R, VS)) {
+        if (b.lanes > LEVEL + 1) return launch_batch_lanes<V, X, ACC, VS, MB, R, LEVEL + 1>(b, s);
+    }
+    launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, R, LEVEL>, s);
+}
+
 template <class V, class X, class ACC, int VS, int MB>
 void launch_batch(const spc5_hip_batch& b, hipStream_t s) {
     if (b.sorted) {
@@ -223,10 +239,10 @@ void launch_batch(const spc5_hip_batch& b, hipStream_t s) {
     case 2: launch_batch_kernel(b, k_spmv_batch<V, X, ACC, VS, MB, 2>, s); break;
     case 4: launch_batch_kernel(b, k_spmv_batch<V, X, ACC, VS, MB, 4>, s); break;
     case 8: launch_batch_kernel(b, k_spmv_batch<V, X, ACC, VS, MB, 8>, s); break;
-    case -1: launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, 1>, s); break;
-    case -2: launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, 2>, s); break;
-    case -4: launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, 4>, s); break;
-    case -8: launch_batch_kernel(b, k_spmv_batch_lanes<V, X, ACC, VS, MB, 8>, s); break;
+    case -1: launch_batch_lanes<V, X, ACC, VS, MB, 1>(b, s); break;
+    case -2: launch_batch_lanes<V, X, ACC, VS, MB, 2>(b, s); break;
+    case -4: launch_batch_lanes<V, X, ACC, VS, MB, 4>(b, s); break;
+    case -8: launch_batch_lanes<V, X, ACC, VS, MB, 8>(b, s); break;
     default: launch_batch_kernel(b, k_spmv_batch_mixed<V, X, ACC, VS, MB>, s); break;
     }
 }
@@ -299,13 +315,15 @@ int spc5_hip_batch_create(int nmats, const spc5_hip_mat_t* mats, const void* con
     SPC5_HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     b->only_r = mats[0]->r;
     bool all_sorted = true, all_lanes = true, any_lanes = false;
+    int level = 0;
     for (int i = 0; i < nmats; ++i) {
         if (mats[i]->r != mats[0]->r) b->only_r = 0;
         all_lanes = all_lanes && mats[i]->lane_body;
         any_lanes = any_lanes || mats[i]->lane_body;
+        level = std::max(level, mats[i]->lane_body);
         all_sorted = all_sorted && mats[i]->row_sort != 0;
     }
-    b->lanes = b->only_r && all_lanes ? 1 : 0;
+    b->lanes = b->only_r && all_lanes ? level : 0;
     b->sorted = (b->only_r == 2 || b->only_r == 4) && !b->lanes && all_sorted ? 1 : 0;
     if (b->only_r && !b->lanes && !b->sorted && any_lanes) b->only_r = 0;  // both tiles: the mixed kernel
     int64_t wv = waves > 0 ? waves : (int64_t)ncu * 4 * batch_kernel_waves(*b) * kWaveRounds;

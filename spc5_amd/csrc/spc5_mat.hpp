@@ -92,7 +92,7 @@ struct spc5_hip_mat {
     int spmm_cols = 0;                    // SPC5_HIP_OPT_SPMM_COLUMNS
     int spmm_x16 = -1;                    // SPC5_HIP_OPT_SPMM_X16; -1: 1 for double vectors, else 0
     double scatter = 0.0;                 // distinct 128-byte lines of x per block, among 64 neighbours (sampled)
-    int lane_body = 0;                    // products run the lane-block tile (spmv_lane.hpp; see lane_block_wins)
+    int lane_body = 0;                    // 1 + stage level: products run the lane-block tile (spmv_lane.hpp); else 0
     spc5::Plan plan;
     std::vector<std::shared_ptr<spc5::DeviceBuffer>> owned;  // buffers the handle allocated itself
 };
@@ -111,6 +111,7 @@ int build_plan(spc5_hip_mat& m, hipStream_t s);
 int default_tile_values(int64_t nnz);
 // Whether a handle's products run the lane-block tile (defined in spmv.hip).
 bool lane_block_wins(const spc5_hip_mat& m);
+int lane_level(const spc5_hip_mat& m);
 // Another tile list of the same matrix with at most `maxrows` rows per tile
 // (needs the value offsets of m.plan; defined in spmv.hip).
 int build_tiles(const spc5_hip_mat& m, Plan& p, int maxrows, int target, hipStream_t s);

@@ -64,18 +64,19 @@ k_spmv_tiles(
     spmv_tile<V, X, ACC, R, VS, MB, SORT>(sm[w], bptr, hdr, val, x, y, tiles[t], tiles[t + 1], nrows, ncols, e);
 }
 
-template <class V, class X, class ACC, int R, int VS, int MB>
-__global__ __launch_bounds__(kWavesPerGroup * 64, lane_waves_per_eu(R, VS, sizeof(X))) void k_spmv_lanes(
+template <class V, class X, class ACC, int R, int VS, int MB, int STAGE>
+__global__ __launch_bounds__(kWavesPerGroup * 64, lane_waves_per_eu(R, VS, sizeof(X)) - (STAGE > 5120 ? 1 : 0)) void k_spmv_lanes(
     const int* __restrict__ bptr, const unsigned char* __restrict__ hdr, const V* __restrict__ val,
     const X* __restrict__ x, X* __restrict__ y, const int4* __restrict__ tiles, int64_t ntiles, int64_t nrows,
     int64_t ncols, Epilogue ep) {
-    __shared__ LaneSmem<V, ACC, R, MB> sm[kWavesPerGroup];
+    __shared__ LaneSmem<V, ACC, R, MB, STAGE> sm[kWavesPerGroup];
     const int w = threadIdx.x >> 6;
     const int64_t t = xcd_tile(w);
     if (t >= ntiles) return;  // whole wave leaves; no workgroup barrier is used
     Epilogue e = ep;
     if (e.dot) e.dot += t;  // one partial per tile
-    spmv_lane_tile<V, X, ACC, R, VS, MB>(sm[w], bptr, hdr, val, x, y, tiles[t], tiles[t + 1], nrows, ncols, e);
+    spmv_lane_tile<V, X, ACC, R, VS, MB, STAGE>(sm[w], STAGE, bptr, hdr, val, x, y, tiles[t], tiles[t + 1], nrows,
+                                                ncols, e);
 }
 
 // ---- access probe ----------------------------------------------------------
@@ -341,11 +342,15 @@ void launch_tiles(const spc5_hip_mat& m, const void* x, void* y, hipStream_t s, 
                        m.ncols, ep);
 }
 
-template <class V, class X, class ACC, int R, int VS, int MB>
+template <class V, class X, class ACC, int R, int VS, int MB, int LEVEL = 0>
 void launch_lanes(const spc5_hip_mat& m, const void* x, void* y, hipStream_t s, const Epilogue& ep) {
+    constexpr int kStage = lane_stage_bytes(sizeof(V), R, VS, LEVEL);
+    if constexpr (LEVEL + 1 < lane_levels(sizeof(V), R, VS)) {
+        if (m.lane_body > LEVEL + 1) return launch_lanes<V, X, ACC, R, VS, MB, LEVEL + 1>(m, x, y, s, ep);
+    }
     const int64_t groups = (m.plan.ntiles + kWavesPerGroup - 1) / kWavesPerGroup;
     const unsigned grid = (unsigned)((groups + 7) / 8 * 8);
-    hipLaunchKernelGGL((k_spmv_lanes<V, X, ACC, R, VS, MB>), dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.bptr,
+    hipLaunchKernelGGL((k_spmv_lanes<V, X, ACC, R, VS, MB, kStage>), dim3(grid), dim3(kWavesPerGroup * 64), 0, s, m.bptr,
                        m.hdr, reinterpret_cast<const V*>(m.values), reinterpret_cast<const X*>(x),
                        reinterpret_cast<X*>(y), m.plan.tiles->as<int4>(), m.plan.ntiles, m.nrows, m.ncols, ep);
 }
@@ -519,7 +524,7 @@ int build_plan(spc5_hip_mat& m, hipStream_t s) {
     }
     p.ntiles = h[4];
     m.scatter = h[2] > 0 ? (double)h[1] / h[2] : 0.0;
-    m.lane_body = lane_block_wins(m);
+    m.lane_body = lane_block_wins(m) ? 1 + lane_level(m) : 0;
     return SPC5_HIP_OK;
 }
 
@@ -556,6 +561,18 @@ bool lane_block_wins(const spc5_hip_mat& m) {
     if (f64) return m.r <= 2 && small;
     if (m.value_type == SPC5_HIP_F32 && m.vs == 16) return m.r <= 4 && small;
     return m.r <= 2 || (m.r == 4 && small);
+}
+
+// The lowest stage level that holds 64 blocks of the matrix's mean size, 0 up to
+// 4 KiB (see lane_stage_bytes).
+int lane_level(const spc5_hip_mat& m) {
+    const int vb = (int)value_bytes(m.value_type);
+    const int levels = lane_levels(vb, m.r, m.vs);
+    if (levels == 1 || m.nblocks == 0) return 0;
+    const double need = 64.0 * vb * (double)m.nnz / (double)m.nblocks;
+    int level = need > 4096.0 ? 1 : 0;
+    while (level > 0 && level + 1 < levels && need > lane_stage_bytes(vb, m.r, m.vs, level)) ++level;
+    return level;
 }
 
 // Values per tile aimed at when no tile size is set (a tile also ends every
@@ -642,7 +659,7 @@ int spc5_hip_mat_create_values_view(spc5_hip_mat_t base, int value_type, const v
     std::unique_ptr<spc5_hip_mat> m(new spc5_hip_mat(*base));
     m->value_type = value_type;
     m->values = d_values;
-    m->lane_body = lane_block_wins(*m);
+    m->lane_body = lane_block_wins(*m) ? 1 + lane_level(*m) : 0;
     *out = m.release();
     return SPC5_HIP_OK;
 }

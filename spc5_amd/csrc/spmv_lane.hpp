@@ -42,15 +42,32 @@ constexpr int lane_waves_per_eu(int r, int vs, int xbytes) {
 // 16-column blocks, which runs the value-order tile).
 constexpr bool lane_block_fits(int vs, int xbytes) { return vs * xbytes <= 64; }
 
-// LDS bytes of staged values per batch.
-template <class V>
-constexpr int lane_stage_bytes() { return sizeof(V) == 8 ? 4096 : 3072; }
+// LDS bytes of staged values per batch.  They bound the values, and so the blocks
+// a batch takes; more of them cost registers and waves.  Double beta(4,8) and
+// float beta(8,16), whose blocks hold up to 32 and 128 values, have more levels
+// and take the lowest that holds 64 of the matrix's mean blocks, or the highest
+// (lane_level in spmv.hip); past 5 KiB float leaves fewer than 5 waves a SIMD.  Stage of 4 / 5 / 6 / 8 KiB, double beta(4,8): banded 60,000 rows,
+// half-width 128, 9.9 values a block 18.3 / 15.8 / 14.6 / 15.4 us, 96 banded
+// matrices in one launch 621 / 571 / 588 / 611, stencil 64^3, 11.9 values a block
+// 20.9 / 20.7 / 16.9 / 17.6, Laplacian 1000^2, 6.7 values a block 17.8 / 18.6 /
+// 20.1 / 21.0.  3 / 4 / 6 / 8 KiB, float beta(8,16): banded 250,000 rows, 37 values
+// a block 42 / 36 / 30 / 27, stencil 128^3, 24 values a block 145 / 129 / 128 / 131,
+// Laplacian, 13 values a block 27.6 / 28.1 / 29.2 / 31.4.  All others lose with
+// more (float beta(2,16) banded 9.7 / 10.4 / 10.6 / 11.5).
+constexpr int lane_levels(int vbytes, int r, int vs) {
+    return vbytes == 8 && r == 4 ? 3 : (vbytes == 4 && vs == 16 && r == 8 ? 2 : 1);
+}
+__host__ __device__ constexpr int lane_stage_bytes(int vbytes, int r, int vs, int level) {
+    if (vbytes == 8) return r == 4 ? 4096 + 1024 * level : 4096;
+    return vs == 16 && vbytes == 4 && r == 8 ? 3072 + 2048 * level : 3072;
+}
 
-template <class V, class ACC, int R, int MB>
+// STAGE: the staged bytes at most (a tile's `stage` may be less).
+template <class V, class ACC, int R, int MB, int STAGE>
 struct LaneSmem {
     static constexpr int kHeader = 4 + R * MB;
     static constexpr int kHdrWords = (15 + 64 * kHeader + 15) / 16;  // 16-byte words over 64 headers
-    alignas(16) unsigned char val[lane_stage_bytes<V>()];
+    alignas(16) unsigned char val[STAGE];
     alignas(16) unsigned hdr[4 * (kHdrWords + 1)];  // + 1: a header's last dword pair may be read past its end
     ACC acc[tile_rows(R)];
     int mark[64];
@@ -82,17 +99,18 @@ __device__ __forceinline__ ACC staged_value(const unsigned char* base, int o) {
 // s_waitcnt operand: no vector memory load outstanding, other counters free.
 constexpr int kWaitVm0 = 0x0f70;
 
-template <class V, class X, class ACC, int R, int VS, int MB>
-__device__ __forceinline__ void spmv_lane_tile(LaneSmem<V, ACC, R, MB>& sm, const int* __restrict__ bptr,
+template <class V, class X, class ACC, int R, int VS, int MB, int STAGE>
+__device__ __forceinline__ void spmv_lane_tile(LaneSmem<V, ACC, R, MB, STAGE>& sm, int stage,
+                                               const int* __restrict__ bptr,
                                                const unsigned char* __restrict__ hdr, const V* __restrict__ val,
                                                const X* __restrict__ x, X* __restrict__ y, int4 first, int4 last,
                                                int64_t nrows, int64_t ncols, const Epilogue& ep) {
     constexpr int H = 4 + R * MB;
     constexpr int NMW = (R * VS + 31) / 32;                 // mask dwords
     constexpr int PER = 16 / (int)sizeof(V);                // values per 16-byte word
-    constexpr int KV = lane_stage_bytes<V>() / 1024;        // 16-byte words of values per lane
-    constexpr int CAP = KV * 64 * PER;                      // staged values
-    constexpr int KH = LaneSmem<V, ACC, R, MB>::kHdrWords > 64 ? 2 : 1;
+    constexpr int KV = STAGE / 1024;                        // 16-byte words of values per lane
+    const int cap = stage / (int)sizeof(V);                 // staged values
+    constexpr int KH = LaneSmem<V, ACC, R, MB, STAGE>::kHdrWords > 64 ? 2 : 1;
     constexpr int XC = 16 / (int)sizeof(X);                 // columns per 16-byte x load
     constexpr int NQ = VS / XC;                             // x loads per window
     using U4 = unsigned int __attribute__((ext_vector_type(4)));
@@ -149,7 +167,7 @@ __device__ __forceinline__ void spmv_lane_tile(LaneSmem<V, ACC, R, MB>& sm, cons
         const int hoff = (int)((reinterpret_cast<uintptr_t>(hdr) + (uint64_t)(unsigned)b * H) & 15);
 #pragma unroll
         for (int k = 0; k < KH; ++k)
-            if (lane + 64 * k < LaneSmem<V, ACC, R, MB>::kHdrWords)
+            if (lane + 64 * k < LaneSmem<V, ACC, R, MB, STAGE>::kHdrWords)
                 *reinterpret_cast<U4*>(&sm.hdr[4 * (lane + 64 * k)]) = hw[k];
         sm.mark[lane] = 0;
         wave_sync();
@@ -169,7 +187,7 @@ __device__ __forceinline__ void spmv_lane_tile(LaneSmem<V, ACC, R, MB>& sm, cons
         // 16-byte words of values from the one that holds value v
         const V* va = val + (unsigned)v;
         const int shift = (int)((reinterpret_cast<uintptr_t>(va) & 15) / sizeof(V));
-        const int fit = __popcll(ballot64(incl <= CAP - shift));
+        const int fit = __popcll(ballot64(incl <= cap - shift));
         const int ntake = fit < n ? fit : n;
         const int total = __builtin_amdgcn_readlane(incl, ntake - 1);
         const int words = (shift + total + PER - 1) / PER;
