@@ -318,7 +318,7 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
         for (int e = 0; e < CPL; ++e) run[e] = (ACC)0;
         int prow = -1;
         // the running sums of row prow go to the tile's LDS sums
-        auto close = [&]() {
+        auto close = [&]() __attribute__((always_inline)) {
             if (prow >= 0) {
 #pragma unroll
                 for (int e = 0; e < CPL; ++e)
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(64) void k_spmm_tiles(const int* __restrict__ bptr,
         // record at a time waited up to U - 1 times (clustered 300 K rows,
         // beta(2,16) float, k = 5, one column a lane: 80 -> 71 us; stencil
         // 64^3, beta(2,8), k = 64, column records: 226 -> 198 us).
-        auto step = [&](auto uu, auto part_step) {
+        auto step = [&](auto uu, auto part_step) __attribute__((always_inline)) {
             constexpr int UU = decltype(uu)::value;
             constexpr bool PART = decltype(part_step)::value;
             if constexpr (ONE && !WIDE && sizeof(X) < 8) {
@@ -517,7 +517,7 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
     // DIRECT: Y of block-row pb, requested when the block-row opens so that
     // the read is in flight while its records are processed
     X yv[DIRECT ? R : 1];
-    auto request_y = [&](int brow) {
+    auto request_y = [&](int brow) __attribute__((always_inline)) {
         if constexpr (DIRECT) {
 #pragma unroll
             for (int tr = 0; tr < R; ++tr) {
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
             }
         }
     };
-    auto write_blockrow = [&](int brow, bool have) {
+    auto write_blockrow = [&](int brow, bool have) __attribute__((always_inline)) {
 #pragma unroll
         for (int tr = 0; tr < R; ++tr) {
             const int rr = brow * R + tr;
@@ -540,13 +540,13 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
         }
     };
     // block-rows [done, upto) hold no value: y = beta * y (nothing when beta == 1)
-    auto skip_to = [&](int upto) {
+    auto skip_to = [&](int upto) __attribute__((always_inline)) {
         if (beta != (ACC)1) {
             for (int br = done; br < upto; ++br) write_blockrow(br, false);
         }
         done = upto > done ? upto : done;
     };
-    auto flush = [&](int brow) {
+    auto flush = [&](int brow) __attribute__((always_inline)) {
         if (pb >= 0) {
             if constexpr (DIRECT) {
                 skip_to(pb);
@@ -644,7 +644,7 @@ __global__ __launch_bounds__(64) void k_spmm_cols(const int* __restrict__ bptr, 
         const int per = DIRECT ? nrec : spmm_run(nrec, part.groups);
         int q = grp * per;
         const int qb = q + per < nrec ? q + per : nrec;
-        auto step = [&](auto uu, auto part_step) {  // as k_spmm_tiles
+        auto step = [&](auto uu, auto part_step) __attribute__((always_inline)) {  // as k_spmm_tiles
             constexpr int UU = decltype(uu)::value;
             constexpr bool PART = decltype(part_step)::value;
             int cu[UU], bu[UU];
@@ -767,6 +767,10 @@ void launch_spmm_vals(const spc5_hip_mat& m, const SpmmArgs& a) {
 // groups share the wave (k = 64 in double on the 27-point stencil at beta(4,8):
 // 3.16 ms with 32-column chunks and 4 requests, 3.53 ms with 8; 2.95 ms with
 // 64-column chunks, two groups, and 8 requests, 3.12 ms with 4).
+// Column records of 8 rows always take 4: 16 running sums a lane and 8 requests
+// leave 3 waves a SIMD (stencil 64^3 in double, k = 48: 219 us, 192 with 4).
+// The kernels' lambdas are inlined by attribute: left to the compiler, the copies
+// of a flush of 8 rows stay calls, and the sums they share go to scratch memory.
 template <class V, class X, class ACC, int R, int VS, int MB, bool WIDE>
 void launch_spmm_r(const spc5_hip_mat& m, const SpmmArgs& a, bool cols, bool vec, bool one) {
     constexpr int CPL = 16 / (int)sizeof(X);
@@ -775,7 +779,7 @@ void launch_spmm_r(const spc5_hip_mat& m, const SpmmArgs& a, bool cols, bool vec
     if constexpr (R > 1) {
         if (cols) {
             constexpr int U = R <= 2 ? 16 : 8;
-            if constexpr (kTwo) {
+            if constexpr (kTwo && R < 8) {
                 if (vec && two) return launch_spmm_cols<V, X, ACC, R, VS, MB, WIDE, CPL, false, U>(m, a);
             }
             if (vec)
@@ -821,7 +825,11 @@ int launch_spmm_t(const spc5_hip_mat& m, const void* x, int64_t ldx, void* y, in
     // a whole request in every chunk.
     const int cpl = 16 / (int)sizeof(X);
     const bool x16 = m.spmm_x16 < 0 ? spmm_x16_default<X>(cols, m.r, kt) : m.spmm_x16 == 1;
-    const bool vec = x16 && kt >= cpl && (k % kt == 0 || k % kt >= cpl);
+    // (asked for with column records narrower than the rule's, only where no
+    // request overlaps another: stencil 64^3, beta(8,8), k = 5, 99 us with one
+    // element, 135 with 16 bytes)
+    const bool vec = x16 && kt >= cpl && (k % kt == 0 || k % kt >= cpl) &&
+                     !(cols && kt < 3 * m.r && (kt % cpl != 0 || k % cpl != 0));
     // one column per lane and the whole wave on one record; with column
     // records it writes Y directly, on whole SpMV-sized tiles
     const bool one = !vec && kt > 32 && (k % kt == 0 || k % kt > 32);

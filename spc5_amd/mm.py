@@ -4,7 +4,7 @@
 loadMM, examples/load_mm_and_compare.cpp:287-428: 0-based indices, pattern
 values 1, mirrored symmetric / skew-symmetric entries).  `coo_to_csr` is the
 reference's COO_unsorted_to_CSR / COO_sorted_to_CSR (src/spc5.hpp:77-114) on
-the GPU: a stable radix sort by (row, column), duplicates kept in input
+the GPU: stable by (row, column), duplicates kept in input
 order.  `load_csr` chains the two into device CSR arrays ready for
 DeviceMatrix.from_csr.
 """
