@@ -180,8 +180,8 @@ int spc5_hip_spmv(spc5_hip_mat_t h, const void* d_x, void* d_y, void* stream);
 
 /* COO (device) -> CSR (device): the reference's COO_unsorted_to_CSR
  * (src/spc5.hpp:106-114; sorted = 0) and COO_sorted_to_CSR (77-104;
- * sorted = 1, order checked).  Entries are ordered by (row, column) with a
- * stable radix sort; duplicates are kept in input order.  value_bytes is 8
+ * sorted = 1, order checked).  Entries are ordered by (row, column), stably:
+ * duplicates are kept in input order.  value_bytes is 8
  * (double) or 4 (float).  d_rowptr gets nrows+1 entries, d_col / d_val nnz.
  * Indices out of range or an unsorted input with sorted = 1 are errors. */
 int spc5_hip_coo_to_csr(int value_bytes, int64_t nrows, int64_t ncols, int64_t nnz, int sorted, const int* d_i,
