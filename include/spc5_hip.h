@@ -165,7 +165,8 @@ int spc5_hip_mat_load(const char* path, spc5_hip_mat_t* out);
  * (two doubles or four floats, adjacent columns, at any element's address)
  * instead of one element.  Fewer lanes then share a record, which halves
  * (double) or quarters (float) the address work per column.  Column chunks
- * narrower than a request take one element per lane.  Unless set: on for
+ * narrower than a request take one element per lane, and so do column records
+ * of fewer than 3 r columns that requests do not divide.  Unless set: on for
  * double vectors (with column records from 3 r columns per chunk), and for
  * float vectors with value records from 5 columns (r > 1: up to 48).
  * Results agree with one element per lane to rounding.  No counterpart in the
@@ -301,7 +302,7 @@ int spc5_hip_mixed_cg(spc5_hip_mat_t A64, spc5_hip_mat_t Alo, const double* d_b,
                       void* stream);
 
 /* ---------------------------------------------------------------------- */
-/* Batching form: many independent matrices in one persistent launch      */
+/* Batching form: many independent matrices in one launch                 */
 /* (no counterpart in the reference).                                     */
 /* ---------------------------------------------------------------------- */
 

@@ -1,5 +1,5 @@
 """Autotuner of the SpMV and its batching form: per matrix, r (rows per
-block), the tile size of the product, the persistent wave count of a batch,
+block), the tile size of the product, the wave count of a batch,
 and the column chunk and record kind of multi-right-hand-side products.
 
 r is chosen from a cost model evaluated on GPU block counts (one count pass
@@ -25,7 +25,7 @@ used here.
 
 `mode="measure"` converts the matrix with each candidate r and times it
 instead (exact, costs four conversions).  `tune_tiles` times candidate tile
-sizes of one matrix's product, `tune_batch_waves` candidate persistent wave
+sizes of one matrix's product, `tune_batch_waves` candidate wave
 counts of a batch, `tune_spmm_kt` the column chunks of a product with k
 right-hand sides, and `tune_spmm` picks r, the chunk and the record kind
 (per value or per block column) by timing.

@@ -1,5 +1,5 @@
 """Batching form: many independent beta(r,VS) matrices multiplied in one
-persistent, hipGraph-captured launch (libspc5_hip.so spc5_hip_batch_*)."""
+hipGraph-captured launch (libspc5_hip.so spc5_hip_batch_*)."""
 from __future__ import annotations
 
 import ctypes as C

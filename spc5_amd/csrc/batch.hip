@@ -94,7 +94,7 @@ union MixedSmem {
 // Waves per SIMD of the batch kernel: with every r body (ONLY_R = 0) the
 // most that compile without spills; with one r, the tile kernel's rule.
 constexpr int batch_waves_per_eu(int only_r, bool wide_x, int value_bytes, bool sorted = false) {
-    // the persistent loop's own state costs one wave (two with 8-byte values)
+    // the tile loop's own state costs one wave (two with 8-byte values)
     return only_r == 0 ? 5 : tile_waves_per_eu(only_r, sorted, wide_x) - (value_bytes == 8 ? 2 : 1);
 }
 
